@@ -88,6 +88,11 @@ SIGNATURES: dict[str, tuple[object, list[object]]] = {
         _I32,
         [_P, _P, _P, _P, _P, _P, _I32, _I64, _I64, _I64, _I64, _F, _P, _SZ, _P],
     ),
+    "cf_lora_forward_workspace_bytes": (_SZ, [_I32, _I64, _I64, _I64, _I64]),
+    "cf_lora_forward": (
+        _I32,
+        [_P, _P, _P, _P, _P, _P, _I32, _I64, _I64, _I64, _I64, _F, _P, _SZ, _P],
+    ),
     "cf_matmul": (_I32, [_P, _P, _P, _I32, _I64, _I64, _I64, _P]),
     "cf_lora_backward_workspace_bytes": (_SZ, [_I64, _I64, _I64, _I64]),
     "cf_lora_backward": (

@@ -35,6 +35,7 @@ HIP_SOURCES = (
     "cf_activations.hip",
     "cf_lora.hip",
     "cf_lora_fused.hip",
+    "cf_lora_skinny.hip",
     "cf_lora_bwd.hip",
     "cf_lora_f32.hip",
     "cf_matmul_f32.hip",

@@ -6,7 +6,8 @@
 //   y = x @ w + scale * ((x @ a) @ b)
 //
 // Fast path (bf16, K % 64 == 0, N % 8 == 0, r <= 16, 16-byte aligned): the
-// fused MFMA kernel in cf_lora_fused.hip, one launch.
+// fused MFMA kernel in cf_lora_fused.hip, one launch. With at most 64 rows
+// and a workspace, the kernels of cf_lora_skinny.hip (any rank up to 256).
 //
 // fp32 (r <= 16, K and N multiples of 4, 16-byte aligned): the MFMA kernel of
 // cf_lora_f32.hip, operands split into bf16 high and low parts on the way
@@ -29,6 +30,7 @@
 #include "cf_lora_bwd.hpp"
 #include "cf_lora_f32.hpp"
 #include "cf_lora_fused.hpp"
+#include "cf_lora_skinny.hpp"
 
 namespace cf {
 namespace {
@@ -391,6 +393,41 @@ cf_status cf_lora_linear_ws(const void* x, const void* w, const void* a, const v
     }
     return cf_lora_linear(x, w, a, b, y, xa_out, dtype, batch, in_features, out_features, rank,
                           scale, stream);
+}
+
+size_t cf_lora_forward_workspace_bytes(cf_dtype dtype, int64_t batch, int64_t in_features,
+                                       int64_t out_features, int64_t rank) {
+    const size_t plain = cf_lora_linear_ws_bytes(dtype, batch, in_features, out_features, rank);
+    size_t needed = 0;
+    if (dtype == CF_BF16 && cf::lora_skinny_shape(batch, out_features, in_features, rank)) {
+        needed = cf::lora_skinny_workspace_bytes(batch, out_features, in_features, rank);
+    }
+    return needed > plain ? needed : plain;
+}
+
+cf_status cf_lora_forward(const void* x, const void* w, const void* a, const void* b, void* y,
+                          float* xa_out, cf_dtype dtype, int64_t batch, int64_t in_features,
+                          int64_t out_features, int64_t rank, float scale, void* workspace,
+                          size_t workspace_bytes, void* stream) {
+    CF_ENTRY();
+    if (batch <= 0 || out_features <= 0) return CF_OK;
+    CF_REQUIRE(in_features >= 0 && rank >= 0, "cf_lora_forward: negative dimension");
+    CF_REQUIRE(dtype == CF_F32 || dtype == CF_BF16,
+               "cf_lora_forward: dtype %s has no kernel (float32 or bfloat16)", cf::dtype_name(dtype));
+    CF_REQUIRE(x != nullptr && w != nullptr && y != nullptr, "cf_lora_forward: null pointer");
+    CF_REQUIRE(rank == 0 || (a != nullptr && b != nullptr), "cf_lora_forward: null adapter");
+    const size_t needed =
+        cf_lora_forward_workspace_bytes(dtype, batch, in_features, out_features, rank);
+    CF_REQUIRE(needed == 0 || (workspace != nullptr && workspace_bytes >= needed),
+               "cf_lora_forward: workspace of %zu bytes given, %zu needed", workspace_bytes, needed);
+    CF_REQUIRE(cf::host_aligned(workspace, 16), "cf_lora_forward: workspace must be 16-byte aligned");
+    if (dtype == CF_BF16 &&
+        cf::lora_skinny_eligible(x, w, a, b, y, batch, out_features, in_features, rank)) {
+        return cf::launch_lora_skinny(x, w, a, b, y, xa_out, batch, out_features, in_features, rank,
+                                      scale, workspace, static_cast<hipStream_t>(stream));
+    }
+    return cf_lora_linear_ws(x, w, a, b, y, xa_out, dtype, batch, in_features, out_features, rank,
+                             scale, workspace, workspace_bytes, stream);
 }
 
 cf_status cf_matmul(const void* a, const void* b, void* c, cf_dtype dtype, int64_t m, int64_t n,

@@ -286,6 +286,27 @@ cf_status cf_lora_linear_ws(const void* x, const void* w, const void* a, const v
                             int64_t out_features, int64_t rank, float scale, void* workspace,
                             size_t workspace_bytes, void* stream);
 
+/* Workspace bytes cf_lora_forward needs for these sizes (0: none). At least
+ * cf_lora_linear_ws_bytes of the same arguments. It has no counterpart in the
+ * reference. */
+size_t cf_lora_forward_workspace_bytes(cf_dtype dtype, int64_t batch, int64_t in_features,
+                                       int64_t out_features, int64_t rank);
+
+/* cf_lora_linear_ws for callers that give it the larger workspace of
+ * cf_lora_forward_workspace_bytes(...) bytes (16-byte aligned, in any state;
+ * NULL when that is 0): the same operation, free to pick kernels whose
+ * partial sums live there. bf16 with at most 64 rows, in_features and
+ * out_features multiples of 8 and a rank up to 256 streams w once, cut over
+ * columns and the reduction range, and sums the slices in a fixed order
+ * (deterministic; fp32 accumulation and the same bf16 rounding of x @ a).
+ * Every other problem runs as cf_lora_linear_ws. Calls that overlap (other
+ * streams) need workspaces of their own. Replaces launch_lora_linear
+ * (cuda/include/cudaforge/lora_linear.cuh:49-51). */
+cf_status cf_lora_forward(const void* x, const void* w, const void* a, const void* b, void* y,
+                          float* xa_out, cf_dtype dtype, int64_t batch, int64_t in_features,
+                          int64_t out_features, int64_t rank, float scale, void* workspace,
+                          size_t workspace_bytes, void* stream);
+
 /* c[m, n] = a[m, k] @ b[k, n], row-major, one dtype (fp32 or bf16), fp32
  * accumulation. Replaces launch_matmul (cuda/include/cudaforge/lora_linear.cuh:57-58). */
 cf_status cf_matmul(const void* a, const void* b, void* c, cf_dtype dtype, int64_t m, int64_t n,
