@@ -36,6 +36,7 @@ HIP_SOURCES = (
     "cf_lora.hip",
     "cf_lora_fused.hip",
     "cf_lora_skinny.hip",
+    "cf_lora_tile.hip",
     "cf_lora_bwd.hip",
     "cf_lora_f32.hip",
     "cf_matmul_f32.hip",

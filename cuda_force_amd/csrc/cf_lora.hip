@@ -7,7 +7,9 @@
 //
 // Fast path (bf16, K % 64 == 0, N % 8 == 0, r <= 16, 16-byte aligned): the
 // fused MFMA kernel in cf_lora_fused.hip, one launch. With at most 64 rows
-// and a workspace, the kernels of cf_lora_skinny.hip (any rank up to 256).
+// and a workspace, the kernels of cf_lora_skinny.hip (any rank up to 256);
+// with a workspace, smaller tiles and any rank up to 128 (K a multiple of 8)
+// in cf_lora_tile.hip.
 //
 // fp32 (r <= 16, K and N multiples of 4, 16-byte aligned): the MFMA kernel of
 // cf_lora_f32.hip, operands split into bf16 high and low parts on the way
@@ -31,6 +33,7 @@
 #include "cf_lora_f32.hpp"
 #include "cf_lora_fused.hpp"
 #include "cf_lora_skinny.hpp"
+#include "cf_lora_tile.hpp"
 
 namespace cf {
 namespace {
@@ -295,6 +298,19 @@ cf_status launch_generic(const void* x, const void* w, const void* a, const void
     return check_launch("launching the tiled LoRA GEMM", stream);
 }
 
+/// The kernels of cf_lora_forward for a bf16 problem, by its sizes.
+enum class Route { kLinear, kSkinny, kTile };
+
+Route route_of(int64_t M, int64_t N, int64_t K, int64_t rank) {
+    if (lora_skinny_shape(M, N, K, rank)) return Route::kSkinny;
+    if (!lora_tile_shape(M, N, K, rank)) return Route::kLinear;
+    // The 256x256-tile kernel where it runs and is estimated no slower.
+    const bool fused = K % 64 == 0 && rank <= 16 && rank % 2 == 0;
+    return fused && lora_fused_estimate_us(M, N, K) <= 1.05f * lora_tile_estimate_us(M, N, K, rank)
+               ? Route::kLinear
+               : Route::kTile;
+}
+
 }  // namespace
 }  // namespace cf
 
@@ -398,9 +414,17 @@ cf_status cf_lora_linear_ws(const void* x, const void* w, const void* a, const v
 size_t cf_lora_forward_workspace_bytes(cf_dtype dtype, int64_t batch, int64_t in_features,
                                        int64_t out_features, int64_t rank) {
     const size_t plain = cf_lora_linear_ws_bytes(dtype, batch, in_features, out_features, rank);
+    if (dtype != CF_BF16) return plain;
     size_t needed = 0;
-    if (dtype == CF_BF16 && cf::lora_skinny_shape(batch, out_features, in_features, rank)) {
-        needed = cf::lora_skinny_workspace_bytes(batch, out_features, in_features, rank);
+    switch (cf::route_of(batch, out_features, in_features, rank)) {
+        case cf::Route::kSkinny:
+            needed = cf::lora_skinny_workspace_bytes(batch, out_features, in_features, rank);
+            break;
+        case cf::Route::kTile:
+            needed = cf::lora_tile_workspace_bytes(batch, out_features, in_features, rank);
+            break;
+        case cf::Route::kLinear:
+            break;
     }
     return needed > plain ? needed : plain;
 }
@@ -421,10 +445,18 @@ cf_status cf_lora_forward(const void* x, const void* w, const void* a, const voi
     CF_REQUIRE(needed == 0 || (workspace != nullptr && workspace_bytes >= needed),
                "cf_lora_forward: workspace of %zu bytes given, %zu needed", workspace_bytes, needed);
     CF_REQUIRE(cf::host_aligned(workspace, 16), "cf_lora_forward: workspace must be 16-byte aligned");
-    if (dtype == CF_BF16 &&
-        cf::lora_skinny_eligible(x, w, a, b, y, batch, out_features, in_features, rank)) {
-        return cf::launch_lora_skinny(x, w, a, b, y, xa_out, batch, out_features, in_features, rank,
-                                      scale, workspace, static_cast<hipStream_t>(stream));
+    if (dtype == CF_BF16) {
+        const cf::Route route = cf::route_of(batch, out_features, in_features, rank);
+        if (route == cf::Route::kSkinny &&
+            cf::lora_skinny_eligible(x, w, a, b, y, batch, out_features, in_features, rank)) {
+            return cf::launch_lora_skinny(x, w, a, b, y, xa_out, batch, out_features, in_features, rank,
+                                          scale, workspace, static_cast<hipStream_t>(stream));
+        }
+        if (route == cf::Route::kTile &&
+            cf::lora_tile_eligible(x, w, a, b, y, batch, out_features, in_features, rank)) {
+            return cf::launch_lora_tile(x, w, a, b, y, xa_out, batch, out_features, in_features, rank,
+                                        scale, workspace, static_cast<hipStream_t>(stream));
+        }
     }
     return cf_lora_linear_ws(x, w, a, b, y, xa_out, dtype, batch, in_features, out_features, rank,
                              scale, workspace, workspace_bytes, stream);

@@ -712,6 +712,13 @@ bool lora_fused_eligible(const void* x, const void* w, const void* a, const void
            ceil_div<int64_t>(M, kBM) * ceil_div<int64_t>(N, kBN) < (1LL << 31);
 }
 
+float lora_fused_estimate_us(int64_t M, int64_t N, int64_t K) {
+    const int64_t tiles = ceil_div<int64_t>(M, kBM) * ceil_div<int64_t>(N, kBN);
+    const int64_t rounds = ceil_div<int64_t>(tiles, 256);
+    const float full = tiles >= 256 ? 1.0f : static_cast<float>(tiles) / 256.0f;
+    return 3.0f + static_cast<float>(rounds * (K / kBK)) * (0.61f + 0.21f * full);
+}
+
 size_t lora_fused_workspace_bytes(int64_t M, int64_t rank) {
     if (M <= 0 || rank <= 0) return 0;
     const int64_t tiles_m = ceil_div<int64_t>(M, kBM);

@@ -299,7 +299,9 @@ size_t cf_lora_forward_workspace_bytes(cf_dtype dtype, int64_t batch, int64_t in
  * out_features multiples of 8 and a rank up to 256 streams w once, cut over
  * columns and the reduction range, and sums the slices in a fixed order
  * (deterministic; fp32 accumulation and the same bf16 rounding of x @ a).
- * Every other problem runs as cf_lora_linear_ws. Calls that overlap (other
+ * bf16 with more rows and a rank up to 128, where 256 x 256 tiles would leave
+ * the GPU idle or the fused kernel does not take the rank or in_features,
+ * runs smaller tiles on the MFMA units. Every other problem runs as cf_lora_linear_ws. Calls that overlap (other
  * streams) need workspaces of their own. Replaces launch_lora_linear
  * (cuda/include/cudaforge/lora_linear.cuh:49-51). */
 cf_status cf_lora_forward(const void* x, const void* w, const void* a, const void* b, void* y,
