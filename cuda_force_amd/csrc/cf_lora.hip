@@ -24,7 +24,7 @@
 //   G      = dy @ b^T            [M, r]
 //   grad_b = scale * xa^T @ dy   [r, N]   column reduction over M
 //   grad_a = scale * x^T @ G     [K, r]   column reduction over M
-// bf16 with rank <= 16 runs the MFMA kernels of cf_lora_bwd.hip. The generic
+// bf16 with rank <= 64 runs the MFMA kernels of cf_lora_bwd.hip. The generic
 // path here (fp32, other shapes): G one wave per row of dy, the column
 // reductions in row chunks into an fp32 workspace and a second kernel summing
 // the chunks in a fixed order (deterministic).
@@ -493,7 +493,7 @@ size_t cf_lora_backward_workspace_bytes(int64_t batch, int64_t in_features, int6
     const size_t part = static_cast<size_t>(chunks * rank * widest) * sizeof(float);
     const size_t generic = ((g + 255) / 256) * 256 + part;
     // Enough for either path: which one runs depends on dtype and alignment.
-    const size_t fast = cf::lora_backward_fast_workspace_bytes(batch, in_features, out_features);
+    const size_t fast = cf::lora_backward_fast_workspace_bytes(batch, in_features, out_features, rank);
     return generic > fast ? generic : fast;
 }
 

@@ -10,23 +10,31 @@
 //
 // The work is two reductions over M of HBM-sized operands, so the design
 // reads dy once and x once (the HBM floor) and keeps everything else small:
-//   1. One pass over dy in 512-row x 256-column tiles (Mp = M rounded up to
-//      512), two 64-row chunks in flight per workgroup, loaded with the
-//      non-temporal hint (every byte is read once): each chunk goes
+//   1. One pass over dy in tiles of 512, 256 or 128 rows x 256 columns (Mp = M
+//      rounded up to 512), two 64-row chunks in flight per workgroup, loaded
+//      with the non-temporal hint (every byte is read once): each chunk goes
 //      HBM -> registers -> LDS; G partial rows = chunk @
 //      b^T (16x16x32 MFMA, row fragments by ds_read_b128, b fragments held in
-//      registers) and grad_b partials += bf16(xa)^T-chunk @ chunk (16x16x32
+//      registers up to rank 16, in LDS above) and grad_b partials +=
+//      bf16(xa)^T-chunk @ chunk (16x16x32
 //      MFMA; the chunk's fp32 xa arrives with one 16-byte load per thread
-//      and is rounded and transposed into LDS, the m-contiguous operand is
-//      read by ds_read_b64_tr_b16). Partials
+//      and 16 of rank and is rounded and transposed into LDS, the m-contiguous
+//      operand is read by ds_read_b64_tr_b16 and meets every block of 16 of
+//      the rank). Partials
 //      go to fp32 workspaces, one slice per 256-column tile (G) and per
-//      512-row tile (grad_b). 512-row tiles halve the grad_b/grad_a partials
-//      of 256-row ones (37.8 against 39.5 us at 8192 x 4096 x 4096 r16,
-//      operands cache-cold); three or four chunks in flight were slower.
+//      row tile (grad_b). Tall tiles mean few partials (512 rows against 256:
+//      37.8 against 39.5 us at 8192 x 4096 x 4096 r16, operands cache-cold),
+//      so they are lowered only until every CU has a workgroup; three or four
+//      chunks in flight were slower.
 //   2. One launch sums both in a fixed order: grad_b (times scale, cast) and
-//      G -> GT (bf16 [16, Mp]).
+//      G -> GT (bf16 [rank padded to 16, 32 or 64, Mp]).
 //   3. The same column-reduction pass over x with GT: grad_a partials.
 //   4. Their fixed-order sum, times scale, cast, stored transposed.
+// Measured, operands rotating: 2000 x 4096 x 4096 r64 31.9 us (1910 on the
+// generic path), r16 18.6 (23.7 with 512-row tiles), 4096 x 4096 x 4096 r16
+// 23.4 (26.3), 8192 x 4096 x 4096 r16 34.7 as before. The sums are compiled
+// per rank padding: with it as a variable they held 32 addresses in 130
+// registers and took 1.3 us longer.
 // Deterministic: every sum has a fixed order, no atomics.
 #include "cf_lora_bwd.hpp"
 
@@ -41,12 +49,12 @@ typedef float f32x4_t __attribute__((ext_vector_type(4)));
 typedef __attribute__((address_space(3))) s16x4_t lds_s16x4_t;
 typedef __attribute__((address_space(3))) uint8_t lds_u8_t;
 
-constexpr int kTileRows = 512;   // rows (M) per workgroup
+constexpr int kTileRows = 512;   // rows (M) per workgroup, at most
 constexpr int kTileCols = 256;   // columns per workgroup
 constexpr int kChunkRows = 64;   // rows staged in LDS at a time
 constexpr int kInFlight = 2;     // chunks loaded ahead per workgroup
 constexpr int kThreads = 256;
-constexpr int kRankPad = 16;     // adapter rank padded to one MFMA dimension
+constexpr int kMaxRank = 64;     // the rank is padded to 16, 32 or 64 (kRB MFMA blocks of 16)
 constexpr int kRowBytes = kTileCols * 2;
 constexpr int kPiecesPerThread = kChunkRows * kTileCols * 2 / 16 / kThreads;  // 8
 constexpr uint32_t kOutOfRange = 0x80000000u;
@@ -83,26 +91,32 @@ __device__ __forceinline__ uint32_t buffer_load4(__amdgpu_buffer_rsrc_t rsrc, ui
 
 struct ColumnArgs {
     const uint16_t* v;     // [M, C] bf16, the operand reduced over rows
-    const uint16_t* pt;    // [16, Mp] bf16, the other factor, m-contiguous (x pass)
+    const uint16_t* pt;    // [16 kRB, Mp] bf16, the other factor, m-contiguous (x pass)
     const float* xa;       // [M, rank] fp32, the other factor of the dy pass
     const uint16_t* b;     // [rank, C] bf16 (row-dot pass only)
-    float* colpart;        // [Mp / 256][16][C] fp32
-    float* gpart;          // [ceil(C / 256)][Mp][16] fp32 (row-dot pass only)
+    float* colpart;        // [row tiles][16 kRB][C] fp32
+    float* gpart;          // [ceil(C / 256)][Mp][16 kRB] fp32 (row-dot pass only)
     int64_t M;
     int64_t Mp;
     int64_t C;
     int64_t rank;
 };
 
-/// One kTileRows x 256-column tile of v: colpart[tile row][j][n] =
+/// One tile of kChunks x 64 rows and 256 columns of v: colpart[tile row][j][n] =
 /// sum_m pt[j, m] * v[m, n] over the tile's rows; with kRowDot also
 /// gpart[tile column][m][j] = sum_n v[m, n] * b[j, n] over its columns.
-template <bool kRowDot>
-__global__ __launch_bounds__(kThreads) void column_mfma_kernel(ColumnArgs args) {
+template <bool kRowDot, int kRB, int kChunks>
+__global__ __launch_bounds__(kThreads, kRB == 1 ? 1 : 2) void column_mfma_kernel(ColumnArgs args) {
+    constexpr int kRankPad = 16 * kRB;
+    constexpr int kXaLoads = kRB;  // 16-byte loads per thread of a chunk's xa (64 rows x rank fp32)
     __shared__ __attribute__((aligned(16))) uint8_t tile[kChunkRows * kRowBytes];  // 32 KiB
     // dy pass: the chunk's xa, rounded to bf16 and transposed ([16 j][64 m],
     // rows padded by 16 bytes); rows j >= rank stay zero.
     __shared__ __attribute__((aligned(16))) uint16_t xat[kRowDot ? kRankPad : 1][kXatStride];
+    // dy pass with more than one rank block: b's 256 columns (rows of 512
+    // bytes, laid out as the tile's); one block's fragments stay in registers.
+    constexpr bool kLdsB = kRowDot && kRB > 1;
+    __shared__ __attribute__((aligned(16))) uint8_t btile[kLdsB ? kRankPad * kRowBytes : 16];
 
     const int tid = static_cast<int>(threadIdx.x);
     const int lane = tid & 63;
@@ -112,7 +126,7 @@ __global__ __launch_bounds__(kThreads) void column_mfma_kernel(ColumnArgs args) 
     const int64_t C = args.C;
     const int64_t n0 = static_cast<int64_t>(blockIdx.x) * kTileCols;
     const int64_t mt = blockIdx.y;
-    const int64_t m0 = mt * kTileRows;
+    const int64_t m0 = mt * (kChunks * kChunkRows);
 
     // Staging roles: piece i of thread tid is row 8 i + tid / 32, chunk
     // tid % 32 of the chunk; one wave reads two 512-byte row segments.
@@ -127,24 +141,29 @@ __global__ __launch_bounds__(kThreads) void column_mfma_kernel(ColumnArgs args) 
     // with c % kInFlight == s (the chunk loop below is unrolled, so slots are
     // registers).
     uint4 staged[kInFlight][kPiecesPerThread];
-    // dy pass: thread t also loads bytes 16 t .. +15 of the chunk's xa rows
-    // (64 x rank fp32, contiguous), i.e. flat elements 4 t .. 4 t + 3:
-    // element q is xa[row0 + xa_row[q]][xa_col[q]].
-    uint4 staged_xa[kInFlight];
+    // dy pass: thread t also loads pieces t, t + 256, ... of the chunk's xa rows
+    // (64 x rank fp32, contiguous): element q of piece p is flat element
+    // 4 p + q = xa[row][col], stored at xat[col][row].
+    uint4 staged_xa[kInFlight][kXaLoads];
 #pragma unroll
-    for (int s = 0; s < kInFlight; ++s) staged_xa[s] = make_uint4(0u, 0u, 0u, 0u);
+    for (int s = 0; s < kInFlight; ++s) {
+#pragma unroll
+        for (int p = 0; p < kXaLoads; ++p) staged_xa[s][p] = make_uint4(0u, 0u, 0u, 0u);
+    }
     // x pass: the chunk's pt fragments, pt[j = lane % 16][row0 + 32 ms +
     // 8 (lane / 16) .. +7], loaded with the chunk so that waiting for them
     // never waits for a later chunk's loads.
-    bf16x8_t staged_pt[kInFlight][2];
-    int xa_row[4];
-    int xa_col[4];
+    bf16x8_t staged_pt[kInFlight][kRB][2];
+    int xat_at[kXaLoads][4];
     if constexpr (kRowDot) {
 #pragma unroll
-        for (int q = 0; q < 4; ++q) {
-            const int idx = 4 * tid + q;
-            xa_row[q] = idx / static_cast<int>(args.rank);
-            xa_col[q] = idx % static_cast<int>(args.rank);
+        for (int p = 0; p < kXaLoads; ++p) {
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+                const int idx = 4 * (tid + p * kThreads) + q;
+                const int rank = static_cast<int>(args.rank);
+                xat_at[p][q] = (idx % rank) * kXatStride + idx / rank;
+            }
         }
         // Rows j >= rank of the transposed chunk are never written: zero
         // them once (the loop's first barrier orders this before any read).
@@ -163,17 +182,24 @@ __global__ __launch_bounds__(kThreads) void column_mfma_kernel(ColumnArgs args) 
             staged[slot][i] = buffer_load16_stream(vbuf, off, 0);
         }
         if constexpr (kRowDot) {
-            // Past the chunk's kChunkRows x rank elements (rank < 16), or past
-            // M: zeros.
-            const uint32_t off = 4 * tid < kChunkRows * args.rank
-                                     ? static_cast<uint32_t>((row0 * args.rank + 4 * tid) * 4)
-                                     : kOutOfRange;
-            staged_xa[slot] = buffer_load16(xabuf, off, 0);
+            // Past the chunk's kChunkRows x rank elements, or past M: zeros.
+#pragma unroll
+            for (int p = 0; p < kXaLoads; ++p) {
+                const int at = 4 * (tid + p * kThreads);
+                const uint32_t off = at < kChunkRows * args.rank
+                                         ? static_cast<uint32_t>((row0 * args.rank + at) * 4)
+                                         : kOutOfRange;
+                staged_xa[slot][p] = buffer_load16(xabuf, off, 0);
+            }
         } else {
 #pragma unroll
-            for (int ms = 0; ms < 2; ++ms) {
-                const uint32_t off = static_cast<uint32_t>((jl * args.Mp + row0 + 32 * ms + 8 * g) * 2);
-                staged_pt[slot][ms] = as_bf16x8(buffer_load16(ptbuf, off, 0));
+            for (int rb = 0; rb < kRB; ++rb) {
+#pragma unroll
+                for (int ms = 0; ms < 2; ++ms) {
+                    const uint32_t off =
+                        static_cast<uint32_t>(((16 * rb + jl) * args.Mp + row0 + 32 * ms + 8 * g) * 2);
+                    staged_pt[slot][rb][ms] = as_bf16x8(buffer_load16(ptbuf, off, 0));
+                }
             }
         }
     };
@@ -184,12 +210,15 @@ __global__ __launch_bounds__(kThreads) void column_mfma_kernel(ColumnArgs args) 
             *reinterpret_cast<uint4*>(tile + tile_offset(row, piece_chunk)) = staged[slot][i];
         }
         if constexpr (kRowDot) {
-            if (4 * tid < kChunkRows * args.rank) {
-                const uint32_t v[4] = {staged_xa[slot].x, staged_xa[slot].y, staged_xa[slot].z,
-                                       staged_xa[slot].w};
+#pragma unroll
+            for (int p = 0; p < kXaLoads; ++p) {
+                if (4 * (tid + p * kThreads) >= kChunkRows * args.rank) continue;
+                const uint32_t v[4] = {staged_xa[slot][p].x, staged_xa[slot][p].y, staged_xa[slot][p].z,
+                                       staged_xa[slot][p].w};
 #pragma unroll
                 for (int q = 0; q < 4; ++q) {
-                    xat[xa_col[q]][xa_row[q]] = static_cast<uint16_t>(f32_to_bf16_bits(__uint_as_float(v[q])));
+                    (&xat[0][0])[xat_at[p][q]] =
+                        static_cast<uint16_t>(f32_to_bf16_bits(__uint_as_float(v[q])));
                 }
             }
         }
@@ -197,8 +226,19 @@ __global__ __launch_bounds__(kThreads) void column_mfma_kernel(ColumnArgs args) 
 
     // Row-dot role: wave w owns chunk rows 16 w .. +15; b fragment s holds
     // b[j = lane % 16][n0 + 32 s + 8 (lane / 16) .. +7].
-    bf16x8_t bfrag[8];
-    if constexpr (kRowDot) {
+    bf16x8_t bfrag[kLdsB ? 1 : 8];
+    if constexpr (kLdsB) {
+        const __amdgpu_buffer_rsrc_t bbuf =
+            make_buffer(args.b, static_cast<uint32_t>(args.rank * C * 2));
+#pragma unroll
+        for (int i = 0; i < kRankPad / 8; ++i) {
+            const int row = 8 * i + (tid >> 5);
+            const uint32_t off = row < args.rank && col_ok
+                                     ? static_cast<uint32_t>((row * C + piece_col) * 2)
+                                     : kOutOfRange;
+            *reinterpret_cast<uint4*>(btile + tile_offset(row, piece_chunk)) = buffer_load16(bbuf, off, 0);
+        }
+    } else if constexpr (kRowDot) {
         const __amdgpu_buffer_rsrc_t bbuf =
             make_buffer(args.b, static_cast<uint32_t>(args.rank * C * 2));
 #pragma unroll
@@ -214,11 +254,13 @@ __global__ __launch_bounds__(kThreads) void column_mfma_kernel(ColumnArgs args) 
     // Column-reduction role: wave w owns column blocks 4 w .. 4 w + 3 (16
     // columns each); accumulator lane holds [j = 4 (lane / 16) + t][column
     // 16 cb + lane % 16].
-    f32x4_t acc[4];
+    f32x4_t acc[kRB][4];
 #pragma unroll
-    for (int c = 0; c < 4; ++c) acc[c] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
+    for (int rb = 0; rb < kRB; ++rb) {
+#pragma unroll
+        for (int c = 0; c < 4; ++c) acc[rb][c] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
+    }
 
-    constexpr int kChunks = kTileRows / kChunkRows;
 #pragma unroll
     for (int c = 0; c < kInFlight && c < kChunks; ++c) load_chunk(c, m0 + c * kChunkRows);
 #pragma unroll
@@ -232,13 +274,17 @@ __global__ __launch_bounds__(kThreads) void column_mfma_kernel(ColumnArgs args) 
         // pt fragments. The dy pass reads them from the transposed bf16 copy
         // of the chunk's xa in LDS (rounded as the transposed copy of the x
         // pass is); rows past M and columns past the rank are zero.
-        bf16x8_t ptfrag[2];
+        bf16x8_t ptfrag[kRB][2];
 #pragma unroll
-        for (int ms = 0; ms < 2; ++ms) {
-            if constexpr (kRowDot) {
-                ptfrag[ms] = *reinterpret_cast<const bf16x8_t*>(&xat[jl][32 * ms + 8 * g]);
-            } else {
-                ptfrag[ms] = staged_pt[slot][ms];
+        for (int rb = 0; rb < kRB; ++rb) {
+#pragma unroll
+            for (int ms = 0; ms < 2; ++ms) {
+                if constexpr (kRowDot) {
+                    ptfrag[rb][ms] =
+                        *reinterpret_cast<const bf16x8_t*>(&xat[16 * rb + jl][32 * ms + 8 * g]);
+                } else {
+                    ptfrag[rb][ms] = staged_pt[slot][rb][ms];
+                }
             }
         }
         if (chunk + kInFlight < kChunks) load_chunk(slot, row0 + kInFlight * kChunkRows);
@@ -255,35 +301,56 @@ __global__ __launch_bounds__(kThreads) void column_mfma_kernel(ColumnArgs args) 
                 // recompute rather than add.
                 const int off_hi = tile_offset(row + 4, ch) + (jl & 1) * 8;
                 const bf16x8_t vfrag = concat(lds_read_tr(tile, off), lds_read_tr(tile, off_hi));
-                acc[c] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ptfrag[ms], vfrag, acc[c], 0, 0, 0);
+#pragma unroll
+                for (int rb = 0; rb < kRB; ++rb) {
+                    acc[rb][c] =
+                        __builtin_amdgcn_mfma_f32_16x16x32_bf16(ptfrag[rb][ms], vfrag, acc[rb][c], 0, 0, 0);
+                }
             }
         }
 
         if constexpr (kRowDot) {
-            f32x4_t gacc = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
+            f32x4_t gacc[kRB];
+#pragma unroll
+            for (int rb = 0; rb < kRB; ++rb) gacc[rb] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
             const int row = 16 * wave + jl;
 #pragma unroll
             for (int s = 0; s < 8; ++s) {
                 const bf16x8_t afrag =
                     *reinterpret_cast<const bf16x8_t*>(tile + tile_offset(row, 4 * s + g));
-                gacc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(afrag, bfrag[s], gacc, 0, 0, 0);
+#pragma unroll
+                for (int rb = 0; rb < kRB; ++rb) {
+                    bf16x8_t fb;
+                    if constexpr (kLdsB) {
+                        fb = *reinterpret_cast<const bf16x8_t*>(btile + tile_offset(16 * rb + jl, 4 * s + g));
+                    } else {
+                        fb = bfrag[s];
+                    }
+                    gacc[rb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(afrag, fb, gacc[rb], 0, 0, 0);
+                }
             }
-            // gacc lane holds G[row 16 wave + 4 (lane / 16) + t][j = lane % 16].
+            // gacc[rb] lane holds G[row 16 wave + 4 (lane / 16) + t][j = 16 rb + lane % 16].
             float* gp = args.gpart + (static_cast<int64_t>(blockIdx.x) * args.Mp + row0 +
                                       16 * wave + 4 * g) * kRankPad + jl;
 #pragma unroll
-            for (int t = 0; t < 4; ++t) gp[t * kRankPad] = gacc[t];
+            for (int rb = 0; rb < kRB; ++rb) {
+#pragma unroll
+                for (int t = 0; t < 4; ++t) gp[t * kRankPad + 16 * rb] = gacc[rb][t];
+            }
         }
     }
 
-    // colpart[mt][j][n]: lane holds j = 4 (lane / 16) + t, n = n0 + 16 cb + lane % 16.
+    // colpart[mt][j][n]: lane holds j = 16 rb + 4 (lane / 16) + t, n = n0 + 16 cb + lane % 16.
 #pragma unroll
     for (int c = 0; c < 4; ++c) {
         const int64_t col = n0 + 16 * (4 * wave + c) + jl;
         if (col >= C) continue;
 #pragma unroll
-        for (int t = 0; t < 4; ++t) {
-            args.colpart[(mt * kRankPad + 4 * g + t) * C + col] = acc[c][t];
+        for (int rb = 0; rb < kRB; ++rb) {
+#pragma unroll
+            for (int t = 0; t < 4; ++t) {
+                args.colpart[(mt * kRankPad + 16 * rb + 4 * g + t) * C + col] = acc[rb][c][t];
+            }
         }
     }
 }
@@ -314,20 +381,23 @@ __device__ __forceinline__ float ordered_sum(int64_t tiles, At at) {
 
 /// gt[j, m] = bf16(sum over column tiles of gpart[tile][m][j]), fixed order;
 /// thread i of the launch handles element i.
+template <int kRankPad>
 __device__ __forceinline__ void sum_g(const float* __restrict__ gpart, uint16_t* __restrict__ gt,
-                                      int64_t Mp, int64_t tiles, int64_t i) {
+                                      int64_t M, int64_t Mp, int64_t tiles, int64_t i) {
     if (i >= kRankPad * Mp) return;
     const int64_t m = i / kRankPad;
     const int64_t j = i % kRankPad;
-    const float total =
-        ordered_sum(tiles, [&](int64_t t) { return gpart[(t * Mp + m) * kRankPad + j]; });
+    // Rows past M are zero, whether or not the dy pass's tiles reach them
+    // (the x pass's may be taller).
+    float total = 0.0f;
+    if (m < M) total = ordered_sum(tiles, [&](int64_t t) { return gpart[(t * Mp + m) * kRankPad + j]; });
     gt[j * Mp + m] = static_cast<uint16_t>(f32_to_bf16_bits(total));
 }
 
 /// out = scale * sum over row tiles of colpart[tile][j][n], j < rank, as
 /// [rank, C] or (kTransposed) [C, rank]; fixed order; thread i handles
 /// element i.
-template <bool kTransposed>
+template <bool kTransposed, int kRankPad>
 __device__ __forceinline__ void finish(const float* __restrict__ colpart, uint16_t* __restrict__ out,
                                        int64_t tiles, int64_t rank, int64_t C, float scale, int64_t i) {
     if (i >= rank * C) return;
@@ -341,27 +411,30 @@ __device__ __forceinline__ void finish(const float* __restrict__ colpart, uint16
 
 /// After the dy pass: grad_b's fixed-order sum (first grad_b_blocks
 /// workgroups) and G's (the rest) are independent, so one launch does both.
+template <int kRankPad>
 __global__ __launch_bounds__(kThreads) void after_dy_kernel(const float* __restrict__ colpart,
                                                             uint16_t* __restrict__ grad_b,
                                                             const float* __restrict__ gpart,
                                                             uint16_t* __restrict__ gt,
                                                             int64_t grad_b_blocks, int64_t row_tiles,
                                                             int64_t rank, int64_t N, float scale,
-                                                            int64_t Mp, int64_t col_tiles) {
+                                                            int64_t M, int64_t Mp,
+                                                            int64_t col_tiles) {
     const int64_t block = blockIdx.x;
     if (block < grad_b_blocks) {
-        finish<false>(colpart, grad_b, row_tiles, rank, N, scale, block * kThreads + threadIdx.x);
+        finish<false, kRankPad>(colpart, grad_b, row_tiles, rank, N, scale, block * kThreads + threadIdx.x);
     } else {
-        sum_g(gpart, gt, Mp, col_tiles, (block - grad_b_blocks) * kThreads + threadIdx.x);
+        sum_g<kRankPad>(gpart, gt, M, Mp, col_tiles, (block - grad_b_blocks) * kThreads + threadIdx.x);
     }
 }
 
 /// grad_a's fixed-order sum after the x pass, stored transposed ([K, rank]).
+template <int kRankPad>
 __global__ __launch_bounds__(kThreads) void finish_grad_a_kernel(const float* __restrict__ colpart,
                                                                  uint16_t* __restrict__ grad_a,
                                                                  int64_t row_tiles, int64_t rank,
                                                                  int64_t K, float scale) {
-    finish<true>(colpart, grad_a, row_tiles, rank, K, scale,
+    finish<true, kRankPad>(colpart, grad_a, row_tiles, rank, K, scale,
                  static_cast<int64_t>(blockIdx.x) * kThreads + threadIdx.x);
 }
 
@@ -373,38 +446,82 @@ struct Workspace {
 
 size_t align256(size_t bytes) { return (bytes + 255) / 256 * 256; }
 
-Workspace carve(void* base, int64_t M, int64_t K, int64_t N) {
-    const int64_t Mp = ceil_div<int64_t>(M, kTileRows) * kTileRows;
+int rank_pad_of(int64_t rank) { return rank <= 16 ? 16 : rank <= 32 ? 32 : 64; }
+
+/// Chunks of 64 rows per workgroup: 8, 4 or 2, the most that still give the
+/// pass over `cols` columns a workgroup per CU (partials grow as it shrinks);
+/// at most 4 for four rank blocks, whose eight unrolled chunks spill.
+int chunks_for(int64_t M, int64_t cols, int rank_pad) {
+    const int64_t tiles = ceil_div<int64_t>(cols, kTileCols);
+    for (int chunks = rank_pad == 64 ? 4 : 8; chunks > 2; chunks /= 2) {
+        if (ceil_div<int64_t>(M, chunks * kChunkRows) * tiles >= 256) return chunks;
+    }
+    return 2;
+}
+
+int64_t padded_rows(int64_t M) { return ceil_div<int64_t>(M, kTileRows) * kTileRows; }
+
+size_t colpart_bytes(int64_t M, int64_t cols, int rank_pad) {
+    return static_cast<size_t>(ceil_div<int64_t>(M, chunks_for(M, cols, rank_pad) * kChunkRows) * rank_pad * cols) * 4;
+}
+
+Workspace carve(void* base, int64_t M, int64_t N, int rank_pad) {
+    const int64_t Mp = padded_rows(M);
     uint8_t* p = static_cast<uint8_t*>(base);
     Workspace ws;
     ws.gt = reinterpret_cast<uint16_t*>(p);
-    p += align256(static_cast<size_t>(kRankPad * Mp) * 2);
+    p += align256(static_cast<size_t>(rank_pad * Mp) * 2);
     ws.gpart = reinterpret_cast<float*>(p);
-    p += align256(static_cast<size_t>(ceil_div<int64_t>(N, kTileCols) * Mp * kRankPad) * 4);
+    p += align256(static_cast<size_t>(ceil_div<int64_t>(N, kTileCols) * Mp * rank_pad) * 4);
     ws.colpart = reinterpret_cast<float*>(p);
-    (void)K;
     return ws;
+}
+
+template <bool kRowDot, int kRB>
+void launch_pass(const ColumnArgs& args, int chunks, hipStream_t stream) {
+    const dim3 grid(static_cast<unsigned>(ceil_div<int64_t>(args.C, kTileCols)),
+                    static_cast<unsigned>(ceil_div<int64_t>(args.M, chunks * kChunkRows)));
+    if (kRB < 4 && chunks == 8) {
+        launch(column_mfma_kernel<kRowDot, kRB < 4 ? kRB : 1, 8>, grid, dim3(kThreads), 0, stream, args);
+    } else if (chunks == 4) {
+        launch(column_mfma_kernel<kRowDot, kRB, 4>, grid, dim3(kThreads), 0, stream, args);
+    } else {
+        launch(column_mfma_kernel<kRowDot, kRB, 2>, grid, dim3(kThreads), 0, stream, args);
+    }
+}
+
+template <bool kRowDot>
+void launch_pass(const ColumnArgs& args, int rank_pad, int chunks, hipStream_t stream) {
+    if (rank_pad == 16) {
+        launch_pass<kRowDot, 1>(args, chunks, stream);
+    } else if (rank_pad == 32) {
+        launch_pass<kRowDot, 2>(args, chunks, stream);
+    } else {
+        launch_pass<kRowDot, 4>(args, chunks, stream);
+    }
 }
 
 }  // namespace
 
-size_t lora_backward_fast_workspace_bytes(int64_t M, int64_t K, int64_t N) {
-    if (M <= 0) return 0;
-    const int64_t Mp = ceil_div<int64_t>(M, kTileRows) * kTileRows;
-    const int64_t widest = K > N ? K : N;
-    return align256(static_cast<size_t>(kRankPad * Mp) * 2) +
-           align256(static_cast<size_t>(ceil_div<int64_t>(N, kTileCols) * Mp * kRankPad) * 4) +
-           static_cast<size_t>(Mp / kTileRows * kRankPad * widest) * 4;
+size_t lora_backward_fast_workspace_bytes(int64_t M, int64_t K, int64_t N, int64_t rank) {
+    if (M <= 0 || rank > kMaxRank) return 0;
+    const int64_t Mp = padded_rows(M);
+    const int rank_pad = rank_pad_of(rank);
+    const size_t dy = colpart_bytes(M, N, rank_pad);
+    const size_t x = colpart_bytes(M, K, rank_pad);
+    return align256(static_cast<size_t>(rank_pad * Mp) * 2) +
+           align256(static_cast<size_t>(ceil_div<int64_t>(N, kTileCols) * Mp * rank_pad) * 4) +
+           (dy > x ? dy : x);
 }
 
 bool lora_backward_fast_eligible(const void* x, const void* dy, const void* b, int64_t M,
                                  int64_t K, int64_t N, int64_t rank) {
     // Buffer offsets are 32-bit with an out-of-range marker at 2^31.
-    const int64_t Mp = ceil_div<int64_t>(M, kTileRows) * kTileRows;
+    const int64_t Mp = padded_rows(M);
     const bool fits = Mp * K * 2 < (1LL << 31) && Mp * N * 2 < (1LL << 31) &&
-                      rank * N * 2 < (1LL << 31) && kRankPad * Mp * 2 < (1LL << 31) &&
+                      rank * N * 2 < (1LL << 31) && kMaxRank * Mp * 2 < (1LL << 31) &&
                       Mp * rank * 4 < (1LL << 31);
-    return M > 0 && K > 0 && N > 0 && rank > 0 && rank <= kRankPad && K % 8 == 0 && N % 8 == 0 &&
+    return M > 0 && K > 0 && N > 0 && rank > 0 && rank <= kMaxRank && K % 8 == 0 && N % 8 == 0 &&
            fits && host_aligned(x, 16) && host_aligned(dy, 16) && host_aligned(b, 16);
 }
 
@@ -412,10 +529,9 @@ cf_status launch_lora_backward_fast(const void* x, const void* dy, const void* b
                                     void* grad_a, void* grad_b, int64_t M, int64_t K, int64_t N,
                                     int64_t rank, float scale, void* workspace,
                                     hipStream_t stream) {
-    const int64_t Mp = ceil_div<int64_t>(M, kTileRows) * kTileRows;
-    const int64_t row_tiles = Mp / kTileRows;
-    const Workspace ws = carve(workspace, M, K, N);
-    const unsigned small_grid = static_cast<unsigned>(ceil_div<int64_t>(kRankPad * Mp, kThreads));
+    const int64_t Mp = padded_rows(M);
+    const int rank_pad = rank_pad_of(rank);
+    const Workspace ws = carve(workspace, M, N, rank_pad);
 
     ColumnArgs dy_pass;
     dy_pass.v = static_cast<const uint16_t*>(dy);
@@ -428,14 +544,19 @@ cf_status launch_lora_backward_fast(const void* x, const void* dy, const void* b
     dy_pass.Mp = Mp;
     dy_pass.C = N;
     dy_pass.rank = rank;
-    const int64_t n_tiles = ceil_div<int64_t>(N, kTileCols);
-    launch(column_mfma_kernel<true>,
-           dim3(dim3(static_cast<unsigned>(n_tiles), static_cast<unsigned>(row_tiles))),
-           dim3(kThreads), 0, stream, dy_pass);
+    const int dy_chunks = chunks_for(M, N, rank_pad);
+    launch_pass<true>(dy_pass, rank_pad, dy_chunks, stream);
     const int64_t grad_b_blocks = ceil_div<int64_t>(rank * N, kThreads);
-    launch(after_dy_kernel, dim3(static_cast<unsigned>(grad_b_blocks + small_grid)), dim3(kThreads),
-           0, stream, ws.colpart, static_cast<uint16_t*>(grad_b), ws.gpart, ws.gt, grad_b_blocks,
-           row_tiles, rank, N, scale, Mp, n_tiles);
+    const int64_t g_blocks = ceil_div<int64_t>(rank_pad * Mp, kThreads);
+    auto after_dy = [&](auto kernel) {
+        launch(kernel, dim3(static_cast<unsigned>(grad_b_blocks + g_blocks)), dim3(kThreads), 0, stream,
+               ws.colpart, static_cast<uint16_t*>(grad_b), ws.gpart, ws.gt, grad_b_blocks,
+               ceil_div<int64_t>(M, dy_chunks * kChunkRows), rank, N, scale, M, Mp,
+               ceil_div<int64_t>(N, kTileCols));
+    };
+    rank_pad == 16   ? after_dy(after_dy_kernel<16>)
+    : rank_pad == 32 ? after_dy(after_dy_kernel<32>)
+                     : after_dy(after_dy_kernel<64>);
 
     ColumnArgs x_pass;
     x_pass.v = static_cast<const uint16_t*>(x);
@@ -448,13 +569,16 @@ cf_status launch_lora_backward_fast(const void* x, const void* dy, const void* b
     x_pass.Mp = Mp;
     x_pass.C = K;
     x_pass.rank = rank;
-    const int64_t k_tiles = ceil_div<int64_t>(K, kTileCols);
-    launch(column_mfma_kernel<false>,
-           dim3(dim3(static_cast<unsigned>(k_tiles), static_cast<unsigned>(row_tiles))),
-           dim3(kThreads), 0, stream, x_pass);
-    launch(finish_grad_a_kernel, dim3(static_cast<unsigned>(ceil_div<int64_t>(rank * K, kThreads))),
-           dim3(kThreads), 0, stream, ws.colpart, static_cast<uint16_t*>(grad_a), row_tiles, rank,
-           K, scale);
+    const int x_chunks = chunks_for(M, K, rank_pad);
+    launch_pass<false>(x_pass, rank_pad, x_chunks, stream);
+    auto finish_grad_a = [&](auto kernel) {
+        launch(kernel, dim3(static_cast<unsigned>(ceil_div<int64_t>(rank * K, kThreads))), dim3(kThreads), 0,
+               stream, ws.colpart, static_cast<uint16_t*>(grad_a),
+               ceil_div<int64_t>(M, x_chunks * kChunkRows), rank, K, scale);
+    };
+    rank_pad == 16   ? finish_grad_a(finish_grad_a_kernel<16>)
+    : rank_pad == 32 ? finish_grad_a(finish_grad_a_kernel<32>)
+                     : finish_grad_a(finish_grad_a_kernel<64>);
     return check_launch("launching the bf16 LoRA backward", stream);
 }
 

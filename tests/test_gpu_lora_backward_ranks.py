@@ -1,0 +1,35 @@
+"""The bf16 adapter backward above rank 16 (rank blocks of 16, b in LDS) and
+its row tiles of 128, 256 and 512 rows, against the float64 oracle: ranks at
+and off the block edges, tiles of different heights in the dy and x passes
+(rows past M between them), ragged rows and columns, poisoned workspace."""
+
+from __future__ import annotations
+
+import numpy as np
+import pytest
+
+import oracle
+
+from . import gpu_util as g
+from .test_gpu_lora import assert_gemm_close, rng, run_backward
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("shape", [
+    (1, 8, 8, 17), (100, 64, 11008, 32), (130, 11008, 72, 33), (333, 4096, 264, 64), (700, 264, 4096, 48),
+    (1000, 1032, 2048, 24), (2000, 4096, 4096, 64), (4096, 2048, 1024, 32), (64, 688, 256, 16), (520, 256, 4104, 5),
+], ids=str)
+def test_backward_ranks_and_row_tiles(shape):
+    m, k, n, r = shape
+    g.announce(f"adapter backward bf16 {shape}")
+    gen = rng(sum(shape))
+    x = g.storage_bits(gen.standard_normal((m, k)).astype(np.float32), "bf16")
+    dy = g.storage_bits(gen.standard_normal((m, n)).astype(np.float32), "bf16")
+    b = g.storage_bits((0.02 * gen.standard_normal((r, n))).astype(np.float32), "bf16")
+    xa = (gen.standard_normal((m, r)) * 0.5).astype(np.float32)
+    ga, gb = run_backward(x, dy, b, xa, "bf16", 0.5)
+    exact_a, exact_b = oracle.lora_backward(
+        g.host_values(x, "bf16"), g.host_values(dy, "bf16"), g.host_values(b, "bf16"), xa, 0.5, True)
+    assert_gemm_close(ga, exact_a, "bf16", f"grad_a {shape}")
+    assert_gemm_close(gb, exact_b, "bf16", f"grad_b {shape}")
