@@ -99,6 +99,10 @@ SIGNATURES: dict[str, tuple[object, list[object]]] = {
         _I32,
         [_P, _P, _P, _P, _P, _P, _I32, _I64, _I64, _I64, _I64, _F, _P, _SZ, _P],
     ),
+    "cf_lora_backward_input": (
+        _I32,
+        [_P, _P, _P, _P, _P, _P, _P, _P, _I32, _I64, _I64, _I64, _I64, _F, _P, _SZ, _P],
+    ),
     "cf_silu": (_I32, [_P, _P, _I32, _I64, _P]),
     "cf_gelu": (_I32, [_P, _P, _I32, _I64, _P]),
     "cf_swiglu": (_I32, [_P, _P, _P, _I32, _I64, _P]),

@@ -11,9 +11,12 @@ adapter intermediate ``x @ a`` it computes anyway, and the backward computes
 
 with HIP kernels (cf_lora_backward). These are the gradients ATen autograd
 produces for the reference composition (tests/python/test_autograd.py:81-91).
-The gradients of x and w, which a LoRA layer rarely needs (the base weight is
-frozen; x needs one only below the first adapted layer), are plain GEMMs and
-go to the vendor BLAS through torch.
+The gradient of x is a plain GEMM, dy @ w^T, which goes to the vendor BLAS, plus
+the adapter's rank-r part, which a HIP kernel adds in place from the dy @ b^T
+that the adapter gradients need anyway. The gradient of w (the base weight is
+usually frozen) is a plain GEMM too. When the backward itself is recorded
+(create_graph) the gradient of x is composed from torch operators, which can
+be differentiated again.
 """
 
 from __future__ import annotations
@@ -34,9 +37,15 @@ class _LoRALinearFunction(torch.autograd.Function):
         x, weight, lora_a, lora_b, xa = ctx.saved_tensors
         grad_y = grad_y.contiguous()
         grad_x = grad_w = grad_a = grad_b = None
-        if ctx.needs_input_grad[2] or ctx.needs_input_grad[3]:
+        adapter_grads = ctx.needs_input_grad[2] or ctx.needs_input_grad[3]
+        fused_x = (adapter_grads and ctx.needs_input_grad[0] and not torch.is_grad_enabled()
+                   and x.dtype == torch.bfloat16)
+        if fused_x:
+            grad_x, grad_a, grad_b = torch.ops.cudaforge.lora_linear_bwd_input(
+                x, grad_y, weight, lora_a, lora_b, xa, ctx.scale)
+        elif adapter_grads:
             grad_a, grad_b = torch.ops.cudaforge.lora_linear_bwd(x, grad_y, lora_b, xa, ctx.scale)
-        if ctx.needs_input_grad[0]:
+        if ctx.needs_input_grad[0] and not fused_x:
             adapter = (grad_y @ lora_b.t()) @ lora_a.t()
             grad_x = grad_y @ weight.t() + ctx.scale * adapter
         if ctx.needs_input_grad[1]:

@@ -24,6 +24,7 @@
 //   G      = dy @ b^T            [M, r]
 //   grad_b = scale * xa^T @ dy   [r, N]   column reduction over M
 //   grad_a = scale * x^T @ G     [K, r]   column reduction over M
+//   grad_x = dy @ w^T (the caller's GEMM) + scale * G @ a^T, in place
 // bf16 with rank <= 64 runs the MFMA kernels of cf_lora_bwd.hip. The generic
 // path here (fp32, other shapes): G one wave per row of dy, the column
 // reductions in row chunks into an fp32 workspace and a second kernel summing
@@ -252,6 +253,59 @@ cf_status column_reduce(const float* p, const void* v, void* out, bool transpose
                part, static_cast<T*>(out), chunks, rank, cols, scale);
     }
     return check_launch("launching the LoRA backward column reduction", stream);
+}
+
+constexpr int kUpdateRowsGeneric = 8;
+
+/// grad_x += scale * round_T(g) @ a^T: a thread per column and 8 rows, g's
+/// rows broadcast from LDS 16 adapter columns at a time.
+template <typename T>
+__global__ __launch_bounds__(kDefaultBlockSize) void adapter_update_kernel(
+    const float* __restrict__ g, const T* __restrict__ a, T* __restrict__ grad_x, int64_t rows,
+    int64_t cols, int64_t rank, float scale) {
+    __shared__ float gs[kUpdateRowsGeneric][16];
+    const int tid = static_cast<int>(threadIdx.x);
+    const int64_t k = static_cast<int64_t>(blockIdx.x) * kDefaultBlockSize + tid;
+    const int64_t row0 = static_cast<int64_t>(blockIdx.y) * kUpdateRowsGeneric;
+    float acc[kUpdateRowsGeneric];
+#pragma unroll
+    for (int i = 0; i < kUpdateRowsGeneric; ++i) acc[i] = 0.0f;
+    for (int64_t j0 = 0; j0 < rank; j0 += 16) {
+        __syncthreads();
+        for (int e = tid; e < kUpdateRowsGeneric * 16; e += kDefaultBlockSize) {
+            const int64_t row = row0 + e / 16;
+            const int64_t j = j0 + e % 16;
+            gs[e / 16][e % 16] = row < rows && j < rank ? round_to<T>(g[row * rank + j]) : 0.0f;
+        }
+        float av[16];
+#pragma unroll
+        for (int j = 0; j < 16; ++j) {
+            av[j] = k < cols && j0 + j < rank ? Storage<T>::load(a + k * rank + j0 + j) : 0.0f;
+        }
+        __syncthreads();
+#pragma unroll
+        for (int i = 0; i < kUpdateRowsGeneric; ++i) {
+#pragma unroll
+            for (int j = 0; j < 16; ++j) acc[i] += gs[i][j] * av[j];
+        }
+    }
+    if (k >= cols) return;
+#pragma unroll
+    for (int i = 0; i < kUpdateRowsGeneric; ++i) {
+        if (row0 + i < rows) {
+            T* dst = grad_x + (row0 + i) * cols + k;
+            Storage<T>::store(dst, Storage<T>::load(dst) + scale * acc[i]);
+        }
+    }
+}
+
+template <typename T>
+void launch_adapter_update(const float* g, const void* a, void* grad_x, int64_t rows, int64_t cols,
+                           int64_t rank, float scale, hipStream_t stream) {
+    const dim3 grid(static_cast<unsigned>(ceil_div<int64_t>(cols, kDefaultBlockSize)),
+                    static_cast<unsigned>(ceil_div<int64_t>(rows, kUpdateRowsGeneric)));
+    launch(adapter_update_kernel<T>, grid, dim3(kDefaultBlockSize), 0, stream, g, static_cast<const T*>(a),
+           static_cast<T*>(grad_x), rows, cols, rank, scale);
 }
 
 template <typename T>
@@ -501,6 +555,16 @@ cf_status cf_lora_backward(const void* x, const void* dy, const void* b, const f
                            void* grad_a, void* grad_b, cf_dtype dtype, int64_t batch,
                            int64_t in_features, int64_t out_features, int64_t rank, float scale,
                            void* workspace, size_t workspace_bytes, void* stream) {
+    return cf_lora_backward_input(x, dy, nullptr, b, xa, grad_a, grad_b, nullptr, dtype, batch,
+                                  in_features, out_features, rank, scale, workspace, workspace_bytes,
+                                  stream);
+}
+
+cf_status cf_lora_backward_input(const void* x, const void* dy, const void* a, const void* b,
+                                 const float* xa, void* grad_a, void* grad_b, void* grad_x,
+                                 cf_dtype dtype, int64_t batch, int64_t in_features,
+                                 int64_t out_features, int64_t rank, float scale, void* workspace,
+                                 size_t workspace_bytes, void* stream) {
     CF_ENTRY();
     if (rank <= 0) return CF_OK;
     CF_REQUIRE(batch >= 0 && in_features >= 0 && out_features >= 0,
@@ -519,16 +583,17 @@ cf_status cf_lora_backward(const void* x, const void* dy, const void* b, const f
     }
     CF_REQUIRE(x != nullptr && dy != nullptr && b != nullptr && xa != nullptr,
                "cf_lora_backward: null input");
+    CF_REQUIRE(grad_x == nullptr || a != nullptr, "cf_lora_backward_input: null adapter");
     const size_t needed = cf_lora_backward_workspace_bytes(batch, in_features, out_features, rank);
     CF_REQUIRE(workspace != nullptr && workspace_bytes >= needed,
                "cf_lora_backward: workspace of %zu bytes given, %zu needed", workspace_bytes,
                needed);
     CF_REQUIRE(cf::host_aligned(workspace, 16), "cf_lora_backward: workspace must be 16-byte aligned");
     auto s = static_cast<hipStream_t>(stream);
-    if (dtype == CF_BF16 && cf::lora_backward_fast_eligible(x, dy, b, batch, in_features,
+    if (dtype == CF_BF16 && cf::lora_backward_fast_eligible(x, dy, b, grad_x, batch, in_features,
                                                             out_features, rank)) {
-        return cf::launch_lora_backward_fast(x, dy, b, xa, grad_a, grad_b, batch, in_features,
-                                             out_features, rank, scale, workspace, s);
+        return cf::launch_lora_backward_fast(x, dy, a, b, xa, grad_a, grad_b, grad_x, batch,
+                                             in_features, out_features, rank, scale, workspace, s);
     }
     float* g = static_cast<float*>(workspace);
     const size_t g_bytes = ((static_cast<size_t>(batch * rank) * sizeof(float) + 255) / 256) * 256;
@@ -538,6 +603,9 @@ cf_status cf_lora_backward(const void* x, const void* dy, const void* b, const f
         cf_status st = cf::column_reduce<float>(xa, dy, grad_b, false, batch, out_features, rank,
                                                 scale, part, s);
         if (st != CF_OK) return st;
+        if (grad_x != nullptr) {
+            cf::launch_adapter_update<float>(g, a, grad_x, batch, in_features, rank, scale, s);
+        }
         return cf::column_reduce<float>(g, x, grad_a, true, batch, in_features, rank, scale, part,
                                         s);
     }
@@ -545,6 +613,9 @@ cf_status cf_lora_backward(const void* x, const void* dy, const void* b, const f
     cf_status st = cf::column_reduce<cf::bf16_t>(xa, dy, grad_b, false, batch, out_features, rank,
                                                  scale, part, s);
     if (st != CF_OK) return st;
+    if (grad_x != nullptr) {
+        cf::launch_adapter_update<cf::bf16_t>(g, a, grad_x, batch, in_features, rank, scale, s);
+    }
     return cf::column_reduce<cf::bf16_t>(g, x, grad_a, true, batch, in_features, rank, scale, part,
                                          s);
 }

@@ -30,6 +30,7 @@
 //      G -> GT (bf16 [rank padded to 16, 32 or 64, Mp]).
 //   3. The same column-reduction pass over x with GT: grad_a partials.
 //   4. Their fixed-order sum, times scale, cast, stored transposed.
+//   5. With grad_x (dy @ w^T from the caller's GEMM): += scale * G @ a^T.
 // Measured, operands rotating: 2000 x 4096 x 4096 r64 31.9 us (1910 on the
 // generic path), r16 18.6 (23.7 with 512-row tiles), 4096 x 4096 x 4096 r16
 // 23.4 (26.3), 8192 x 4096 x 4096 r16 34.7 as before. The sums are compiled
@@ -379,11 +380,12 @@ __device__ __forceinline__ float ordered_sum(int64_t tiles, At at) {
     return total;
 }
 
-/// gt[j, m] = bf16(sum over column tiles of gpart[tile][m][j]), fixed order;
-/// thread i of the launch handles element i.
+/// gt[j, m] = bf16(sum over column tiles of gpart[tile][m][j]), fixed order,
+/// and the same row by row in g when that is wanted; thread i of the launch
+/// handles element i.
 template <int kRankPad>
 __device__ __forceinline__ void sum_g(const float* __restrict__ gpart, uint16_t* __restrict__ gt,
-                                      int64_t M, int64_t Mp, int64_t tiles, int64_t i) {
+                                      uint16_t* __restrict__ g, int64_t M, int64_t Mp, int64_t tiles, int64_t i) {
     if (i >= kRankPad * Mp) return;
     const int64_t m = i / kRankPad;
     const int64_t j = i % kRankPad;
@@ -391,7 +393,9 @@ __device__ __forceinline__ void sum_g(const float* __restrict__ gpart, uint16_t*
     // (the x pass's may be taller).
     float total = 0.0f;
     if (m < M) total = ordered_sum(tiles, [&](int64_t t) { return gpart[(t * Mp + m) * kRankPad + j]; });
-    gt[j * Mp + m] = static_cast<uint16_t>(f32_to_bf16_bits(total));
+    const uint16_t bits = static_cast<uint16_t>(f32_to_bf16_bits(total));
+    gt[j * Mp + m] = bits;
+    if (g != nullptr) g[i] = bits;
 }
 
 /// out = scale * sum over row tiles of colpart[tile][j][n], j < rank, as
@@ -416,6 +420,7 @@ __global__ __launch_bounds__(kThreads) void after_dy_kernel(const float* __restr
                                                             uint16_t* __restrict__ grad_b,
                                                             const float* __restrict__ gpart,
                                                             uint16_t* __restrict__ gt,
+                                                            uint16_t* __restrict__ g,
                                                             int64_t grad_b_blocks, int64_t row_tiles,
                                                             int64_t rank, int64_t N, float scale,
                                                             int64_t M, int64_t Mp,
@@ -424,7 +429,7 @@ __global__ __launch_bounds__(kThreads) void after_dy_kernel(const float* __restr
     if (block < grad_b_blocks) {
         finish<false, kRankPad>(colpart, grad_b, row_tiles, rank, N, scale, block * kThreads + threadIdx.x);
     } else {
-        sum_g<kRankPad>(gpart, gt, M, Mp, col_tiles, (block - grad_b_blocks) * kThreads + threadIdx.x);
+        sum_g<kRankPad>(gpart, gt, g, M, Mp, col_tiles, (block - grad_b_blocks) * kThreads + threadIdx.x);
     }
 }
 
@@ -438,8 +443,110 @@ __global__ __launch_bounds__(kThreads) void finish_grad_a_kernel(const float* __
                  static_cast<int64_t>(blockIdx.x) * kThreads + threadIdx.x);
 }
 
+constexpr int kUpdateCols = 256;  // columns of a workgroup
+
+/// Rows of a workgroup: the smallest a is cheaper to read again than to hold
+/// fewer workgroups for (4096 x 4096 r16 17.1 us with 16 rows, 19.4 with 64;
+/// 2000 x 4096 r64 15.8 and 10.1).
+constexpr int update_rows(int rank_blocks) { return rank_blocks == 1 ? 16 : 64; }
+
+struct UpdateArgs {
+    const uint16_t* g;  // [Mp, 16 kRB] bf16(dy @ b^T), zero past the rank
+    const uint16_t* a;  // [K, rank]
+    uint16_t* grad_x;   // [M, K]
+    int64_t M;
+    int64_t K;
+    int rank;
+    float scale;
+    bool vector_a;      // rows of a are whole aligned 16-byte pieces
+};
+
+/// grad_x += scale * g @ a^T in place, the sum and the product in fp32 and one
+/// rounding. Bound by reading and writing grad_x once: a wave takes 64 columns
+/// (whole 128-byte lines) of 16 or 64 rows, reading their rows of a once, 16
+/// rows at a time with two loads of grad_x per lane (all eight before the first store
+/// ran slower). The two MFMAs of 32 columns
+/// take the rows of a in an order that leaves a lane eight consecutive columns
+/// (16 bytes): row i of the first is column 8 (i / 4) + i % 4, of the second
+/// four further.
+template <int kRB>
+__global__ __launch_bounds__(kThreads) void lora_update_kernel(UpdateArgs args) {
+    constexpr int kRankPad = 16 * kRB;
+    constexpr int kSteps = (kRankPad + 31) / 32;
+    constexpr int kRowBlocks = update_rows(kRB) / 16;
+    const int tid = static_cast<int>(threadIdx.x);
+    const int lane = tid & 63;
+    const int wave = tid >> 6;
+    const int g = lane >> 4;
+    const int jl = lane & 15;
+    const int64_t row0 = static_cast<int64_t>(blockIdx.y) * (16 * kRowBlocks) + jl;
+    const int64_t col0 = static_cast<int64_t>(blockIdx.x) * kUpdateCols + 64 * wave;
+    const int64_t M = args.M;
+    const int64_t K = args.K;
+    auto load_a = [&](int64_t k, int j) {
+        uint4 v = make_uint4(0u, 0u, 0u, 0u);
+        if (k >= K || j >= args.rank) return as_bf16x8(v);
+        const uint16_t* src = args.a + k * args.rank + j;
+        if (args.vector_a) return as_bf16x8(*reinterpret_cast<const uint4*>(src));
+        uint32_t h[8];
+#pragma unroll
+        for (int e = 0; e < 8; ++e) h[e] = j + e < args.rank ? src[e] : 0u;
+        return as_bf16x8(make_uint4(h[0] | (h[1] << 16), h[2] | (h[3] << 16), h[4] | (h[5] << 16),
+                                    h[6] | (h[7] << 16)));
+    };
+    bf16x8_t af[2][2][kSteps];
+#pragma unroll
+    for (int p = 0; p < 2; ++p) {
+        const int64_t k = col0 + 32 * p + 8 * (jl >> 2) + (jl & 3);
+#pragma unroll
+        for (int s = 0; s < kSteps; ++s) {
+            af[p][0][s] = load_a(k, 32 * s + 8 * g);
+            af[p][1][s] = load_a(k + 4, 32 * s + 8 * g);
+        }
+    }
+#pragma unroll 1
+    for (int i = 0; i < kRowBlocks; ++i) {
+        const int64_t row = row0 + 16 * i;
+        uint4 old[2];
+#pragma unroll
+        for (int p = 0; p < 2; ++p) {
+            const int64_t col = col0 + 32 * p + 8 * g;
+            old[p] = make_uint4(0u, 0u, 0u, 0u);
+            if (row < M && col < K) old[p] = *reinterpret_cast<const uint4*>(args.grad_x + row * K + col);
+        }
+        bf16x8_t gf[kSteps];
+#pragma unroll
+        for (int s = 0; s < kSteps; ++s) {
+            const int j = 32 * s + 8 * g;
+            uint4 v = make_uint4(0u, 0u, 0u, 0u);
+            if (row < M && j < kRankPad) v = *reinterpret_cast<const uint4*>(args.g + row * kRankPad + j);
+            gf[s] = as_bf16x8(v);
+        }
+#pragma unroll
+        for (int p = 0; p < 2; ++p) {
+            f32x4_t lo = {0.0f, 0.0f, 0.0f, 0.0f};
+            f32x4_t hi = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+            for (int s = 0; s < kSteps; ++s) {
+                lo = __builtin_amdgcn_mfma_f32_16x16x32_bf16(af[p][0][s], gf[s], lo, 0, 0, 0);
+                hi = __builtin_amdgcn_mfma_f32_16x16x32_bf16(af[p][1][s], gf[s], hi, 0, 0, 0);
+            }
+            const int64_t col = col0 + 32 * p + 8 * g;
+            float v[8];
+            unpack16<bf16_t>(old[p], v);
+#pragma unroll
+            for (int t = 0; t < 4; ++t) {
+                v[t] += args.scale * lo[t];
+                v[4 + t] += args.scale * hi[t];
+            }
+            if (row < M && col < K) store_stream16(args.grad_x + row * K + col, pack16<bf16_t>(v));
+        }
+    }
+}
+
 struct Workspace {
     uint16_t* gt;
+    uint16_t* g;
     float* gpart;
     float* colpart;
 };
@@ -470,6 +577,8 @@ Workspace carve(void* base, int64_t M, int64_t N, int rank_pad) {
     uint8_t* p = static_cast<uint8_t*>(base);
     Workspace ws;
     ws.gt = reinterpret_cast<uint16_t*>(p);
+    p += align256(static_cast<size_t>(rank_pad * Mp) * 2);
+    ws.g = reinterpret_cast<uint16_t*>(p);
     p += align256(static_cast<size_t>(rank_pad * Mp) * 2);
     ws.gpart = reinterpret_cast<float*>(p);
     p += align256(static_cast<size_t>(ceil_div<int64_t>(N, kTileCols) * Mp * rank_pad) * 4);
@@ -509,26 +618,27 @@ size_t lora_backward_fast_workspace_bytes(int64_t M, int64_t K, int64_t N, int64
     const int rank_pad = rank_pad_of(rank);
     const size_t dy = colpart_bytes(M, N, rank_pad);
     const size_t x = colpart_bytes(M, K, rank_pad);
-    return align256(static_cast<size_t>(rank_pad * Mp) * 2) +
+    return 2 * align256(static_cast<size_t>(rank_pad * Mp) * 2) +
            align256(static_cast<size_t>(ceil_div<int64_t>(N, kTileCols) * Mp * rank_pad) * 4) +
            (dy > x ? dy : x);
 }
 
-bool lora_backward_fast_eligible(const void* x, const void* dy, const void* b, int64_t M,
-                                 int64_t K, int64_t N, int64_t rank) {
+bool lora_backward_fast_eligible(const void* x, const void* dy, const void* b, const void* grad_x,
+                                 int64_t M, int64_t K, int64_t N, int64_t rank) {
     // Buffer offsets are 32-bit with an out-of-range marker at 2^31.
     const int64_t Mp = padded_rows(M);
     const bool fits = Mp * K * 2 < (1LL << 31) && Mp * N * 2 < (1LL << 31) &&
                       rank * N * 2 < (1LL << 31) && kMaxRank * Mp * 2 < (1LL << 31) &&
                       Mp * rank * 4 < (1LL << 31);
     return M > 0 && K > 0 && N > 0 && rank > 0 && rank <= kMaxRank && K % 8 == 0 && N % 8 == 0 &&
-           fits && host_aligned(x, 16) && host_aligned(dy, 16) && host_aligned(b, 16);
+           fits && host_aligned(x, 16) && host_aligned(dy, 16) && host_aligned(b, 16) &&
+           host_aligned(grad_x, 16);
 }
 
-cf_status launch_lora_backward_fast(const void* x, const void* dy, const void* b, const float* xa,
-                                    void* grad_a, void* grad_b, int64_t M, int64_t K, int64_t N,
-                                    int64_t rank, float scale, void* workspace,
-                                    hipStream_t stream) {
+cf_status launch_lora_backward_fast(const void* x, const void* dy, const void* a, const void* b,
+                                    const float* xa, void* grad_a, void* grad_b, void* grad_x,
+                                    int64_t M, int64_t K, int64_t N, int64_t rank, float scale,
+                                    void* workspace, hipStream_t stream) {
     const int64_t Mp = padded_rows(M);
     const int rank_pad = rank_pad_of(rank);
     const Workspace ws = carve(workspace, M, N, rank_pad);
@@ -550,7 +660,8 @@ cf_status launch_lora_backward_fast(const void* x, const void* dy, const void* b
     const int64_t g_blocks = ceil_div<int64_t>(rank_pad * Mp, kThreads);
     auto after_dy = [&](auto kernel) {
         launch(kernel, dim3(static_cast<unsigned>(grad_b_blocks + g_blocks)), dim3(kThreads), 0, stream,
-               ws.colpart, static_cast<uint16_t*>(grad_b), ws.gpart, ws.gt, grad_b_blocks,
+               ws.colpart, static_cast<uint16_t*>(grad_b), ws.gpart, ws.gt,
+               grad_x != nullptr ? ws.g : nullptr, grad_b_blocks,
                ceil_div<int64_t>(M, dy_chunks * kChunkRows), rank, N, scale, M, Mp,
                ceil_div<int64_t>(N, kTileCols));
     };
@@ -579,6 +690,26 @@ cf_status launch_lora_backward_fast(const void* x, const void* dy, const void* b
     rank_pad == 16   ? finish_grad_a(finish_grad_a_kernel<16>)
     : rank_pad == 32 ? finish_grad_a(finish_grad_a_kernel<32>)
                      : finish_grad_a(finish_grad_a_kernel<64>);
+    if (grad_x != nullptr) {
+        UpdateArgs update;
+        update.g = ws.g;
+        update.a = static_cast<const uint16_t*>(a);
+        update.grad_x = static_cast<uint16_t*>(grad_x);
+        update.M = M;
+        update.K = K;
+        update.rank = static_cast<int>(rank);
+        update.scale = scale;
+        update.vector_a = rank % 8 == 0 && host_aligned(a, 16);
+        const dim3 grid(static_cast<unsigned>(ceil_div<int64_t>(K, kUpdateCols)),
+                        static_cast<unsigned>(ceil_div<int64_t>(M, update_rows(rank_pad / 16))));
+        if (rank_pad == 16) {
+            launch(lora_update_kernel<1>, grid, dim3(kThreads), 0, stream, update);
+        } else if (rank_pad == 32) {
+            launch(lora_update_kernel<2>, grid, dim3(kThreads), 0, stream, update);
+        } else {
+            launch(lora_update_kernel<4>, grid, dim3(kThreads), 0, stream, update);
+        }
+    }
     return check_launch("launching the bf16 LoRA backward", stream);
 }
 

@@ -15,7 +15,8 @@
 //   * a few extra operators the Python layer uses: dequantize_int8_to (half
 //     outputs), quantize_dequantize, softmax_as (output dtype),
 //     softmax_scaled (scaled, causally masked attention scores), row_sum,
-//     lora_linear_fwd / lora_linear_bwd for the adapter autograd path, and
+//     lora_linear_fwd / lora_linear_bwd / lora_linear_bwd_input for the adapter
+//     autograd path, and
 //     attention_scores_causal / attention_pv_causal, the two causal attention
 //     products of the transformer block.
 #include <c10/hip/HIPStream.h>
@@ -223,11 +224,11 @@ torch::Tensor lora_linear_hip(const torch::Tensor& x, const torch::Tensor& w,
     return std::get<0>(lora_linear_fwd_hip(x, w, a, b, scale));
 }
 
-std::tuple<torch::Tensor, torch::Tensor> lora_linear_bwd_hip(const torch::Tensor& x,
-                                                             const torch::Tensor& dy,
-                                                             const torch::Tensor& b,
-                                                             const torch::Tensor& xa,
-                                                             double scale) {
+// Adapter gradients; with w and a also the input gradient: the plain GEMM
+// dy @ w^T through the vendor BLAS, the adapter's part added in place.
+std::tuple<torch::Tensor, torch::Tensor, torch::Tensor> lora_backward_hip(
+    const torch::Tensor& x, const torch::Tensor& dy, const torch::Tensor* w, const torch::Tensor* a,
+    const torch::Tensor& b, const torch::Tensor& xa, double scale) {
     check_2d(x, "x");
     check_2d(dy, "dy");
     check_2d(b, "b");
@@ -247,17 +248,47 @@ std::tuple<torch::Tensor, torch::Tensor> lora_linear_bwd_hip(const torch::Tensor
     TORCH_CHECK(dy.size(0) == batch && dy.size(1) == out_features, "dy must be [", batch, ", ",
                 out_features, "]");
     TORCH_CHECK(xa.size(0) == batch && xa.size(1) == rank, "xa must be [", batch, ", ", rank, "]");
+    if (w != nullptr) {
+        for (const auto& [tensor, name] : {std::pair<const torch::Tensor*, const char*>{w, "w"}, {a, "a"}}) {
+            check_2d(*tensor, name);
+            check_contiguous(*tensor, name);
+            check_same_device(x, *tensor, name);
+            TORCH_CHECK(tensor->scalar_type() == x.scalar_type(), "x and ", name, " must share a dtype");
+        }
+        TORCH_CHECK(w->size(0) == in_features && w->size(1) == out_features, "w must be [", in_features,
+                    ", ", out_features, "]");
+        TORCH_CHECK(a->size(0) == in_features && a->size(1) == rank, "a must be [", in_features, ", ",
+                    rank, "]");
+    }
     const at::DeviceGuard guard(x.device());
+    torch::Tensor grad_x;
+    if (w != nullptr) grad_x = at::mm(dy, w->t());
     torch::Tensor grad_a = torch::empty({in_features, rank}, x.options());
     torch::Tensor grad_b = torch::empty({rank, out_features}, x.options());
     const size_t bytes = cf_lora_backward_workspace_bytes(batch, in_features, out_features, rank);
     torch::Tensor workspace =
         torch::empty({static_cast<int64_t>(bytes > 0 ? bytes : 1)}, x.options().dtype(torch::kUInt8));
-    check_status(cf_lora_backward(x.data_ptr(), dy.data_ptr(), b.data_ptr(), xa.data_ptr<float>(),
-                                  grad_a.data_ptr(), grad_b.data_ptr(), to_cf(x, "x"), batch,
-                                  in_features, out_features, rank, static_cast<float>(scale),
-                                  workspace.data_ptr(), bytes, stream_for(x)));
+    check_status(cf_lora_backward_input(
+        x.data_ptr(), dy.data_ptr(), a != nullptr ? a->data_ptr() : nullptr, b.data_ptr(),
+        xa.data_ptr<float>(), grad_a.data_ptr(), grad_b.data_ptr(),
+        w != nullptr ? grad_x.data_ptr() : nullptr, to_cf(x, "x"), batch, in_features, out_features, rank,
+        static_cast<float>(scale), workspace.data_ptr(), bytes, stream_for(x)));
+    return {grad_x, grad_a, grad_b};
+}
+
+std::tuple<torch::Tensor, torch::Tensor> lora_linear_bwd_hip(const torch::Tensor& x,
+                                                             const torch::Tensor& dy,
+                                                             const torch::Tensor& b,
+                                                             const torch::Tensor& xa,
+                                                             double scale) {
+    auto [grad_x, grad_a, grad_b] = lora_backward_hip(x, dy, nullptr, nullptr, b, xa, scale);
     return {grad_a, grad_b};
+}
+
+std::tuple<torch::Tensor, torch::Tensor, torch::Tensor> lora_linear_bwd_input_hip(
+    const torch::Tensor& x, const torch::Tensor& dy, const torch::Tensor& w, const torch::Tensor& a,
+    const torch::Tensor& b, const torch::Tensor& xa, double scale) {
+    return lora_backward_hip(x, dy, &w, &a, b, xa, scale);
 }
 
 std::vector<torch::Tensor> fused_residual_rmsnorm_hip(const torch::Tensor& x,
@@ -485,6 +516,15 @@ std::tuple<torch::Tensor, torch::Tensor> lora_linear_bwd_cpu(const torch::Tensor
     return {grad_a, grad_b};
 }
 
+std::tuple<torch::Tensor, torch::Tensor, torch::Tensor> lora_linear_bwd_input_cpu(
+    const torch::Tensor& x, const torch::Tensor& dy, const torch::Tensor& w, const torch::Tensor& a,
+    const torch::Tensor& b, const torch::Tensor& xa, double scale) {
+    const torch::Tensor grad_x =
+        torch::matmul(dy, w.t()) + scale * torch::matmul(torch::matmul(dy, b.t()), a.t());
+    auto [grad_a, grad_b] = lora_linear_bwd_cpu(x, dy, b, xa, scale);
+    return {grad_x, grad_a, grad_b};
+}
+
 torch::Tensor sum_cpu(const torch::Tensor& input) { return input.sum(); }
 
 torch::Tensor row_sum_cpu(const torch::Tensor& input) {
@@ -583,6 +623,9 @@ TORCH_LIBRARY(cudaforge, m) {
     m.def(
         "lora_linear_bwd(Tensor x, Tensor dy, Tensor b, Tensor xa, float scale) "
         "-> (Tensor, Tensor)");
+    m.def(
+        "lora_linear_bwd_input(Tensor x, Tensor dy, Tensor w, Tensor a, Tensor b, Tensor xa, float scale) "
+        "-> (Tensor, Tensor, Tensor)");
     m.def("attention_scores_causal(Tensor q, Tensor k, int heads) -> Tensor");
     m.def("attention_pv_causal(Tensor probs, Tensor v, int heads) -> Tensor");
 }
@@ -595,8 +638,8 @@ TORCH_LIBRARY_IMPL(cudaforge, Autograd, m) {
     for (const char* name :
          {"rmsnorm", "softmax", "lora_linear", "sum", "silu", "gelu", "swiglu", "quantize_int8",
           "dequantize_int8", "dequantize_int8_to", "quantize_dequantize", "softmax_as",
-          "softmax_scaled", "row_sum", "lora_linear_fwd", "lora_linear_bwd", "attention_scores_causal",
-          "attention_pv_causal"}) {
+          "softmax_scaled", "row_sum", "lora_linear_fwd", "lora_linear_bwd", "lora_linear_bwd_input",
+          "attention_scores_causal", "attention_pv_causal"}) {
         m.impl(name, torch::autograd::autogradNotImplementedFallback());
     }
 }
@@ -620,6 +663,7 @@ TORCH_LIBRARY_IMPL(cudaforge, CPU, m) {
     m.impl("row_sum", &row_sum_cpu);
     m.impl("lora_linear_fwd", &lora_linear_fwd_cpu);
     m.impl("lora_linear_bwd", &lora_linear_bwd_cpu);
+    m.impl("lora_linear_bwd_input", &lora_linear_bwd_input_cpu);
     m.impl("attention_scores_causal", &attention_scores_causal_cpu);
     m.impl("attention_pv_causal", &attention_pv_causal_cpu);
 }
@@ -643,6 +687,7 @@ TORCH_LIBRARY_IMPL(cudaforge, CUDA, m) {
     m.impl("row_sum", &row_sum_hip);
     m.impl("lora_linear_fwd", &lora_linear_fwd_hip);
     m.impl("lora_linear_bwd", &lora_linear_bwd_hip);
+    m.impl("lora_linear_bwd_input", &lora_linear_bwd_input_hip);
     m.impl("attention_scores_causal", &attention_scores_causal_hip);
     m.impl("attention_pv_causal", &attention_pv_causal_hip);
 }

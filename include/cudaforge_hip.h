@@ -334,6 +334,19 @@ cf_status cf_lora_backward(const void* x, const void* dy, const void* b, const f
                            int64_t in_features, int64_t out_features, int64_t rank, float scale,
                            void* workspace, size_t workspace_bytes, void* stream);
 
+/* cf_lora_backward, and the adapter's part of the input gradient:
+ *   grad_x [batch, in] += scale * (dy @ b^T) @ a^T
+ * in place, the product and the sum in fp32 with one rounding. `grad_x` holds
+ * dy @ w^T on entry (a plain GEMM of the caller's); NULL leaves that part out
+ * and `a` unread. Workspace as cf_lora_backward's. It has no counterpart in
+ * the reference, whose operator is guarded against differentiation
+ * (cpp/src/bindings.cpp:369-377). */
+cf_status cf_lora_backward_input(const void* x, const void* dy, const void* a, const void* b,
+                                 const float* xa, void* grad_a, void* grad_b, void* grad_x,
+                                 cf_dtype dtype, int64_t batch, int64_t in_features,
+                                 int64_t out_features, int64_t rank, float scale, void* workspace,
+                                 size_t workspace_bytes, void* stream);
+
 /* ---- elementwise activations ------------------------------------------- */
 
 /* silu(x) = x * sigmoid(x), fp32 arithmetic for every dtype.
