@@ -38,8 +38,7 @@ class _LoRALinearFunction(torch.autograd.Function):
         grad_y = grad_y.contiguous()
         grad_x = grad_w = grad_a = grad_b = None
         adapter_grads = ctx.needs_input_grad[2] or ctx.needs_input_grad[3]
-        fused_x = (adapter_grads and ctx.needs_input_grad[0] and not torch.is_grad_enabled()
-                   and x.dtype == torch.bfloat16)
+        fused_x = adapter_grads and ctx.needs_input_grad[0] and not torch.is_grad_enabled()
         if fused_x:
             grad_x, grad_a, grad_b = torch.ops.cudaforge.lora_linear_bwd_input(
                 x, grad_y, weight, lora_a, lora_b, xa, ctx.scale)

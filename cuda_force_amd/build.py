@@ -38,6 +38,7 @@ HIP_SOURCES = (
     "cf_lora_skinny.hip",
     "cf_lora_tile.hip",
     "cf_lora_bwd.hip",
+    "cf_lora_bwd_f32.hip",
     "cf_lora_f32.hip",
     "cf_matmul_f32.hip",
     "cf_scheduler.hip",

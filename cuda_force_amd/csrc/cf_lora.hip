@@ -25,8 +25,9 @@
 //   grad_b = scale * xa^T @ dy   [r, N]   column reduction over M
 //   grad_a = scale * x^T @ G     [K, r]   column reduction over M
 //   grad_x = dy @ w^T (the caller's GEMM) + scale * G @ a^T, in place
-// bf16 with rank <= 64 runs the MFMA kernels of cf_lora_bwd.hip. The generic
-// path here (fp32, other shapes): G one wave per row of dy, the column
+// bf16 with rank <= 64 runs the MFMA kernels of cf_lora_bwd.hip, fp32 those
+// of cf_lora_bwd_f32.hip. The generic
+// path here (other shapes): G one wave per row of dy, the column
 // reductions in row chunks into an fp32 workspace and a second kernel summing
 // the chunks in a fixed order (deterministic).
 #include "cf_common.hpp"
@@ -548,7 +549,9 @@ size_t cf_lora_backward_workspace_bytes(int64_t batch, int64_t in_features, int6
     const size_t generic = ((g + 255) / 256) * 256 + part;
     // Enough for either path: which one runs depends on dtype and alignment.
     const size_t fast = cf::lora_backward_fast_workspace_bytes(batch, in_features, out_features, rank);
-    return generic > fast ? generic : fast;
+    const size_t f32 = cf::lora_backward_f32_workspace_bytes(batch, in_features, out_features, rank);
+    const size_t mfma = fast > f32 ? fast : f32;
+    return generic > mfma ? generic : mfma;
 }
 
 cf_status cf_lora_backward(const void* x, const void* dy, const void* b, const float* xa,
@@ -598,6 +601,16 @@ cf_status cf_lora_backward_input(const void* x, const void* dy, const void* a, c
     float* g = static_cast<float*>(workspace);
     const size_t g_bytes = ((static_cast<size_t>(batch * rank) * sizeof(float) + 255) / 256) * 256;
     float* part = reinterpret_cast<float*>(static_cast<uint8_t*>(workspace) + g_bytes);
+    if (dtype == CF_F32 &&
+        cf::lora_backward_f32_eligible(x, dy, b, batch, in_features, out_features, rank)) {
+        const cf_status st = cf::launch_lora_backward_f32(
+            static_cast<const float*>(x), static_cast<const float*>(dy), static_cast<const float*>(b), xa,
+            static_cast<float*>(grad_a), static_cast<float*>(grad_b), batch, in_features, out_features, rank,
+            scale, workspace, s);
+        if (st != CF_OK || grad_x == nullptr) return st;
+        cf::launch_adapter_update<float>(g, a, grad_x, batch, in_features, rank, scale, s);
+        return cf::check_launch("launching the LoRA input gradient", s);
+    }
     if (dtype == CF_F32) {
         cf::launch_row_dot<float>(dy, b, g, batch, out_features, rank, 1, out_features, s);
         cf_status st = cf::column_reduce<float>(xa, dy, grad_b, false, batch, out_features, rank,

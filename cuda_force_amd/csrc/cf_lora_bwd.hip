@@ -39,8 +39,6 @@
 // Deterministic: every sum has a fixed order, no atomics.
 #include "cf_lora_bwd.hpp"
 
-#include <type_traits>
-
 namespace cf {
 namespace {
 
@@ -354,30 +352,6 @@ __global__ __launch_bounds__(kThreads, kRB == 1 ? 1 : 2) void column_mfma_kernel
             }
         }
     }
-}
-
-/// total += at(t) for t = t .. tiles - 1 in that order, loads issued in
-/// groups of 32, 16, 4, then 1 so a thread waits for memory a few times
-/// rather than once per eight partials.
-template <typename At>
-__device__ __forceinline__ float ordered_sum(int64_t tiles, At at) {
-    float total = 0.0f;
-    int64_t t = 0;
-    auto groups = [&](auto group) {
-        constexpr int kGroup = decltype(group)::value;
-        for (; t + kGroup <= tiles; t += kGroup) {
-            float v[kGroup];
-#pragma unroll
-            for (int k = 0; k < kGroup; ++k) v[k] = at(t + k);
-#pragma unroll
-            for (int k = 0; k < kGroup; ++k) total += v[k];
-        }
-    };
-    groups(std::integral_constant<int, 32>{});
-    groups(std::integral_constant<int, 16>{});
-    groups(std::integral_constant<int, 4>{});
-    groups(std::integral_constant<int, 1>{});
-    return total;
 }
 
 /// gt[j, m] = bf16(sum over column tiles of gpart[tile][m][j]), fixed order,

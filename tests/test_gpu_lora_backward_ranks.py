@@ -33,3 +33,21 @@ def test_backward_ranks_and_row_tiles(shape):
         g.host_values(x, "bf16"), g.host_values(dy, "bf16"), g.host_values(b, "bf16"), xa, 0.5, True)
     assert_gemm_close(ga, exact_a, "bf16", f"grad_a {shape}")
     assert_gemm_close(gb, exact_b, "bf16", f"grad_b {shape}")
+
+
+@pytest.mark.parametrize("shape", [
+    (1, 4, 4, 1), (31, 132, 68, 16), (33, 128, 4096, 17), (128, 4096, 260, 16), (511, 64, 192, 32), (512, 260, 132, 33),
+    (700, 1024, 516, 64), (1025, 68, 64, 8),
+], ids=str)
+def test_fp32_backward_tiles(shape):
+    """The fp32 MFMA backward: both row tiles with remainders, part column
+    tiles, every rank block count."""
+    m, k, n, r = shape
+    g.announce(f"adapter backward fp32 {shape}")
+    gen = rng(sum(shape))
+    x, dy, b, xa = (gen.standard_normal(s).astype(np.float32) for s in ((m, k), (m, n), (r, n), (m, r)))
+    ga, gb = run_backward(x, dy, b, xa, "f32", 0.5)
+    exact_a, exact_b = oracle.lora_backward(x, dy, b, xa, 0.5, False)
+    # fp32 sums of up to 4096 products: 1e-5 of the result's scale.
+    for got, exact in ((ga, exact_a), (gb, exact_b)):
+        assert (np.abs(got - exact) <= 1e-5 * np.abs(exact) + 1e-5 * np.abs(exact).max()).all()
