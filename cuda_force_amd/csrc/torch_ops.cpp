@@ -19,13 +19,18 @@
 //     autograd path, and
 //     attention_scores_causal / attention_pv_causal, the two causal attention
 //     products of the transformer block.
+#include <ATen/PythonTorchFunctionTLS.h>
+#include <ATen/record_function.h>
+#include <c10/core/impl/LocalDispatchKeySet.h>
 #include <c10/hip/HIPStream.h>
 #include <torch/csrc/autograd/autograd_not_implemented_fallback.h>
+#include <torch/csrc/autograd/python_variable.h>
 #include <torch/extension.h>
 
 #include <limits>
 #include <string>
 #include <tuple>
+#include <utility>
 #include <vector>
 
 #include "cudaforge_hip.h"
@@ -182,12 +187,12 @@ std::tuple<torch::Tensor, torch::Tensor> lora_linear_fwd_hip(const torch::Tensor
     check_2d(w, "w");
     check_2d(a, "a");
     check_2d(b, "b");
-    for (const auto& [tensor, name] : std::vector<std::pair<torch::Tensor, const char*>>{
-             {x, "x"}, {w, "w"}, {a, "a"}, {b, "b"}}) {
-        check_contiguous(tensor, name);
-        check_same_device(x, tensor, name);
-        TORCH_CHECK(tensor.scalar_type() == x.scalar_type(), name, " has dtype ",
-                    tensor.scalar_type(), " but x has ", x.scalar_type());
+    for (const auto& [tensor, name] : {std::pair<const torch::Tensor*, const char*>{&x, "x"},
+                                       {&w, "w"}, {&a, "a"}, {&b, "b"}}) {
+        check_contiguous(*tensor, name);
+        check_same_device(x, *tensor, name);
+        TORCH_CHECK(tensor->scalar_type() == x.scalar_type(), name, " has dtype ",
+                    tensor->scalar_type(), " but x has ", x.scalar_type());
     }
     TORCH_CHECK(x.scalar_type() == torch::kFloat32 || x.scalar_type() == torch::kBFloat16,
                 "lora_linear has HIP kernels for float32 and bfloat16, got ", x.scalar_type());
@@ -233,10 +238,10 @@ std::tuple<torch::Tensor, torch::Tensor, torch::Tensor> lora_backward_hip(
     check_2d(dy, "dy");
     check_2d(b, "b");
     check_2d(xa, "xa");
-    for (const auto& [tensor, name] : std::vector<std::pair<torch::Tensor, const char*>>{
-             {x, "x"}, {dy, "dy"}, {b, "b"}, {xa, "xa"}}) {
-        check_contiguous(tensor, name);
-        check_same_device(x, tensor, name);
+    for (const auto& [tensor, name] : {std::pair<const torch::Tensor*, const char*>{&x, "x"},
+                                       {&dy, "dy"}, {&b, "b"}, {&xa, "xa"}}) {
+        check_contiguous(*tensor, name);
+        check_same_device(x, *tensor, name);
     }
     TORCH_CHECK(dy.scalar_type() == x.scalar_type() && b.scalar_type() == x.scalar_type(),
                 "x, dy and b must share a dtype");
@@ -594,6 +599,291 @@ torch::Tensor quantize_dequantize_cpu(const torch::Tensor& input) {
 
 bool cuda_kernels_available() { return true; }
 
+// ---- direct entry for ordinary GPU calls ---------------------------------------
+//
+// A call from Python through torch.ops costs 4-5 us of host time (schema
+// parsing, boxing, the autograd fallback) on top of the checks in ops.py, more
+// than the smallest kernels take. The try_* functions below are what ops.py
+// asks first: when a call is an ordinary one they run the HIP implementation
+// directly, otherwise they return None and ops.py goes its general way
+// (validation messages, copies of non-contiguous inputs, fallbacks, the
+// dispatcher). A call is ordinary when every tensor is a plain dense GPU tensor
+// (exact type, no dispatch key beyond CUDA and its autograd), nothing is
+// tracing, profiling, transforming or overriding it, no gradient is needed,
+// and the arguments are ones the general way would pass to the same HIP
+// implementation unchanged.
+
+bool ordinary_context() {
+    // Dispatch keys switched on for the thread: beyond these two, a mode
+    // (tracing, functorch, Python dispatch) is active; autocast's key is always
+    // on a tensor and excluded for the thread unless autocast is on.
+    static const c10::DispatchKeySet usual({c10::DispatchKey::BackendSelect, c10::DispatchKey::ADInplaceOrView});
+    const c10::impl::LocalDispatchKeySet local = c10::impl::tls_local_dispatch_key_set();
+    return (local.included_.raw_repr() & ~usual.raw_repr()) == 0 &&
+           local.excluded_.has(c10::DispatchKey::AutocastCUDA) && !at::impl::torch_function_mode_enabled() && !at::hasCallbacks();
+}
+
+/// The tensor behind `object`, or null when it is not a plain dense GPU tensor
+/// that is contiguous and not empty.
+const at::Tensor* ordinary(py::handle object) {
+    static const c10::DispatchKeySet usual(
+        {c10::DispatchKey::CUDA, c10::DispatchKey::AutogradCUDA, c10::DispatchKey::AutocastCUDA,
+         c10::DispatchKey::ADInplaceOrView});
+    if (!THPVariable_CheckTypeExact(Py_TYPE(object.ptr()))) return nullptr;
+    const at::Tensor& t = THPVariable_Unpack(object.ptr());
+    if (!t.defined() || !t.key_set().has(c10::DispatchKey::CUDA) || (t.key_set().raw_repr() & ~usual.raw_repr()) != 0) {
+        return nullptr;
+    }
+    return t.is_contiguous() && t.numel() > 0 ? &t : nullptr;
+}
+
+bool kernel_dtype(at::ScalarType t) {
+    return t == torch::kFloat32 || t == torch::kBFloat16 || t == torch::kFloat16;
+}
+
+bool grad_needed(std::initializer_list<const at::Tensor*> tensors) {
+    if (!at::GradMode::is_enabled()) return false;
+    for (const at::Tensor* t : tensors) {
+        if (t->requires_grad()) return true;
+    }
+    return false;
+}
+
+/// Plain, same dtype and device, a dtype with kernels, no gradient needed.
+bool ordinary_set(std::initializer_list<const at::Tensor*> tensors) {
+    const at::Tensor* first = *tensors.begin();
+    for (const at::Tensor* t : tensors) {
+        if (t == nullptr || t->scalar_type() != first->scalar_type() || t->device() != first->device()) return false;
+    }
+    return kernel_dtype(first->scalar_type()) && !grad_needed(tensors);
+}
+
+py::object wrap(const at::Tensor& t) { return py::reinterpret_steal<py::object>(THPVariable_Wrap(t)); }
+
+/// `fn` on x as [rows, last dim], the result in x's shape.
+template <typename Fn>
+py::object by_rows(const at::Tensor& x, Fn fn) {
+    at::Tensor y;
+    {
+        py::gil_scoped_release no_gil;
+        if (x.dim() == 2) {
+            y = fn(x);
+        } else {
+            y = fn(x.view({-1, x.size(-1)})).view(x.sizes());
+        }
+    }
+    return wrap(y);
+}
+
+py::object try_rmsnorm(py::handle x_, py::handle weight_, double eps) {
+    const at::Tensor* x = ordinary(x_);
+    const at::Tensor* w = ordinary(weight_);
+    if (x == nullptr || w == nullptr || !ordinary_context() || !ordinary_set({x, w})) return py::none();
+    if (x->dim() < 1 || w->dim() != 1 || x->size(-1) != w->size(0)) return py::none();
+    return by_rows(*x, [&](const at::Tensor& rows) { return rmsnorm_hip(rows, *w, eps); });
+}
+
+py::object try_fused_residual_rmsnorm(py::handle x_, py::handle residual_, py::handle weight_, double eps) {
+    const at::Tensor* x = ordinary(x_);
+    const at::Tensor* r = ordinary(residual_);
+    const at::Tensor* w = ordinary(weight_);
+    if (x == nullptr || r == nullptr || w == nullptr || !ordinary_context() || !ordinary_set({x, r, w})) {
+        return py::none();
+    }
+    if (x->dim() != 2 || r->sizes() != x->sizes() || w->dim() != 1 || x->size(1) != w->size(0)) return py::none();
+    std::vector<at::Tensor> out;
+    {
+        py::gil_scoped_release no_gil;
+        out = fused_residual_rmsnorm_hip(*x, *r, *w, eps);
+    }
+    return py::make_tuple(wrap(out[0]), wrap(out[1]));
+}
+
+py::object try_softmax(py::handle x_, const std::optional<at::ScalarType>& dtype) {
+    const at::Tensor* x = ordinary(x_);
+    if (x == nullptr || !ordinary_context() || !ordinary_set({x}) || x->dim() < 1) return py::none();
+    const at::ScalarType out = dtype.value_or(x->scalar_type());
+    if (!kernel_dtype(out)) return py::none();
+    return by_rows(*x, [&](const at::Tensor& rows) { return softmax_as_hip(rows, out); });
+}
+
+py::object try_softmax_scaled(py::handle x_, double scale, int64_t causal_period,
+                              const std::optional<at::ScalarType>& dtype) {
+    const at::Tensor* x = ordinary(x_);
+    if (x == nullptr || !ordinary_context() || !ordinary_set({x}) || x->dim() < 1) return py::none();
+    const at::ScalarType out = dtype.value_or(x->scalar_type());
+    if (!kernel_dtype(out) || causal_period < 0) return py::none();
+    return by_rows(*x, [&](const at::Tensor& rows) { return softmax_scaled_hip(rows, scale, causal_period, out); });
+}
+
+template <at::Tensor (*kFn)(const at::Tensor&)>
+py::object try_unary(py::handle x_) {
+    const at::Tensor* x = ordinary(x_);
+    if (x == nullptr || !ordinary_context() || !ordinary_set({x})) return py::none();
+    at::Tensor y;
+    {
+        py::gil_scoped_release no_gil;
+        y = kFn(*x);
+    }
+    return wrap(y);
+}
+
+py::object try_swiglu(py::handle gate_, py::handle up_) {
+    const at::Tensor* gate = ordinary(gate_);
+    const at::Tensor* up = ordinary(up_);
+    if (gate == nullptr || up == nullptr || !ordinary_context() || !ordinary_set({gate, up})) return py::none();
+    if (gate->sizes() != up->sizes()) return py::none();
+    at::Tensor y;
+    {
+        py::gil_scoped_release no_gil;
+        y = swiglu_hip(*gate, *up);
+    }
+    return wrap(y);
+}
+
+py::object try_quantize_int8(py::handle x_) {
+    const at::Tensor* x = ordinary(x_);
+    if (x == nullptr || !ordinary_context() || !ordinary_set({x})) return py::none();
+    std::vector<at::Tensor> out;
+    {
+        py::gil_scoped_release no_gil;
+        out = quantize_int8_hip(*x);
+    }
+    return py::make_tuple(wrap(out[0]), wrap(out[1]));
+}
+
+py::object try_dequantize_int8(py::handle codes_, py::handle scales_, const std::optional<at::ScalarType>& dtype) {
+    const at::Tensor* codes = ordinary(codes_);
+    const at::Tensor* scales = ordinary(scales_);
+    if (codes == nullptr || scales == nullptr || !ordinary_context()) return py::none();
+    const at::ScalarType out = dtype.value_or(torch::kFloat32);
+    if (codes->scalar_type() != torch::kInt8 || scales->scalar_type() != torch::kFloat32 ||
+        codes->device() != scales->device() || !kernel_dtype(out) || grad_needed({scales}) ||
+        scales->numel() != cf_quant_scale_count(codes->numel())) {
+        return py::none();
+    }
+    at::Tensor y;
+    {
+        py::gil_scoped_release no_gil;
+        y = dequantize_int8_to_hip(*codes, *scales, out);
+    }
+    return wrap(y);
+}
+
+/// [batch, seq, hidden] rows of bf16 that the causal attention kernels take.
+bool attention_rows(const at::Tensor& t, int64_t heads) {
+    if (t.scalar_type() != torch::kBFloat16 || t.dim() != 3 || heads <= 0 || t.size(2) % heads != 0) return false;
+    const int64_t d = t.size(2) / heads;
+    return (d == 32 || d == 64 || d == 96 || d == 128) && t.size(1) % 8 == 0;
+}
+
+bool aligned16(const at::Tensor& t) { return reinterpret_cast<uintptr_t>(t.data_ptr()) % 16 == 0; }
+
+py::object try_attention_scores(py::handle q_, py::handle k_, int64_t heads) {
+    const at::Tensor* q = ordinary(q_);
+    const at::Tensor* k = ordinary(k_);
+    if (q == nullptr || k == nullptr || !ordinary_context() || !ordinary_set({q, k})) return py::none();
+    if (!attention_rows(*q, heads) || k->sizes() != q->sizes() || !aligned16(*q) || !aligned16(*k)) return py::none();
+    at::Tensor y;
+    {
+        py::gil_scoped_release no_gil;
+        y = attention_scores_causal_hip(*q, *k, heads);
+    }
+    return wrap(y);
+}
+
+py::object try_attention_pv(py::handle probs_, py::handle v_, int64_t heads) {
+    const at::Tensor* probs = ordinary(probs_);
+    const at::Tensor* v = ordinary(v_);
+    if (probs == nullptr || v == nullptr || !ordinary_context() || !ordinary_set({probs, v})) return py::none();
+    if (!attention_rows(*v, heads) || probs->dim() != 4 || probs->size(0) != v->size(0) ||
+        probs->size(1) != heads || probs->size(2) != v->size(1) || probs->size(3) != v->size(1) ||
+        !aligned16(*probs) || !aligned16(*v)) {
+        return py::none();
+    }
+    at::Tensor y;
+    {
+        py::gil_scoped_release no_gil;
+        y = attention_pv_causal_hip(*probs, *v, heads);
+    }
+    return wrap(y);
+}
+
+// ---- the LoRA linear, with its autograd node ------------------------------------
+
+/// The autograd function of cuda_force_amd/autograd.py as a native node: the
+/// same saved tensors, kernels and composed path under create_graph, without
+/// the interpreter in either direction.
+struct LoraLinear : public torch::autograd::Function<LoraLinear> {
+    static at::Tensor forward(torch::autograd::AutogradContext* ctx, const at::Tensor& x, const at::Tensor& w,
+                              const at::Tensor& a, const at::Tensor& b, double scale) {
+        auto [y, xa] = lora_linear_fwd_hip(x, w, a, b, scale);
+        ctx->save_for_backward({x, w, a, b, xa});
+        ctx->saved_data["scale"] = scale;
+        return y;
+    }
+
+    static torch::autograd::variable_list backward(torch::autograd::AutogradContext* ctx,
+                                                   torch::autograd::variable_list grads) {
+        const auto saved = ctx->get_saved_variables();
+        const at::Tensor &x = saved[0], &w = saved[1], &a = saved[2], &b = saved[3], &xa = saved[4];
+        const double scale = ctx->saved_data["scale"].toDouble();
+        const at::Tensor dy = grads[0].contiguous();
+        at::Tensor grad_x, grad_w, grad_a, grad_b;
+        const bool adapter = ctx->needs_input_grad(2) || ctx->needs_input_grad(3);
+        const bool recorded = at::GradMode::is_enabled();
+        const bool fused_x = adapter && ctx->needs_input_grad(0) && !recorded;
+        if (adapter && recorded) {
+            // Through the dispatcher, whose autograd entry refuses to
+            // differentiate the adapter gradients.
+            static const auto op = c10::Dispatcher::singleton()
+                                       .findSchemaOrThrow("cudaforge::lora_linear_bwd", "")
+                                       .typed<std::tuple<at::Tensor, at::Tensor>(
+                                           const at::Tensor&, const at::Tensor&, const at::Tensor&,
+                                           const at::Tensor&, double)>();
+            std::tie(grad_a, grad_b) = op.call(x, dy, b, xa, scale);
+        } else if (adapter) {
+            std::tie(grad_x, grad_a, grad_b) =
+                lora_backward_hip(x, dy, fused_x ? &w : nullptr, fused_x ? &a : nullptr, b, xa, scale);
+        }
+        if (ctx->needs_input_grad(0) && !fused_x) {
+            grad_x = at::matmul(dy, w.t()) + scale * at::matmul(at::matmul(dy, b.t()), a.t());
+        }
+        if (ctx->needs_input_grad(1)) grad_w = at::matmul(x.t(), dy);
+        return {grad_x, grad_w, grad_a, grad_b, at::Tensor()};
+    }
+};
+
+py::object try_lora_linear(py::handle x_, py::handle w_, py::handle a_, py::handle b_, double scale) {
+    const at::Tensor* x = ordinary(x_);
+    const at::Tensor* w = ordinary(w_);
+    const at::Tensor* a = ordinary(a_);
+    const at::Tensor* b = ordinary(b_);
+    if (x == nullptr || w == nullptr || a == nullptr || b == nullptr || !ordinary_context()) return py::none();
+    const at::ScalarType dtype = x->scalar_type();
+    if (dtype != torch::kFloat32 && dtype != torch::kBFloat16) return py::none();
+    for (const at::Tensor* t : {w, a, b}) {
+        if (t->scalar_type() != dtype || t->device() != x->device() || t->dim() != 2) return py::none();
+    }
+    if (x->dim() < 2 || x->size(-1) != w->size(0) || a->size(0) != w->size(0) || b->size(0) != a->size(1) ||
+        b->size(1) != w->size(1)) {
+        return py::none();
+    }
+    const bool grad = grad_needed({x, w, a, b});
+    at::Tensor y;
+    {
+        py::gil_scoped_release no_gil;
+        const at::Tensor rows = x->dim() == 2 ? *x : x->view({-1, x->size(-1)});
+        y = grad ? LoraLinear::apply(rows, *w, *a, *b, scale) : lora_linear_hip(rows, *w, *a, *b, scale);
+        if (x->dim() != 2) {
+            std::vector<int64_t> shape = x->sizes().vec();
+            shape.back() = w->size(1);
+            y = y.view(shape);
+        }
+    }
+    return wrap(y);
+}
+
 }  // namespace
 }  // namespace cudaforge_amd
 
@@ -696,4 +986,17 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
     m.doc() = "cudaforge operators on MI355X (gfx950) HIP kernels";
     m.def("cuda_kernels_available", &cudaforge_amd::cuda_kernels_available,
           "True when the extension was compiled with its HIP kernels");
+    // Each returns None when the call is not an ordinary GPU one.
+    m.def("try_rmsnorm", &cudaforge_amd::try_rmsnorm);
+    m.def("try_fused_residual_rmsnorm", &cudaforge_amd::try_fused_residual_rmsnorm);
+    m.def("try_softmax", &cudaforge_amd::try_softmax);
+    m.def("try_softmax_scaled", &cudaforge_amd::try_softmax_scaled);
+    m.def("try_silu", &cudaforge_amd::try_unary<&cudaforge_amd::silu_hip>);
+    m.def("try_gelu", &cudaforge_amd::try_unary<&cudaforge_amd::gelu_hip>);
+    m.def("try_swiglu", &cudaforge_amd::try_swiglu);
+    m.def("try_quantize_int8", &cudaforge_amd::try_quantize_int8);
+    m.def("try_dequantize_int8", &cudaforge_amd::try_dequantize_int8);
+    m.def("try_attention_scores", &cudaforge_amd::try_attention_scores);
+    m.def("try_attention_pv", &cudaforge_amd::try_attention_pv);
+    m.def("try_lora_linear", &cudaforge_amd::try_lora_linear);
 }

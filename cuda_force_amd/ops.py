@@ -54,6 +54,14 @@ def _load_extension() -> tuple[bool, bool, str]:
 
 _EXTENSION_LOADED, _CUDA_COMPILED, _LOAD_MESSAGE = _load_extension()
 
+# The extension's direct entry for ordinary GPU calls (torch_ops.cpp): each
+# _DIRECT.try_* returns None for a call it does not take, and the operator goes
+# on below. None without the extension.
+if _EXTENSION_LOADED and _CUDA_COMPILED:
+    from cuda_force_amd import _C as _DIRECT  # type: ignore[attr-defined]
+else:
+    _DIRECT = None
+
 #: True when the HIP kernels are compiled in *and* a GPU is visible.
 CUDA_KERNELS_AVAILABLE: bool = _CUDA_COMPILED and torch.cuda.is_available()
 
@@ -209,6 +217,10 @@ def rmsnorm(x: torch.Tensor, weight: torch.Tensor, eps: float = 1e-6) -> torch.T
     Raises:
         ValueError: if ``weight`` is not 1-D or does not match the last dim.
     """
+    if _DIRECT is not None:
+        direct = _DIRECT.try_rmsnorm(x, weight, eps)
+        if direct is not None:
+            return direct
     if weight.ndim != 1:
         raise ValueError(f"weight must be 1-D, got shape {tuple(weight.shape)}")
     if x.shape[-1] != weight.shape[0]:
@@ -233,6 +245,10 @@ def rmsnorm(x: torch.Tensor, weight: torch.Tensor, eps: float = 1e-6) -> torch.T
 
 def softmax(x: torch.Tensor) -> torch.Tensor:
     """Row softmax over the last dimension (max-subtracted, fp32 arithmetic)."""
+    if _DIRECT is not None:
+        direct = _DIRECT.try_softmax(x, None)
+        if direct is not None:
+            return direct
     if x.numel() == 0:
         return x.clone()
     x = x.contiguous()
@@ -247,6 +263,10 @@ def softmax_as(x: torch.Tensor, dtype: torch.dtype) -> torch.Tensor:
 
     Not in the reference: lets bf16 logits produce fp32 probabilities in one
     pass (torch.softmax(x.float(), -1).to(dtype) otherwise)."""
+    if _DIRECT is not None:
+        direct = _DIRECT.try_softmax(x, dtype)
+        if direct is not None:
+            return direct
     if x.numel() == 0:
         return x.to(dtype).clone()
     x = x.contiguous()
@@ -282,6 +302,10 @@ def softmax_scaled(
     causal`` and ``softmax``, in one pass that does not read the masked
     scores. Result in ``dtype`` (default: the input's); fp32 arithmetic. Not
     in the reference's API."""
+    if _DIRECT is not None and type(causal_period) is int:
+        direct = _DIRECT.try_softmax_scaled(x, float(scale), causal_period, dtype)
+        if direct is not None:
+            return direct
     dtype = x.dtype if dtype is None else dtype
     if causal_period < 0:
         raise ValueError(f"causal_period must be >= 0, got {causal_period}")
@@ -332,6 +356,10 @@ def attention_scores_causal(q: torch.Tensor, k: torch.Tensor, heads: int) -> tor
     follow it with ``softmax_scaled(..., causal_period=seq)``, which never
     reads them. bf16 with head_dim 32/64/96/128 and seq a multiple of 8 runs
     the MFMA kernel on a GPU. Not in the reference's API."""
+    if _DIRECT is not None and type(heads) is int:
+        direct = _DIRECT.try_attention_scores(q, k, heads)
+        if direct is not None:
+            return direct
     _check_attention_rows(q, heads, "q")
     if k.shape != q.shape:
         raise ValueError(f"q and k differ in shape: {tuple(q.shape)} and {tuple(k.shape)}")
@@ -358,6 +386,10 @@ def attention_pv_causal(probs: torch.Tensor, v: torch.Tensor, heads: int) -> tor
     The product of examples/transformer_block.py:63 with its transpose and
     reshape folded in. Same kernel rules as ``attention_scores_causal``. Not
     in the reference's API."""
+    if _DIRECT is not None and type(heads) is int:
+        direct = _DIRECT.try_attention_pv(probs, v, heads)
+        if direct is not None:
+            return direct
     _check_attention_rows(v, heads, "v")
     batch, seq, hidden = v.shape
     if probs.shape != (batch, heads, seq, seq):
@@ -393,6 +425,10 @@ def lora_linear(
     A PEFT-layout layer (W ``[out, in]``, A ``[r, in]``, B ``[out, r]``) maps to
     ``lora_linear(x, W.t().contiguous(), A.t().contiguous(), B.t().contiguous(), alpha / r)``.
     """
+    if _DIRECT is not None:
+        direct = _DIRECT.try_lora_linear(x, weight, lora_a, lora_b, scale)
+        if direct is not None:
+            return direct
     if x.shape[-1] != weight.shape[0]:
         raise ValueError(f"x has {x.shape[-1]} input features but weight expects {weight.shape[0]}")
     if lora_a.shape[0] != weight.shape[0]:
@@ -436,6 +472,10 @@ def fused_residual_rmsnorm(
     ``x`` and ``residual`` differ in shape or ``weight`` does not match their
     last dimension.
     """
+    if _DIRECT is not None:
+        direct = _DIRECT.try_fused_residual_rmsnorm(x, residual, weight, eps)
+        if direct is not None:
+            return direct
     if x.shape != residual.shape:
         raise ValueError(
             f"x and residual must have the same shape, got {tuple(x.shape)} "
@@ -463,6 +503,10 @@ def fused_residual_rmsnorm(
 
 def silu(x: torch.Tensor) -> torch.Tensor:
     """SiLU (swish): ``x * sigmoid(x)``."""
+    if _DIRECT is not None:
+        direct = _DIRECT.try_silu(x)
+        if direct is not None:
+            return direct
     if x.numel() == 0:
         return x.clone()
     x = x.contiguous()
@@ -474,6 +518,10 @@ def silu(x: torch.Tensor) -> torch.Tensor:
 
 def gelu(x: torch.Tensor) -> torch.Tensor:
     """GELU, tanh approximation."""
+    if _DIRECT is not None:
+        direct = _DIRECT.try_gelu(x)
+        if direct is not None:
+            return direct
     if x.numel() == 0:
         return x.clone()
     x = x.contiguous()
@@ -489,6 +537,10 @@ def swiglu(gate: torch.Tensor, up: torch.Tensor) -> torch.Tensor:
     ``gate`` and ``up`` must agree in shape and dtype; otherwise a
     ``ValueError`` is raised before anything runs.
     """
+    if _DIRECT is not None:
+        direct = _DIRECT.try_swiglu(gate, up)
+        if direct is not None:
+            return direct
     if gate.shape != up.shape:
         raise ValueError(
             f"gate and up must have the same shape, got {tuple(gate.shape)} and {tuple(up.shape)}"
@@ -536,6 +588,10 @@ def quantize_int8(x: torch.Tensor) -> tuple[torch.Tensor, torch.Tensor]:
         ``(quantised, scales)``: int8 codes shaped like ``x`` and one fp32
         scale per ``QUANT_BLOCK_SIZE`` elements of the flattened input.
     """
+    if _DIRECT is not None:
+        direct = _DIRECT.try_quantize_int8(x)
+        if direct is not None:
+            return direct
     x = x.contiguous()
     if _dispatch_available("quantize_int8", x) and x.dtype in KERNEL_DTYPES:
         quantised, scales = torch.ops.cudaforge.quantize_int8(x)
@@ -553,6 +609,10 @@ def dequantize_int8(
     the scales' dtype, float32. A half dtype equals the float32 result
     followed by ``.to(dtype)``, computed in one pass.
     """
+    if _DIRECT is not None:
+        direct = _DIRECT.try_dequantize_int8(quantised, scales, dtype)
+        if direct is not None:
+            return direct
     expected = (quantised.numel() + QUANT_BLOCK_SIZE - 1) // QUANT_BLOCK_SIZE
     if scales.numel() != expected:
         raise ValueError(
