@@ -366,6 +366,62 @@ struct TileFor<1024, kResidual> {
     using type = TileShape<1024, 4, 256>;
 };
 
+/// Rows of up to kVecs * kThreads 16-byte vectors, any number of them: one
+/// workgroup per row, the row in registers, thread t taking vectors t, t +
+/// kThreads, ... The row's lanes past its end load its last vector again and
+/// add and store nothing.
+template <typename T, int kVecs, int kThreads, bool kResidual>
+__global__ __launch_bounds__(kThreads) void rmsnorm_row_kernel(
+    const T* __restrict__ x, const T* __restrict__ residual, const T* __restrict__ w,
+    T* __restrict__ y, T* __restrict__ residual_out, int64_t rows, int64_t cols, float eps) {
+    constexpr int kPer = Storage<T>::kPerVec;
+    __shared__ float slot[kThreads / kWaveSize];
+    const int tid = static_cast<int>(threadIdx.x);
+    const int64_t vectors = cols / kPer;
+    const int64_t row = blockIdx.x;
+    uint4 v[kVecs];
+    uint4 b[kResidual ? kVecs : 1];
+    uint4 g[kVecs];
+#pragma unroll
+    for (int j = 0; j < kVecs; ++j) {
+        const int64_t idx = static_cast<int64_t>(j) * kThreads + tid;
+        const int64_t at = (idx < vectors ? idx : vectors - 1) * kPer;
+        v[j] = load_stream16(x + row * cols + at);
+        if constexpr (kResidual) b[j] = load_stream16(residual + row * cols + at);
+        g[j] = *reinterpret_cast<const uint4*>(w + at);
+    }
+    bool finite = true;
+    float partial = 0.0f;
+#pragma unroll
+    for (int j = 0; j < kVecs; ++j) {
+        const int64_t idx = static_cast<int64_t>(j) * kThreads + tid;
+        if constexpr (kResidual) {
+            float sum[kPer];
+            float other[kPer];
+            unpack16<T>(v[j], sum);
+            unpack16<T>(b[j], other);
+#pragma unroll
+            for (int i = 0; i < kPer; ++i) sum[i] = sum[i] + other[i];
+            // Rounded to the storage type before the norm, as `x + residual`
+            // is in the reference.
+            v[j] = pack16<T>(sum);
+            if (idx < vectors) store_stream16(residual_out + row * cols + idx * kPer, v[j]);
+        }
+        finite = finite && finite16<T>(g[j]);
+        if (idx < vectors) partial += sum_squares16<T>(v[j]);
+    }
+    const float total = block_reduce_f32<kThreads / kWaveSize, AddF32>(partial, slot);
+    const float scale = inv_rms(total, cols, eps);
+    finite = finite && __builtin_isfinite(total);
+#pragma unroll
+    for (int j = 0; j < kVecs; ++j) {
+        const int64_t idx = static_cast<int64_t>(j) * kThreads + tid;
+        if (idx < vectors) {
+            store_stream16(y + row * cols + idx * kPer, scale16<T>(v[j], g[j], scale, finite));
+        }
+    }
+}
+
 /// Any shape and alignment: one workgroup per row, two passes over the row.
 template <typename T, bool kResidual>
 __global__ __launch_bounds__(kDefaultBlockSize) void rmsnorm_block_kernel(
@@ -422,6 +478,14 @@ void launch_wave(const void* x, const void* residual, const void* w, void* y, vo
     }
 }
 
+template <typename T, int kVecs, int kThreads, bool kResidual>
+void launch_row(const void* x, const void* residual, const void* w, void* y, void* residual_out,
+                int64_t rows, int64_t cols, float eps, hipStream_t stream) {
+    launch(rmsnorm_row_kernel<T, kVecs, kThreads, kResidual>, dim3(static_cast<unsigned>(rows)),
+           dim3(kThreads), 0, stream, static_cast<const T*>(x), static_cast<const T*>(residual),
+           static_cast<const T*>(w), static_cast<T*>(y), static_cast<T*>(residual_out), rows, cols, eps);
+}
+
 template <typename T, bool kResidual>
 cf_status dispatch(const void* x, const void* residual, const void* w, void* y,
                    void* residual_out, int64_t rows, int64_t cols, float eps,
@@ -460,17 +524,32 @@ cf_status dispatch(const void* x, const void* residual, const void* w, void* y,
         } else {
             run(Tile1024{});
         }
-    } else if (vec && vectors_per_lane <= 16) {
+    } else if (vec && rows < (1LL << 31) && row_vectors <= 8192 &&
+               (vectors_per_lane > 8 || (rows <= cu_count() && vectors_per_lane > 4))) {
+        // A workgroup per row where a wave would hold more than eight vectors
+        // per lane (fused residual [8192, 5120] bf16 68.3 -> 56.5 us, [800,
+        // 6712] fp16 19.6 -> 11.3, [8000, 2560] fp32 62.9 -> 54.1), and for
+        // few rows of more than four ([4, 4096] bf16 4.06 -> 3.79). With up to
+        // eight the wave kernel is the faster one ([4096, 4096] bf16 12.0
+        // against 13.8 us, [2048, 4096] fp32 11.0 against 13.3).
+        if (row_vectors <= 512) {
+            launch_row<T, 1, 512, kResidual>(x, residual, w, y, residual_out, rows, cols, eps, stream);
+        } else if (row_vectors <= 1024) {
+            launch_row<T, 2, 512, kResidual>(x, residual, w, y, residual_out, rows, cols, eps, stream);
+        } else if (row_vectors <= 2048) {
+            launch_row<T, 2, 1024, kResidual>(x, residual, w, y, residual_out, rows, cols, eps, stream);
+        } else {
+            launch_row<T, 8, 1024, kResidual>(x, residual, w, y, residual_out, rows, cols, eps, stream);
+        }
+    } else if (vec && vectors_per_lane <= 8) {
         if (vectors_per_lane <= 1) {
             launch_wave<T, 1, kResidual>(x, residual, w, y, residual_out, rows, cols, eps, stream);
         } else if (vectors_per_lane <= 2) {
             launch_wave<T, 2, kResidual>(x, residual, w, y, residual_out, rows, cols, eps, stream);
         } else if (vectors_per_lane <= 4) {
             launch_wave<T, 4, kResidual>(x, residual, w, y, residual_out, rows, cols, eps, stream);
-        } else if (vectors_per_lane <= 8) {
-            launch_wave<T, 8, kResidual>(x, residual, w, y, residual_out, rows, cols, eps, stream);
         } else {
-            launch_wave<T, 16, kResidual>(x, residual, w, y, residual_out, rows, cols, eps, stream);
+            launch_wave<T, 8, kResidual>(x, residual, w, y, residual_out, rows, cols, eps, stream);
         }
     } else {
         const int64_t max_blocks = static_cast<int64_t>(cu_count()) * 8;
