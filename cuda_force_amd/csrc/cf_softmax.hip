@@ -19,12 +19,17 @@
 // a wave reads its whole row before it writes any of it.
 //
 // Rows too long for one wave's registers (more than 1024 16-byte vectors: fp32
-// rows past 4096 columns, 16-bit rows past 8192) take a workgroup of 1024
-// threads per row, the row again in registers (up to 8 vectors per thread),
-// with the two reductions across the workgroup through LDS.
+// rows past 4096 columns, 16-bit rows past 8192) take a workgroup per row, the
+// row again in registers (up to 8 vectors per thread), with the two reductions
+// across the workgroup through LDS: 512 threads up to 4096 vectors, so that
+// two or three workgroups share a CU (257 rows of 32000 bf16 to fp32: 16.0 ->
+// 13.9 us, with 1024 threads the last row had a round to itself), 1024 above.
+// Unaligned pointers and ragged widths up to 65536 columns do the same an
+// element at a time ([300, 50257] fp32 194 -> 38 us, [1024, 32001] bf16 to
+// fp32 142 -> 51).
 //
-// Fallback: longer rows, unaligned pointers or ragged widths use a workgroup
-// per row with three passes over the row (max, sum, normalise).
+// Fallback: longer rows use a workgroup per row with three passes over the row
+// (max, sum, normalise).
 //
 // cf_softmax_scaled is the same kernel on scale * x with an optional causal
 // mask (column c of row r hidden when c > r mod period): the attention-score
@@ -43,14 +48,25 @@ namespace {
 constexpr int kWavesPerBlock = kDefaultBlockSize / kWaveSize;
 
 /// Store `n` (4 or 8) floats as Tout at `p` with 16- or 8-byte streaming stores.
-template <typename Tout, int kN>
+/// kMerge: eight fp32 values, 32 bytes of a lane, go out as plain stores. Each
+/// of the two instructions writes every other 16 bytes, so the lines are only
+/// whole once the L2 has merged the two; streaming stores sent the halves on
+/// ([1024, 32000] bf16 -> fp32 55.3 us, merged 36.9). With one vector per
+/// thread streaming is the faster one ([600, 8000] fp16 -> fp32 8.6 against
+/// 9.5).
+template <typename Tout, int kN, bool kMerge = false>
 __device__ __forceinline__ void store_vec(Tout* p, const float* v) {
     constexpr int kOutPer = Storage<Tout>::kPerVec;
     if constexpr (kN == kOutPer) {
         store_stream16(p, pack16<Tout>(v));
     } else if constexpr (kN == 2 * kOutPer) {
-        store_stream16(p, pack16<Tout>(v));
-        store_stream16(p + kOutPer, pack16<Tout>(v + kOutPer));
+        if constexpr (kMerge) {
+            *reinterpret_cast<uint4*>(p) = pack16<Tout>(v);
+            *reinterpret_cast<uint4*>(p + kOutPer) = pack16<Tout>(v + kOutPer);
+        } else {
+            store_stream16(p, pack16<Tout>(v));
+            store_stream16(p + kOutPer, pack16<Tout>(v + kOutPer));
+        }
     } else {
         // 4 values into a 16-bit type: one 8-byte store.
         static_assert(kN == 4 && kOutPer == 8, "unsupported store width");
@@ -100,7 +116,7 @@ __device__ __forceinline__ uint4 buffer_load_stream16(__amdgpu_buffer_rsrc_t rsr
 /// value is NaN. So for bf16 a row whose 1 / sum is finite is rounded by
 /// v_cvt_pk_bf16_f32 alone, and a NaN row stores the canonical 0x7FC0: the
 /// bits of f32_to_bf16_bits either way, with no per-value NaN test.
-template <typename Tout, int kN>
+template <typename Tout, int kN, bool kMerge = false>
 __device__ __forceinline__ void store_probs(Tout* p, const float* v, bool row_nan) {
     if constexpr (std::is_same_v<Tout, bf16_t> && (kN == 8 || kN == 4)) {
         uint32_t w[kN / 2];
@@ -114,7 +130,7 @@ __device__ __forceinline__ void store_probs(Tout* p, const float* v, bool row_na
             store_stream8(p, make_uint2(w[0], w[1]));
         }
     } else {
-        store_vec<Tout, kN>(p, v);
+        store_vec<Tout, kN, kMerge>(p, v);
     }
 }
 
@@ -292,7 +308,7 @@ __global__ __launch_bounds__(kThreads) void softmax_row_kernel(const Tin* x, Tou
             if (kFullCols || idx < vec_cols) {
 #pragma unroll
                 for (int i = 0; i < kPer; ++i) v[j][i] = v[j][i] * inv_sum;
-                store_probs<Tout, kPer>(y + row * cols + idx * kPer, v[j], row_nan);
+                store_probs<Tout, kPer, (kVecs >= 4)>(y + row * cols + idx * kPer, v[j], row_nan);
             }
         }
     }
@@ -310,6 +326,91 @@ void launch_row(const void* x, void* y, int64_t rows, int64_t cols, const Maskin
     } else {
         launch(softmax_row_kernel<Tin, Tout, kVecs, false, kMasked, kThreads>, dim3(grid), dim3(kThreads), 0, stream,
                xin, out, rows, cols, mask);
+    }
+}
+
+/// Ragged rows (a width that is not whole 16-byte vectors, or unaligned
+/// pointers) of up to kElems * kThreads columns: one workgroup per row, the
+/// row in registers an element per lane at a time, thread t taking columns
+/// t, t + kThreads, ... Still one read and one write, where the kernel below
+/// reads the row three times, each pass a chain of dependent trips to memory.
+/// The row is a buffer resource: a lane's columns differ by a scalar offset
+/// (64 addresses per lane would spill), and columns past the row's end read
+/// as zero and are not written. Groups of eight steps past the end are
+/// skipped. Every thread has read its columns before the first reduction's
+/// barrier, so x and y may alias.
+template <typename Tin, typename Tout, int kElems, bool kMasked, int kThreads>
+__global__ __launch_bounds__(kThreads) void softmax_ragged_kernel(const Tin* x, Tout* y, int64_t rows,
+                                                                  int64_t cols, Masking mask) {
+    constexpr int kGroup = 8;
+    constexpr int kIn = static_cast<int>(sizeof(Tin));
+    constexpr int kOut = static_cast<int>(sizeof(Tout));
+    __shared__ float slot[kThreads / kWaveSize];
+    const int tid = static_cast<int>(threadIdx.x);
+    const int width = static_cast<int>(cols);
+    const float neg_inf = -__builtin_inff();
+    for (int64_t row = blockIdx.x; row < rows; row += gridDim.x) {
+        const int64_t seen = last_visible(mask, row, cols);
+        const int end = kMasked && seen < cols ? static_cast<int>(seen) + 1 : width;  // then -inf, not read
+        const __amdgpu_buffer_rsrc_t in = make_buffer(x + row * cols, static_cast<uint32_t>(end * kIn));
+        const __amdgpu_buffer_rsrc_t out = make_buffer(y + row * cols, static_cast<uint32_t>(width * kOut));
+        float v[kElems];
+#pragma unroll
+        for (int j0 = 0; j0 < kElems; j0 += kGroup) {
+            if (j0 * kThreads < width) {
+#pragma unroll
+                for (int j = j0; j < j0 + kGroup; ++j) {
+                    if constexpr (kIn == 4) {
+                        v[j] = __uint_as_float(
+                            __builtin_amdgcn_raw_buffer_load_b32(in, tid * kIn, j * kThreads * kIn, 0));
+                    } else {
+                        v[j] = Storage<Tin>::from_bits(
+                            __builtin_amdgcn_raw_buffer_load_b16(in, tid * kIn, j * kThreads * kIn, 0));
+                    }
+                }
+            }
+        }
+        float local_max = neg_inf;
+#pragma unroll
+        for (int j0 = 0; j0 < kElems; j0 += kGroup) {
+            if (j0 * kThreads < width) {
+#pragma unroll
+                for (int j = j0; j < j0 + kGroup; ++j) {
+                    v[j] = j * kThreads + tid < end ? (kMasked ? mask.scale * v[j] : v[j]) : neg_inf;
+                    local_max = fmaxf(local_max, v[j]);
+                }
+            }
+        }
+        const float row_max = block_reduce_f32<kThreads / kWaveSize, MaxF32>(local_max, slot);
+        float partial[2] = {0.0f, 0.0f};
+#pragma unroll
+        for (int j0 = 0; j0 < kElems; j0 += kGroup) {
+            if (j0 * kThreads < width) {
+#pragma unroll
+                for (int j = j0; j < j0 + kGroup; ++j) {
+                    v[j] = __expf(v[j] - row_max);
+                    partial[j & 1] += j * kThreads + tid < width ? v[j] : 0.0f;
+                }
+            }
+        }
+        const float inv_sum =
+            1.0f / block_reduce_f32<kThreads / kWaveSize, AddF32>(partial[0] + partial[1], slot);
+#pragma unroll
+        for (int j0 = 0; j0 < kElems; j0 += kGroup) {
+            if (j0 * kThreads < width) {
+#pragma unroll
+                for (int j = j0; j < j0 + kGroup; ++j) {
+                    const float p = v[j] * inv_sum;
+                    if constexpr (kOut == 4) {
+                        __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(p), out, tid * kOut,
+                                                              j * kThreads * kOut, 0);
+                    } else {
+                        __builtin_amdgcn_raw_buffer_store_b16(static_cast<uint16_t>(Storage<Tout>::to_bits(p)),
+                                                              out, tid * kOut, j * kThreads * kOut, 0);
+                    }
+                }
+            }
+        }
     }
 }
 
@@ -422,12 +523,26 @@ cf_status dispatch(const void* x, void* y, int64_t rows, int64_t cols, const Mas
         }
     } else if (vec && vectors_per_lane <= 8 * kRowThreads / kWaveSize) {
         const int64_t per_thread = ceil_div<int64_t>(cols / kPer, kRowThreads);
-        if (per_thread <= 2) {
-            launch_row<Tin, Tout, 2, kMasked>(x, y, rows, cols, mask, stream);
+        if (per_thread <= 2) {  // twice that of 512 threads
+            launch_row<Tin, Tout, 4, kMasked, 512>(x, y, rows, cols, mask, stream);
         } else if (per_thread <= 4) {
-            launch_row<Tin, Tout, 4, kMasked>(x, y, rows, cols, mask, stream);
+            launch_row<Tin, Tout, 8, kMasked, 512>(x, y, rows, cols, mask, stream);
         } else {
             launch_row<Tin, Tout, 8, kMasked>(x, y, rows, cols, mask, stream);
+        }
+    } else if (cols <= 64 * kRowThreads) {
+        const dim3 grid(static_cast<unsigned>(rows < (1 << 20) ? rows : (1 << 20)));
+        const auto* xin = static_cast<const Tin*>(x);
+        auto* out = static_cast<Tout*>(y);
+        if (cols <= 16 * 256) {
+            launch(softmax_ragged_kernel<Tin, Tout, 16, kMasked, 256>, grid, dim3(256), 0, stream, xin, out, rows,
+                   cols, mask);
+        } else if (cols <= 32 * kRowThreads) {
+            launch(softmax_ragged_kernel<Tin, Tout, 32, kMasked, kRowThreads>, grid, dim3(kRowThreads), 0, stream,
+                   xin, out, rows, cols, mask);
+        } else {
+            launch(softmax_ragged_kernel<Tin, Tout, 64, kMasked, kRowThreads>, grid, dim3(kRowThreads), 0, stream,
+                   xin, out, rows, cols, mask);
         }
     } else {
         const int64_t max_blocks = static_cast<int64_t>(cu_count()) * 8;
