@@ -2,7 +2,8 @@
 float64 oracle: each tile shape with part tiles in both directions, K not a
 multiple of the K-step, one K-step and fewer than the stages, ranks whose
 rows are 16-byte pieces, pairs and single elements, adapter parts that fill
-K-steps exactly and that do not, whole tiles, split tiles and both. The
+K-steps exactly and that do not (or lie in several slices), slices of x @ a
+down to empty ones, whole tiles, split tiles and both. The
 tolerance is that of the other bf16 LoRA tests (one bf16 rounding 2^-9
 relative, a floor for cancelling sums)."""
 
@@ -23,7 +24,7 @@ pytestmark = pytest.mark.gpu
 @pytest.mark.parametrize("shape", [
     (65, 8, 8, 1), (65, 32, 128, 32), (100, 4096, 4096, 16), (128, 1024, 1024, 32), (129, 688, 264, 6),
     (300, 1000, 520, 7), (333, 4096, 11008, 16), (513, 264, 4096, 100), (700, 72, 136, 128), (1000, 2048, 4096, 64),
-    (2100, 136, 4104, 24), (5000, 1000, 1032, 64),
+    (2100, 136, 4104, 24), (5000, 1000, 1032, 64), (90, 16, 4096, 128), (66, 544, 2048, 48),
 ], ids=str)
 @pytest.mark.parametrize("scale", [2.0, 16 / 12])
 def test_tiles_match_the_oracle(shape, scale):
