@@ -2,10 +2,9 @@
 float64 oracle: each tile shape with part tiles in both directions, K not a
 multiple of the K-step, one K-step and fewer than the stages, ranks whose
 rows are 16-byte pieces, pairs and single elements, adapter parts that fill
-K-steps exactly and that do not (or lie in several slices), slices of x @ a
-down to empty ones, whole tiles, split tiles and both. The
-tolerance is that of the other bf16 LoRA tests (one bf16 rounding 2^-9
-relative, a floor for cancelling sums)."""
+K-steps exactly and that do not (or lie in several slices), whole tiles, split
+tiles and both. The tolerance is that of the other bf16 LoRA tests (one bf16
+rounding 2^-9 relative, a floor for cancelling sums)."""
 
 from __future__ import annotations
 
