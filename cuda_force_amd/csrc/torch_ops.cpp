@@ -23,6 +23,8 @@
 #include <ATen/record_function.h>
 #include <c10/core/impl/LocalDispatchKeySet.h>
 #include <c10/hip/HIPStream.h>
+#include <torch/csrc/Dtype.h>
+#include <torch/csrc/Exceptions.h>
 #include <torch/csrc/autograd/autograd_not_implemented_fallback.h>
 #include <torch/csrc/autograd/python_variable.h>
 #include <torch/extension.h>
@@ -624,7 +626,7 @@ bool ordinary_context() {
 }
 
 /// The tensor behind `object`, or null when it is not a plain dense GPU tensor
-/// that is contiguous and not empty.
+/// that is contiguous, not empty and without a forward-mode tangent.
 const at::Tensor* ordinary(py::handle object) {
     static const c10::DispatchKeySet usual(
         {c10::DispatchKey::CUDA, c10::DispatchKey::AutogradCUDA, c10::DispatchKey::AutocastCUDA,
@@ -634,7 +636,38 @@ const at::Tensor* ordinary(py::handle object) {
     if (!t.defined() || !t.key_set().has(c10::DispatchKey::CUDA) || (t.key_set().raw_repr() & ~usual.raw_repr()) != 0) {
         return nullptr;
     }
-    return t.is_contiguous() && t.numel() > 0 ? &t : nullptr;
+    return t.is_contiguous() && t.numel() > 0 && !t._fw_grad(0).defined() ? &t : nullptr;
+}
+
+// The other arguments come as Python objects: a value that is not plainly a
+// number or a dtype (a tensor, a NumPy type, a bool, an int out of range) is
+// left to the general way, whose conversions and errors stand.
+
+std::optional<double> plain_double(py::handle object) {
+    if (PyFloat_Check(object.ptr())) return PyFloat_AS_DOUBLE(object.ptr());
+    if (!PyLong_CheckExact(object.ptr())) return std::nullopt;
+    const double value = PyLong_AsDouble(object.ptr());
+    if (value == -1.0 && PyErr_Occurred() != nullptr) {
+        PyErr_Clear();
+        return std::nullopt;
+    }
+    return value;
+}
+
+std::optional<int64_t> plain_int(py::handle object) {
+    if (!PyLong_CheckExact(object.ptr())) return std::nullopt;
+    int overflow = 0;
+    const long long value = PyLong_AsLongLongAndOverflow(object.ptr(), &overflow);
+    return overflow == 0 ? std::optional<int64_t>(value) : std::nullopt;
+}
+
+/// The dtype given, `otherwise` for None, nothing for any other object or a
+/// dtype without kernels.
+std::optional<at::ScalarType> plain_dtype(py::handle object, at::ScalarType otherwise) {
+    if (!object.is_none() && !THPDtype_Check(object.ptr())) return std::nullopt;
+    const at::ScalarType t = object.is_none() ? otherwise : reinterpret_cast<THPDtype*>(object.ptr())->scalar_type;
+    return t == torch::kFloat32 || t == torch::kBFloat16 || t == torch::kFloat16 ? std::optional<at::ScalarType>(t)
+                                                                                 : std::nullopt;
 }
 
 bool kernel_dtype(at::ScalarType t) {
@@ -675,45 +708,48 @@ py::object by_rows(const at::Tensor& x, Fn fn) {
     return wrap(y);
 }
 
-py::object try_rmsnorm(py::handle x_, py::handle weight_, double eps) {
+py::object try_rmsnorm(py::handle x_, py::handle weight_, py::handle eps_) {
     const at::Tensor* x = ordinary(x_);
     const at::Tensor* w = ordinary(weight_);
-    if (x == nullptr || w == nullptr || !ordinary_context() || !ordinary_set({x, w})) return py::none();
+    const std::optional<double> eps = plain_double(eps_);
+    if (x == nullptr || w == nullptr || !eps || !ordinary_context() || !ordinary_set({x, w})) return py::none();
     if (x->dim() < 1 || w->dim() != 1 || x->size(-1) != w->size(0)) return py::none();
-    return by_rows(*x, [&](const at::Tensor& rows) { return rmsnorm_hip(rows, *w, eps); });
+    return by_rows(*x, [&](const at::Tensor& rows) { return rmsnorm_hip(rows, *w, *eps); });
 }
 
-py::object try_fused_residual_rmsnorm(py::handle x_, py::handle residual_, py::handle weight_, double eps) {
+py::object try_fused_residual_rmsnorm(py::handle x_, py::handle residual_, py::handle weight_, py::handle eps_) {
     const at::Tensor* x = ordinary(x_);
     const at::Tensor* r = ordinary(residual_);
     const at::Tensor* w = ordinary(weight_);
-    if (x == nullptr || r == nullptr || w == nullptr || !ordinary_context() || !ordinary_set({x, r, w})) {
+    const std::optional<double> eps = plain_double(eps_);
+    if (x == nullptr || r == nullptr || w == nullptr || !eps || !ordinary_context() || !ordinary_set({x, r, w})) {
         return py::none();
     }
     if (x->dim() != 2 || r->sizes() != x->sizes() || w->dim() != 1 || x->size(1) != w->size(0)) return py::none();
     std::vector<at::Tensor> out;
     {
         py::gil_scoped_release no_gil;
-        out = fused_residual_rmsnorm_hip(*x, *r, *w, eps);
+        out = fused_residual_rmsnorm_hip(*x, *r, *w, *eps);
     }
     return py::make_tuple(wrap(out[0]), wrap(out[1]));
 }
 
-py::object try_softmax(py::handle x_, const std::optional<at::ScalarType>& dtype) {
+py::object try_softmax(py::handle x_, py::handle dtype_) {
     const at::Tensor* x = ordinary(x_);
     if (x == nullptr || !ordinary_context() || !ordinary_set({x}) || x->dim() < 1) return py::none();
-    const at::ScalarType out = dtype.value_or(x->scalar_type());
-    if (!kernel_dtype(out)) return py::none();
-    return by_rows(*x, [&](const at::Tensor& rows) { return softmax_as_hip(rows, out); });
+    const std::optional<at::ScalarType> out = plain_dtype(dtype_, x->scalar_type());
+    if (!out) return py::none();
+    return by_rows(*x, [&](const at::Tensor& rows) { return softmax_as_hip(rows, *out); });
 }
 
-py::object try_softmax_scaled(py::handle x_, double scale, int64_t causal_period,
-                              const std::optional<at::ScalarType>& dtype) {
+py::object try_softmax_scaled(py::handle x_, py::handle scale_, py::handle causal_period_, py::handle dtype_) {
     const at::Tensor* x = ordinary(x_);
     if (x == nullptr || !ordinary_context() || !ordinary_set({x}) || x->dim() < 1) return py::none();
-    const at::ScalarType out = dtype.value_or(x->scalar_type());
-    if (!kernel_dtype(out) || causal_period < 0) return py::none();
-    return by_rows(*x, [&](const at::Tensor& rows) { return softmax_scaled_hip(rows, scale, causal_period, out); });
+    const std::optional<double> scale = plain_double(scale_);
+    const std::optional<int64_t> period = plain_int(causal_period_);
+    const std::optional<at::ScalarType> out = plain_dtype(dtype_, x->scalar_type());
+    if (!scale || !period || !out || *period < 0) return py::none();
+    return by_rows(*x, [&](const at::Tensor& rows) { return softmax_scaled_hip(rows, *scale, *period, *out); });
 }
 
 template <at::Tensor (*kFn)(const at::Tensor&)>
@@ -752,20 +788,20 @@ py::object try_quantize_int8(py::handle x_) {
     return py::make_tuple(wrap(out[0]), wrap(out[1]));
 }
 
-py::object try_dequantize_int8(py::handle codes_, py::handle scales_, const std::optional<at::ScalarType>& dtype) {
+py::object try_dequantize_int8(py::handle codes_, py::handle scales_, py::handle dtype_) {
     const at::Tensor* codes = ordinary(codes_);
     const at::Tensor* scales = ordinary(scales_);
     if (codes == nullptr || scales == nullptr || !ordinary_context()) return py::none();
-    const at::ScalarType out = dtype.value_or(torch::kFloat32);
+    const std::optional<at::ScalarType> out = plain_dtype(dtype_, torch::kFloat32);
     if (codes->scalar_type() != torch::kInt8 || scales->scalar_type() != torch::kFloat32 ||
-        codes->device() != scales->device() || !kernel_dtype(out) || grad_needed({scales}) ||
+        codes->device() != scales->device() || !out || grad_needed({scales}) ||
         scales->numel() != cf_quant_scale_count(codes->numel())) {
         return py::none();
     }
     at::Tensor y;
     {
         py::gil_scoped_release no_gil;
-        y = dequantize_int8_to_hip(*codes, *scales, out);
+        y = dequantize_int8_to_hip(*codes, *scales, *out);
     }
     return wrap(y);
 }
@@ -779,32 +815,34 @@ bool attention_rows(const at::Tensor& t, int64_t heads) {
 
 bool aligned16(const at::Tensor& t) { return reinterpret_cast<uintptr_t>(t.data_ptr()) % 16 == 0; }
 
-py::object try_attention_scores(py::handle q_, py::handle k_, int64_t heads) {
+py::object try_attention_scores(py::handle q_, py::handle k_, py::handle heads_) {
     const at::Tensor* q = ordinary(q_);
     const at::Tensor* k = ordinary(k_);
-    if (q == nullptr || k == nullptr || !ordinary_context() || !ordinary_set({q, k})) return py::none();
-    if (!attention_rows(*q, heads) || k->sizes() != q->sizes() || !aligned16(*q) || !aligned16(*k)) return py::none();
+    const std::optional<int64_t> heads = plain_int(heads_);
+    if (q == nullptr || k == nullptr || !heads || !ordinary_context() || !ordinary_set({q, k})) return py::none();
+    if (!attention_rows(*q, *heads) || k->sizes() != q->sizes() || !aligned16(*q) || !aligned16(*k)) return py::none();
     at::Tensor y;
     {
         py::gil_scoped_release no_gil;
-        y = attention_scores_causal_hip(*q, *k, heads);
+        y = attention_scores_causal_hip(*q, *k, *heads);
     }
     return wrap(y);
 }
 
-py::object try_attention_pv(py::handle probs_, py::handle v_, int64_t heads) {
+py::object try_attention_pv(py::handle probs_, py::handle v_, py::handle heads_) {
     const at::Tensor* probs = ordinary(probs_);
     const at::Tensor* v = ordinary(v_);
-    if (probs == nullptr || v == nullptr || !ordinary_context() || !ordinary_set({probs, v})) return py::none();
-    if (!attention_rows(*v, heads) || probs->dim() != 4 || probs->size(0) != v->size(0) ||
-        probs->size(1) != heads || probs->size(2) != v->size(1) || probs->size(3) != v->size(1) ||
+    const std::optional<int64_t> heads = plain_int(heads_);
+    if (probs == nullptr || v == nullptr || !heads || !ordinary_context() || !ordinary_set({probs, v})) return py::none();
+    if (!attention_rows(*v, *heads) || probs->dim() != 4 || probs->size(0) != v->size(0) ||
+        probs->size(1) != *heads || probs->size(2) != v->size(1) || probs->size(3) != v->size(1) ||
         !aligned16(*probs) || !aligned16(*v)) {
         return py::none();
     }
     at::Tensor y;
     {
         py::gil_scoped_release no_gil;
-        y = attention_pv_causal_hip(*probs, *v, heads);
+        y = attention_pv_causal_hip(*probs, *v, *heads);
     }
     return wrap(y);
 }
@@ -854,12 +892,15 @@ struct LoraLinear : public torch::autograd::Function<LoraLinear> {
     }
 };
 
-py::object try_lora_linear(py::handle x_, py::handle w_, py::handle a_, py::handle b_, double scale) {
+py::object try_lora_linear(py::handle x_, py::handle w_, py::handle a_, py::handle b_, py::handle scale_) {
     const at::Tensor* x = ordinary(x_);
     const at::Tensor* w = ordinary(w_);
     const at::Tensor* a = ordinary(a_);
     const at::Tensor* b = ordinary(b_);
-    if (x == nullptr || w == nullptr || a == nullptr || b == nullptr || !ordinary_context()) return py::none();
+    const std::optional<double> scale = plain_double(scale_);
+    if (x == nullptr || w == nullptr || a == nullptr || b == nullptr || !scale || !ordinary_context()) {
+        return py::none();
+    }
     const at::ScalarType dtype = x->scalar_type();
     if (dtype != torch::kFloat32 && dtype != torch::kBFloat16) return py::none();
     for (const at::Tensor* t : {w, a, b}) {
@@ -874,7 +915,7 @@ py::object try_lora_linear(py::handle x_, py::handle w_, py::handle a_, py::hand
     {
         py::gil_scoped_release no_gil;
         const at::Tensor rows = x->dim() == 2 ? *x : x->view({-1, x->size(-1)});
-        y = grad ? LoraLinear::apply(rows, *w, *a, *b, scale) : lora_linear_hip(rows, *w, *a, *b, scale);
+        y = grad ? LoraLinear::apply(rows, *w, *a, *b, *scale) : lora_linear_hip(rows, *w, *a, *b, *scale);
         if (x->dim() != 2) {
             std::vector<int64_t> shape = x->sizes().vec();
             shape.back() = w->size(1);
@@ -986,17 +1027,19 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
     m.doc() = "cudaforge operators on MI355X (gfx950) HIP kernels";
     m.def("cuda_kernels_available", &cudaforge_amd::cuda_kernels_available,
           "True when the extension was compiled with its HIP kernels");
-    // Each returns None when the call is not an ordinary GPU one.
-    m.def("try_rmsnorm", &cudaforge_amd::try_rmsnorm);
-    m.def("try_fused_residual_rmsnorm", &cudaforge_amd::try_fused_residual_rmsnorm);
-    m.def("try_softmax", &cudaforge_amd::try_softmax);
-    m.def("try_softmax_scaled", &cudaforge_amd::try_softmax_scaled);
-    m.def("try_silu", &cudaforge_amd::try_unary<&cudaforge_amd::silu_hip>);
-    m.def("try_gelu", &cudaforge_amd::try_unary<&cudaforge_amd::gelu_hip>);
-    m.def("try_swiglu", &cudaforge_amd::try_swiglu);
-    m.def("try_quantize_int8", &cudaforge_amd::try_quantize_int8);
-    m.def("try_dequantize_int8", &cudaforge_amd::try_dequantize_int8);
-    m.def("try_attention_scores", &cudaforge_amd::try_attention_scores);
-    m.def("try_attention_pv", &cudaforge_amd::try_attention_pv);
-    m.def("try_lora_linear", &cudaforge_amd::try_lora_linear);
+    // Each returns None when the call is not an ordinary GPU one. The wrapper
+    // raises what the dispatcher would (torch.OutOfMemoryError, an exception of
+    // a saved-tensor hook as it is).
+    m.def("try_rmsnorm", torch::wrap_pybind_function(&cudaforge_amd::try_rmsnorm));
+    m.def("try_fused_residual_rmsnorm", torch::wrap_pybind_function(&cudaforge_amd::try_fused_residual_rmsnorm));
+    m.def("try_softmax", torch::wrap_pybind_function(&cudaforge_amd::try_softmax));
+    m.def("try_softmax_scaled", torch::wrap_pybind_function(&cudaforge_amd::try_softmax_scaled));
+    m.def("try_silu", torch::wrap_pybind_function(&cudaforge_amd::try_unary<&cudaforge_amd::silu_hip>));
+    m.def("try_gelu", torch::wrap_pybind_function(&cudaforge_amd::try_unary<&cudaforge_amd::gelu_hip>));
+    m.def("try_swiglu", torch::wrap_pybind_function(&cudaforge_amd::try_swiglu));
+    m.def("try_quantize_int8", torch::wrap_pybind_function(&cudaforge_amd::try_quantize_int8));
+    m.def("try_dequantize_int8", torch::wrap_pybind_function(&cudaforge_amd::try_dequantize_int8));
+    m.def("try_attention_scores", torch::wrap_pybind_function(&cudaforge_amd::try_attention_scores));
+    m.def("try_attention_pv", torch::wrap_pybind_function(&cudaforge_amd::try_attention_pv));
+    m.def("try_lora_linear", torch::wrap_pybind_function(&cudaforge_amd::try_lora_linear));
 }

@@ -56,7 +56,9 @@ _EXTENSION_LOADED, _CUDA_COMPILED, _LOAD_MESSAGE = _load_extension()
 
 # The extension's direct entry for ordinary GPU calls (torch_ops.cpp): each
 # _DIRECT.try_* returns None for a call it does not take, and the operator goes
-# on below. None without the extension.
+# on below. None without the extension. torch.compile cannot trace it, so under
+# compilation every call goes the general way.
+_compiling = torch.compiler.is_dynamo_compiling
 if _EXTENSION_LOADED and _CUDA_COMPILED:
     from cuda_force_amd import _C as _DIRECT  # type: ignore[attr-defined]
 else:
@@ -217,7 +219,7 @@ def rmsnorm(x: torch.Tensor, weight: torch.Tensor, eps: float = 1e-6) -> torch.T
     Raises:
         ValueError: if ``weight`` is not 1-D or does not match the last dim.
     """
-    if _DIRECT is not None:
+    if _DIRECT is not None and not _compiling():
         direct = _DIRECT.try_rmsnorm(x, weight, eps)
         if direct is not None:
             return direct
@@ -245,7 +247,7 @@ def rmsnorm(x: torch.Tensor, weight: torch.Tensor, eps: float = 1e-6) -> torch.T
 
 def softmax(x: torch.Tensor) -> torch.Tensor:
     """Row softmax over the last dimension (max-subtracted, fp32 arithmetic)."""
-    if _DIRECT is not None:
+    if _DIRECT is not None and not _compiling():
         direct = _DIRECT.try_softmax(x, None)
         if direct is not None:
             return direct
@@ -263,7 +265,7 @@ def softmax_as(x: torch.Tensor, dtype: torch.dtype) -> torch.Tensor:
 
     Not in the reference: lets bf16 logits produce fp32 probabilities in one
     pass (torch.softmax(x.float(), -1).to(dtype) otherwise)."""
-    if _DIRECT is not None:
+    if _DIRECT is not None and not _compiling():
         direct = _DIRECT.try_softmax(x, dtype)
         if direct is not None:
             return direct
@@ -302,8 +304,8 @@ def softmax_scaled(
     causal`` and ``softmax``, in one pass that does not read the masked
     scores. Result in ``dtype`` (default: the input's); fp32 arithmetic. Not
     in the reference's API."""
-    if _DIRECT is not None and type(causal_period) is int:
-        direct = _DIRECT.try_softmax_scaled(x, float(scale), causal_period, dtype)
+    if _DIRECT is not None and not _compiling():
+        direct = _DIRECT.try_softmax_scaled(x, scale, causal_period, dtype)
         if direct is not None:
             return direct
     dtype = x.dtype if dtype is None else dtype
@@ -356,7 +358,7 @@ def attention_scores_causal(q: torch.Tensor, k: torch.Tensor, heads: int) -> tor
     follow it with ``softmax_scaled(..., causal_period=seq)``, which never
     reads them. bf16 with head_dim 32/64/96/128 and seq a multiple of 8 runs
     the MFMA kernel on a GPU. Not in the reference's API."""
-    if _DIRECT is not None and type(heads) is int:
+    if _DIRECT is not None and not _compiling():
         direct = _DIRECT.try_attention_scores(q, k, heads)
         if direct is not None:
             return direct
@@ -386,7 +388,7 @@ def attention_pv_causal(probs: torch.Tensor, v: torch.Tensor, heads: int) -> tor
     The product of examples/transformer_block.py:63 with its transpose and
     reshape folded in. Same kernel rules as ``attention_scores_causal``. Not
     in the reference's API."""
-    if _DIRECT is not None and type(heads) is int:
+    if _DIRECT is not None and not _compiling():
         direct = _DIRECT.try_attention_pv(probs, v, heads)
         if direct is not None:
             return direct
@@ -425,7 +427,7 @@ def lora_linear(
     A PEFT-layout layer (W ``[out, in]``, A ``[r, in]``, B ``[out, r]``) maps to
     ``lora_linear(x, W.t().contiguous(), A.t().contiguous(), B.t().contiguous(), alpha / r)``.
     """
-    if _DIRECT is not None:
+    if _DIRECT is not None and not _compiling():
         direct = _DIRECT.try_lora_linear(x, weight, lora_a, lora_b, scale)
         if direct is not None:
             return direct
@@ -472,7 +474,7 @@ def fused_residual_rmsnorm(
     ``x`` and ``residual`` differ in shape or ``weight`` does not match their
     last dimension.
     """
-    if _DIRECT is not None:
+    if _DIRECT is not None and not _compiling():
         direct = _DIRECT.try_fused_residual_rmsnorm(x, residual, weight, eps)
         if direct is not None:
             return direct
@@ -503,7 +505,7 @@ def fused_residual_rmsnorm(
 
 def silu(x: torch.Tensor) -> torch.Tensor:
     """SiLU (swish): ``x * sigmoid(x)``."""
-    if _DIRECT is not None:
+    if _DIRECT is not None and not _compiling():
         direct = _DIRECT.try_silu(x)
         if direct is not None:
             return direct
@@ -518,7 +520,7 @@ def silu(x: torch.Tensor) -> torch.Tensor:
 
 def gelu(x: torch.Tensor) -> torch.Tensor:
     """GELU, tanh approximation."""
-    if _DIRECT is not None:
+    if _DIRECT is not None and not _compiling():
         direct = _DIRECT.try_gelu(x)
         if direct is not None:
             return direct
@@ -537,7 +539,7 @@ def swiglu(gate: torch.Tensor, up: torch.Tensor) -> torch.Tensor:
     ``gate`` and ``up`` must agree in shape and dtype; otherwise a
     ``ValueError`` is raised before anything runs.
     """
-    if _DIRECT is not None:
+    if _DIRECT is not None and not _compiling():
         direct = _DIRECT.try_swiglu(gate, up)
         if direct is not None:
             return direct
@@ -588,7 +590,7 @@ def quantize_int8(x: torch.Tensor) -> tuple[torch.Tensor, torch.Tensor]:
         ``(quantised, scales)``: int8 codes shaped like ``x`` and one fp32
         scale per ``QUANT_BLOCK_SIZE`` elements of the flattened input.
     """
-    if _DIRECT is not None:
+    if _DIRECT is not None and not _compiling():
         direct = _DIRECT.try_quantize_int8(x)
         if direct is not None:
             return direct
@@ -609,7 +611,7 @@ def dequantize_int8(
     the scales' dtype, float32. A half dtype equals the float32 result
     followed by ``.to(dtype)``, computed in one pass.
     """
-    if _DIRECT is not None:
+    if _DIRECT is not None and not _compiling():
         direct = _DIRECT.try_dequantize_int8(quantised, scales, dtype)
         if direct is not None:
             return direct

@@ -116,3 +116,47 @@ def test_lora_autograd_node_keeps_hooks_and_partial_gradients():
         (exact,) = torch.autograd.grad(ref[0] @ ref[1] + 2.0 * ((ref[0] @ ref[2]) @ ref[3]), ref[i], dy.double())
         # bf16 GEMMs and one rounded intermediate: 2^-7 of the largest value.
         assert (grad.double() - exact).abs().max() <= 2.0**-7 * exact.abs().max()
+
+
+def test_arguments_the_direct_entry_does_not_read():
+    direct = ops._DIRECT
+    x, w = _rand(6, 64), _rand(64, seed=1)
+    for eps in (None, "1", True, 1j, 10**400, torch.tensor(1e-6), torch.ones(64)):
+        assert direct.try_rmsnorm(x, w, eps) is None
+    assert direct.try_rmsnorm(x, w, 0) is not None
+    for dtype in (float, "float32", torch.float64, torch.int32):
+        assert direct.try_softmax(x, dtype) is None
+    for period in (True, 2**70, -1, 2.0):
+        assert direct.try_softmax_scaled(x, 1.0, period, None) is None
+    with pytest.raises(RuntimeError, match="Expected a value of type 'float'"):
+        ops.rmsnorm(x, w, None)
+
+
+def test_forward_mode_is_refused_not_dropped():
+    with torch.autograd.forward_ad.dual_level():
+        x = torch.autograd.forward_ad.make_dual(_rand(6, 64), _rand(6, 64, seed=1))
+        with pytest.raises(NotImplementedError, match="forward AD"):
+            ops.softmax(x)
+
+
+def test_errors_keep_their_types():
+    x = torch.zeros(1 << 24, device="cuda")
+    used = torch.cuda.memory_reserved() / torch.cuda.get_device_properties(0).total_memory
+    torch.cuda.empty_cache()
+    torch.cuda.set_per_process_memory_fraction(min(1.0, used * 0.5), 0)
+    try:
+        with pytest.raises(torch.OutOfMemoryError):
+            kept = [ops.silu(x) for _ in range(64)]
+            del kept
+    finally:
+        torch.cuda.set_per_process_memory_fraction(1.0, 0)
+
+    class Stop(Exception):
+        pass
+
+    def pack(t):
+        raise Stop
+
+    operands = _rand(70, 64), _rand(64, 40, seed=1), _rand(64, 8, seed=2).requires_grad_(), _rand(8, 40, seed=3)
+    with torch.autograd.graph.saved_tensors_hooks(pack, lambda t: t), pytest.raises(Stop):
+        ops.lora_linear(*operands, 2.0)
