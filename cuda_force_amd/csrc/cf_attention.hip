@@ -24,8 +24,8 @@
 // column l % 16, each over k = 8 (l / 16) .. +7, and D rows 4 (l / 16) + i of
 // column l % 16):
 //   * scores are computed transposed, S^T = K Q^T. The tile's q and k rows
-//     are copied into LDS by buffer loads with the LDS destination (whole
-//     256-byte rows, chunks swizzled for conflict-free reads); A and B
+//     are copied into LDS, 64 dims at a time, by buffer loads with the LDS
+//     destination (128-byte pieces, swizzled for conflict-free reads); A and B
 //     fragments are ds_read_b128 of k and q rows (head_dim is the contiguous
 //     reduction index of both), and a lane ends with four consecutive keys
 //     of one query row; each wave's 64 x 64 tile is then staged in LDS and
@@ -54,7 +54,8 @@ constexpr int kScoreTile = 128;  // queries and keys per scores workgroup
 constexpr int kPvRows = 64;      // query rows per out workgroup (16 per wave)
 constexpr int kPvChunk = 64;     // keys per step of the out product (two MFMA k-steps)
 constexpr int kPvSub = kPvChunk / 32;
-constexpr int kVPitch = 256;     // LDS bytes per staged q, k or v row (head_dim <= 128)
+constexpr int kVPitch = 256;     // LDS bytes per staged v row (head_dim <= 128)
+constexpr int kHalfPitch = 128;  // LDS bytes per staged half of a q or k row (64 dims)
 // A buffer offset past every range this file builds (all below 2^31): the
 // load returns zeros. Rows past seq take it rather than their own offset,
 // which for a large pitch could wrap around 2^32.
@@ -96,16 +97,26 @@ __device__ __forceinline__ int64_t xcd_local(int64_t pid, int64_t total) {
 /// scores for the causal tiles. Logical id = bh * tiles + tile, tile
 /// enumerating the tiles (si, ti) with ti <= si row by row. The tile's 128
 /// query rows and 128 key rows are copied HBM -> LDS by buffer loads with
-/// the LDS destination (each load 4 whole rows), so every row is read once
-/// per workgroup in whole 256-byte pieces.
+/// the LDS destination (each load 8 rows of 128 bytes), so every row is read
+/// once per workgroup.
+///
+/// Per tile a CU spends about as long copying 64 KiB of rows, reading LDS and
+/// storing 32 KiB, one after the other in a workgroup, so what counts is how
+/// many workgroups of a CU are in different phases: staging 64 dims at a time
+/// takes 32 KiB of LDS and (with 32-bit offsets) 124 registers, four
+/// workgroups a CU instead of the two of whole 256-byte rows. [1, 2048, 32 x
+/// 128] 62.7 -> 52.4 us, [8, 512, 32 x 128] 38.0 -> 32.0, [1, 1000, 32 x 128]
+/// 15.5 -> 13.2, [2, 1024, 32 x 64] 26.4 -> 22.2 (three workgroups: 55.0,
+/// 33.5, 13.0).
 template <int kD>
-__global__ __launch_bounds__(kThreads) void attention_scores_kernel(const uint16_t* __restrict__ q,
+__global__ __launch_bounds__(kThreads, 4) void attention_scores_kernel(const uint16_t* __restrict__ q,
                                                                     const uint16_t* __restrict__ k,
                                                                     uint16_t* __restrict__ scores, int64_t seq,
                                                                     int64_t heads, int tiles) {
-    // q rows then k rows, 128 each at a 256-byte pitch, 16-byte chunk c of
-    // row r at c ^ (r & 15); afterwards each wave's 8 KiB output staging.
-    __shared__ __attribute__((aligned(16))) uint8_t lds[2 * kScoreTile * kVPitch];  // 64 KiB
+    // 64 dims of the q rows, then of the k rows, 128 rows each at a 128-byte
+    // pitch, 16-byte chunk c of row r at c ^ ((r >> 1) & 7); afterwards each
+    // wave's 8 KiB output staging.
+    __shared__ __attribute__((aligned(16))) uint8_t lds[2 * kScoreTile * kHalfPitch];  // 32 KiB
     const int64_t id = xcd_local(blockIdx.x, static_cast<int64_t>(gridDim.x));
     const int64_t bh = id / tiles;
     const int tile = static_cast<int>(id % tiles);
@@ -127,31 +138,13 @@ __global__ __launch_bounds__(kThreads) void attention_scores_kernel(const uint16
     const int64_t b = bh / heads;
     const int64_t h = bh % heads;
     const int64_t head0 = (b * seq * heads + h) * kD;  // element of row 0, dim 0
-    const int64_t pitch = heads * kD;                  // elements between consecutive rows
+    // The slice is below 2^31 bytes, so rows and offsets are 32-bit.
+    const uint32_t pitch_bytes = static_cast<uint32_t>(heads * kD * 2);
+    const uint32_t rows = static_cast<uint32_t>(seq);
     const uint32_t extent = head_extent(seq, heads, kD);
     const i32x4_t qbuf = uniform(raw_buffer_words(q + head0, extent));
     const i32x4_t kbuf = uniform(raw_buffer_words(k + head0, extent));
     const uint32_t lds_addr = static_cast<uint32_t>(reinterpret_cast<size_t>((lds_u8_t*)lds));
-
-    // Load n (0..31) of an operand fills rows 4 n .. 4 n + 3 of its tile:
-    // lane l lands at byte 16 l, i.e. row 4 n + l / 16, physical chunk
-    // l % 16, so it reads logical chunk (l % 16) ^ (row & 15). Rows past
-    // seq and chunks past the head (head_dim < 128) read as zero.
-    const int phys = lane & 15;
-#pragma unroll
-    for (int i = 0; i < 8; ++i) {
-        const int n = 8 * wave + i;
-        const int r = 4 * n + (lane >> 4);
-        const int c = phys ^ (r & 15);
-        const int64_t qr = q_row0 + r;
-        const int64_t kr = k_row0 + r;
-        const uint32_t qoff = qr < seq && c < kD / 8 ? static_cast<uint32_t>((qr * pitch + 8 * c) * 2) : kPastEnd;
-        const uint32_t koff = kr < seq && c < kD / 8 ? static_cast<uint32_t>((kr * pitch + 8 * c) * 2) : kPastEnd;
-        dma16_m0(qbuf, lds_addr + static_cast<uint32_t>(n * 1024), qoff, 0);
-        dma16_m0(kbuf, lds_addr + static_cast<uint32_t>(kScoreTile * kVPitch + n * 1024), koff, 0);
-    }
-    __builtin_amdgcn_s_waitcnt(vmcnt_imm(0));
-    __syncthreads();
 
     const int j = lane & 15;
     const int g = lane >> 4;
@@ -161,27 +154,52 @@ __global__ __launch_bounds__(kThreads) void attention_scores_kernel(const uint16
 #pragma unroll
         for (int sb = 0; sb < 4; ++sb) acc[tb][sb] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
     }
-    if (active) {
-        // Fragment rows: key block tb is tile row (wave & 1) * 64 + 16 tb + j
-        // (A), query block sb tile row (wave >> 1) * 64 + 16 sb + j (B); both
-        // have row & 15 == j. K-step kk takes logical chunk 4 kk + g.
-        const uint8_t* kt = lds + kScoreTile * kVPitch + ((wave & 1) * 64 + j) * kVPitch;
-        const uint8_t* qt = lds + ((wave >> 1) * 64 + j) * kVPitch;
+    // Load n (0..15) of an operand fills rows 8 n .. 8 n + 7 of its tile:
+    // lane l lands at byte 16 l, i.e. row 8 n + l / 8, physical chunk l % 8,
+    // so it reads logical chunk (l % 8) ^ ((row >> 1) & 7) of the half. Rows
+    // past seq and chunks past the head (head_dim 32 or 96) read as zero.
+    const int phys = lane & 7;
+#pragma unroll 1  // unrolled, the second half's offsets cost 30 registers
+    for (int half = 0; half < (kD + 63) / 64; ++half) {
+        if (half > 0) __syncthreads();  // every wave has read the half before
 #pragma unroll
-        for (int kk = 0; kk < kD / 32; ++kk) {
-            const int off = ((4 * kk + g) ^ j) << 4;
-            bf16x8_t a[4];
-            bf16x8_t bq[4];
+        for (int i = 0; i < 4; ++i) {
+            const int n = 4 * wave + i;
+            const int r = 8 * n + (lane >> 3);
+            const int c = 8 * half + (phys ^ ((r >> 1) & 7));
+            const bool dims = c < kD / 8;
+            const uint32_t qr = static_cast<uint32_t>(q_row0) + r;
+            const uint32_t kr = static_cast<uint32_t>(k_row0) + r;
+            const uint32_t qoff = qr < rows && dims ? qr * pitch_bytes + 16 * c : kPastEnd;
+            const uint32_t koff = kr < rows && dims ? kr * pitch_bytes + 16 * c : kPastEnd;
+            dma16_m0(qbuf, lds_addr + static_cast<uint32_t>(n * 1024), qoff, 0);
+            dma16_m0(kbuf, lds_addr + static_cast<uint32_t>(kScoreTile * kHalfPitch + n * 1024), koff, 0);
+        }
+        __builtin_amdgcn_s_waitcnt(vmcnt_imm(0));
+        __syncthreads();
+        if (active) {
+            // Fragment rows: key block tb is tile row (wave & 1) * 64 + 16 tb
+            // + j (A), query block sb tile row (wave >> 1) * 64 + 16 sb + j
+            // (B); both have (row >> 1) & 7 == j >> 1. K-step kk of the half
+            // takes its logical chunk 4 kk + g.
+            const uint8_t* kt = lds + kScoreTile * kHalfPitch + ((wave & 1) * 64 + j) * kHalfPitch;
+            const uint8_t* qt = lds + ((wave >> 1) * 64 + j) * kHalfPitch;
 #pragma unroll
-            for (int blk = 0; blk < 4; ++blk) {
-                a[blk] = *reinterpret_cast<const bf16x8_t*>(kt + blk * 16 * kVPitch + off);
-                bq[blk] = *reinterpret_cast<const bf16x8_t*>(qt + blk * 16 * kVPitch + off);
-            }
+            for (int kk = 0; kk < 2 && 64 * half + 32 * kk < kD; ++kk) {
+                const int off = ((4 * kk + g) ^ (j >> 1)) << 4;
+                bf16x8_t a[4];
+                bf16x8_t bq[4];
 #pragma unroll
-            for (int tb = 0; tb < 4; ++tb) {
+                for (int blk = 0; blk < 4; ++blk) {
+                    a[blk] = *reinterpret_cast<const bf16x8_t*>(kt + blk * 16 * kHalfPitch + off);
+                    bq[blk] = *reinterpret_cast<const bf16x8_t*>(qt + blk * 16 * kHalfPitch + off);
+                }
 #pragma unroll
-                for (int sb = 0; sb < 4; ++sb) {
-                    acc[tb][sb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[tb], bq[sb], acc[tb][sb], 0, 0, 0);
+                for (int tb = 0; tb < 4; ++tb) {
+#pragma unroll
+                    for (int sb = 0; sb < 4; ++sb) {
+                        acc[tb][sb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[tb], bq[sb], acc[tb][sb], 0, 0, 0);
+                    }
                 }
             }
         }
@@ -210,15 +228,20 @@ __global__ __launch_bounds__(kThreads) void attention_scores_kernel(const uint16
     __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
     __builtin_amdgcn_wave_barrier();
     // seq is a multiple of 8, so eight keys never straddle its end.
-    uint16_t* out = scores + bh * seq * seq;
+    // row & 7 is lane >> 3 for each of a lane's rows.
     const int c = lane & 7;
+    const int row0 = lane >> 3;
+    const uint8_t* from = stage + row0 * 128 + ((c ^ row0) << 4);
+    uint8_t* out = reinterpret_cast<uint8_t*>(scores + bh * seq * seq + s0 * seq + t0);
+    const uint32_t row_bytes = static_cast<uint32_t>(seq) * 2;
+    const int rows_left = static_cast<int>(seq - s0);
+    if (t0 + 8 * c < seq) {
 #pragma unroll
-    for (int i = 0; i < 8; ++i) {
-        const int row = 8 * i + (lane >> 3);
-        const int64_t s = s0 + row;
-        const int64_t t = t0 + 8 * c;
-        const uint4 v = *reinterpret_cast<const uint4*>(stage + row * 128 + ((c ^ (row & 7)) << 4));
-        if (s < seq && t < seq) *reinterpret_cast<uint4*>(out + s * seq + t) = v;
+        for (int i = 0; i < 8; ++i) {
+            const int row = 8 * i + row0;
+            const uint4 v = *reinterpret_cast<const uint4*>(from + i * 1024);
+            if (row < rows_left) *reinterpret_cast<uint4*>(out + (static_cast<uint32_t>(row) * row_bytes + 16 * c)) = v;
+        }
     }
 }
 
