@@ -4,7 +4,8 @@ Same names, signatures, argument meaning, validation errors and fallback rules
 as the reference module (python/cudaforge/ops.py:41-488). What changes is what
 runs underneath: on a GPU tensor every operator here dispatches to
 ``torch.ops.cudaforge.*``, whose CUDA-key implementation calls the gfx950 HIP
-kernels in ``libcudaforge_hip.so``.
+kernels in ``libcudaforge_hip.so``; an ordinary call reaches the same
+implementation without the dispatcher (``_DIRECT`` below).
 
 Dispatch rules (reference ops.py:125-153, widened):
 
