@@ -269,7 +269,15 @@ std::tuple<torch::Tensor, torch::Tensor, torch::Tensor> lora_backward_hip(
     }
     const at::DeviceGuard guard(x.device());
     torch::Tensor grad_x;
-    if (w != nullptr) grad_x = at::mm(dy, w->t());
+    if (w != nullptr) {
+        // A backward inside an autocast block runs here with its keys on: mm
+        // would then return another dtype than the kernel below is told.
+        const c10::impl::ExcludeDispatchKeyGuard no_autocast(c10::autocast_dispatch_keyset);
+        grad_x = at::mm(dy, w->t());
+        TORCH_CHECK(grad_x.scalar_type() == x.scalar_type() && grad_x.is_contiguous() &&
+                        grad_x.sizes() == x.sizes(),
+                    "dy @ w^T is not a contiguous ", x.scalar_type(), " tensor of x's shape");
+    }
     torch::Tensor grad_a = torch::empty({in_features, rank}, x.options());
     torch::Tensor grad_b = torch::empty({rank, out_features}, x.options());
     const size_t bytes = cf_lora_backward_workspace_bytes(batch, in_features, out_features, rank);
@@ -526,6 +534,8 @@ std::tuple<torch::Tensor, torch::Tensor> lora_linear_bwd_cpu(const torch::Tensor
 std::tuple<torch::Tensor, torch::Tensor, torch::Tensor> lora_linear_bwd_input_cpu(
     const torch::Tensor& x, const torch::Tensor& dy, const torch::Tensor& w, const torch::Tensor& a,
     const torch::Tensor& b, const torch::Tensor& xa, double scale) {
+    // As on the GPU: the operands' dtype, whatever autocast is on.
+    const c10::impl::ExcludeDispatchKeyGuard no_autocast(c10::autocast_dispatch_keyset);
     const torch::Tensor grad_x =
         torch::matmul(dy, w.t()) + scale * torch::matmul(torch::matmul(dy, b.t()), a.t());
     auto [grad_a, grad_b] = lora_linear_bwd_cpu(x, dy, b, xa, scale);
