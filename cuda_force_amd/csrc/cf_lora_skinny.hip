@@ -375,8 +375,16 @@ size_t align256(size_t bytes) { return (bytes + 255) / 256 * 256; }
 }  // namespace
 
 bool lora_skinny_shape(int64_t M, int64_t N, int64_t K, int64_t rank) {
-    return M >= 1 && M <= kSkinnyMaxRows && N > 0 && K > 0 && N % 8 == 0 && K % 8 == 0 && rank >= 0 &&
-           rank <= kMaxRank && K * N * 2 < (1LL << 31) && M * K * 2 < (1LL << 31);
+    if (M < 1 || M > kSkinnyMaxRows || N <= 0 || K <= 0 || N % 8 != 0 || K % 8 != 0 || rank < 0 ||
+        rank > kMaxRank) {
+        return false;
+    }
+    // Each operand, and the partials, are read through a buffer whose offsets
+    // are 32-bit with the out-of-range marker at 2^31. (The partials of x @ a,
+    // at most 768 slices of 64 x 256, are 50 MB.)
+    constexpr int64_t kLimit = 1LL << 31;
+    return K < kLimit && N < kLimit && K * N * 2 < kLimit && M * K * 2 < kLimit && K * rank * 2 < kLimit &&
+           rank * N * 2 < kLimit && plan_for(M, N, K, rank).slices * M * N * 4 < kLimit;
 }
 
 bool lora_skinny_eligible(const void* x, const void* w, const void* a, const void* b, const void* y,

@@ -54,6 +54,27 @@ def test_workspace_queries(lib):
     assert lib.cf_abi_version() == 1
 
 
+@pytest.mark.parametrize("m,k,n,rank,few_rows", [
+    (64, 64, 8388600, 16, True),     # partials just below 2 GiB
+    (64, 64, 8388608, 16, False),    # at 2 GiB
+    (64, 64, 9000000, 16, False),
+    (1, 8, 4194296, 256, True),      # b just below 2 GiB
+    (1, 8, 4194304, 256, False),
+    (1, 4194296, 8, 256, True),      # a just below 2 GiB
+    (1, 4194304, 8, 256, False),
+])
+def test_few_row_lora_stops_where_a_buffer_reaches_2_gib(lib, m, k, n, rank, few_rows):
+    # The few-row kernels' fp32 partials are the only workspace that large here.
+    partials = m * n * 4
+    needed = lib.cf_lora_forward_workspace_bytes(_lib.CF_BF16, m, k, n, rank)
+    if few_rows:
+        assert needed >= partials + m * rank * 4
+    elif rank > 128:  # nothing else takes the rank with a workspace
+        assert needed == lib.cf_lora_linear_ws_bytes(_lib.CF_BF16, m, k, n, rank)
+    else:
+        assert needed < partials
+
+
 def test_empty_inputs_return_ok_without_touching_the_device(lib):
     null = ctypes.c_void_p(0)
     assert lib.cf_quantize_int8(null, _lib.CF_F32, null, null, 0, null) == _lib.CF_OK
