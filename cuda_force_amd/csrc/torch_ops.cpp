@@ -635,18 +635,22 @@ bool ordinary_context() {
            local.excluded_.has(c10::DispatchKey::AutocastCUDA) && !at::impl::torch_function_mode_enabled() && !at::hasCallbacks();
 }
 
-/// The tensor behind `object`, or null when it is not a plain dense GPU tensor
-/// that is contiguous, not empty and without a forward-mode tangent.
-const at::Tensor* ordinary(py::handle object) {
+/// Dense GPU storage, no dispatch key beyond CUDA and its autograd, and no
+/// forward-mode tangent.
+bool plain_gpu(const at::Tensor& t) {
     static const c10::DispatchKeySet usual(
         {c10::DispatchKey::CUDA, c10::DispatchKey::AutogradCUDA, c10::DispatchKey::AutocastCUDA,
          c10::DispatchKey::ADInplaceOrView});
+    return t.defined() && t.key_set().has(c10::DispatchKey::CUDA) &&
+           (t.key_set().raw_repr() & ~usual.raw_repr()) == 0 && !t._fw_grad(0).defined();
+}
+
+/// The tensor behind `object`, or null when it is not a plain GPU tensor that
+/// is contiguous and not empty.
+const at::Tensor* ordinary(py::handle object) {
     if (!THPVariable_CheckTypeExact(Py_TYPE(object.ptr()))) return nullptr;
     const at::Tensor& t = THPVariable_Unpack(object.ptr());
-    if (!t.defined() || !t.key_set().has(c10::DispatchKey::CUDA) || (t.key_set().raw_repr() & ~usual.raw_repr()) != 0) {
-        return nullptr;
-    }
-    return t.is_contiguous() && t.numel() > 0 && !t._fw_grad(0).defined() ? &t : nullptr;
+    return plain_gpu(t) && t.is_contiguous() && t.numel() > 0 ? &t : nullptr;
 }
 
 // The other arguments come as Python objects: a value that is not plainly a
@@ -881,18 +885,31 @@ struct LoraLinear : public torch::autograd::Function<LoraLinear> {
         const bool adapter = ctx->needs_input_grad(2) || ctx->needs_input_grad(3);
         const bool recorded = at::GradMode::is_enabled();
         const bool fused_x = adapter && ctx->needs_input_grad(0) && !recorded;
-        if (adapter && recorded) {
-            // Through the dispatcher, whose autograd entry refuses to
-            // differentiate the adapter gradients.
+        // The gradient and what saved-tensor hooks return need not be as plain
+        // as the operands were, nor the context as it was in the forward: a
+        // batched gradient (is_grads_batched) has no storage, a mode or a
+        // profiler may have been entered since. Those calls go through the
+        // dispatcher, and so does a recorded one, whose autograd entry refuses
+        // to differentiate the adapter gradients.
+        const bool direct = !recorded && ordinary_context() && plain_gpu(dy) && plain_gpu(x) && plain_gpu(w) &&
+                            plain_gpu(a) && plain_gpu(b) && plain_gpu(xa);
+        if (adapter && direct) {
+            std::tie(grad_x, grad_a, grad_b) =
+                lora_backward_hip(x, dy, fused_x ? &w : nullptr, fused_x ? &a : nullptr, b, xa, scale);
+        } else if (fused_x) {
+            static const auto op = c10::Dispatcher::singleton()
+                                       .findSchemaOrThrow("cudaforge::lora_linear_bwd_input", "")
+                                       .typed<std::tuple<at::Tensor, at::Tensor, at::Tensor>(
+                                           const at::Tensor&, const at::Tensor&, const at::Tensor&,
+                                           const at::Tensor&, const at::Tensor&, const at::Tensor&, double)>();
+            std::tie(grad_x, grad_a, grad_b) = op.call(x, dy, w, a, b, xa, scale);
+        } else if (adapter) {
             static const auto op = c10::Dispatcher::singleton()
                                        .findSchemaOrThrow("cudaforge::lora_linear_bwd", "")
                                        .typed<std::tuple<at::Tensor, at::Tensor>(
                                            const at::Tensor&, const at::Tensor&, const at::Tensor&,
                                            const at::Tensor&, double)>();
             std::tie(grad_a, grad_b) = op.call(x, dy, b, xa, scale);
-        } else if (adapter) {
-            std::tie(grad_x, grad_a, grad_b) =
-                lora_backward_hip(x, dy, fused_x ? &w : nullptr, fused_x ? &a : nullptr, b, xa, scale);
         }
         if (ctx->needs_input_grad(0) && !fused_x) {
             grad_x = at::matmul(dy, w.t()) + scale * at::matmul(at::matmul(dy, b.t()), a.t());

@@ -1,5 +1,5 @@
-"""The backward of the LoRA linear when it is called inside autocast: the same
-gradients, in the operands' dtype."""
+"""The backward of the LoRA linear when it is called inside autocast (the same
+gradients, in the operands' dtype) and with batched gradients."""
 
 from __future__ import annotations
 
@@ -41,3 +41,14 @@ def test_backward_inside_autocast_equals_the_one_outside():
             grads.append(torch.autograd.grad(y.square().sum(), leaves))
     for u, v in zip(*grads):
         assert torch.equal(u, v)
+
+
+def test_batched_gradients_equal_one_at_a_time():
+    x, w, a, b = _operands(torch.float32)
+    leaves = [x.requires_grad_(), a.requires_grad_(), b.requires_grad_()]
+    y = lora_linear_autograd(x, w, a, b, 0.5)
+    dy = torch.randn(3, 7, 16, generator=torch.Generator().manual_seed(1))
+    batched = torch.autograd.grad(y, leaves, dy, is_grads_batched=True, retain_graph=True)
+    singly = [torch.autograd.grad(y, leaves, row, retain_graph=True) for row in dy]
+    for got, want in zip(batched, (torch.stack(t) for t in zip(*singly))):
+        torch.testing.assert_close(got, want, rtol=1e-5, atol=1e-5)
