@@ -356,17 +356,19 @@ __global__ __launch_bounds__(kThreads, kRB == 1 ? 1 : 2) void column_mfma_kernel
 
 /// gt[j, m] = bf16(sum over column tiles of gpart[tile][m][j]), fixed order,
 /// and the same row by row in g when that is wanted; thread i of the launch
-/// handles element i.
+/// handles element i. Zero past the rank, where the partials of a row with an
+/// infinite dy hold NaN (infinity times the padding of b).
 template <int kRankPad>
 __device__ __forceinline__ void sum_g(const float* __restrict__ gpart, uint16_t* __restrict__ gt,
-                                      uint16_t* __restrict__ g, int64_t M, int64_t Mp, int64_t tiles, int64_t i) {
+                                      uint16_t* __restrict__ g, int64_t M, int64_t Mp, int64_t rank, int64_t tiles,
+                                      int64_t i) {
     if (i >= kRankPad * Mp) return;
     const int64_t m = i / kRankPad;
     const int64_t j = i % kRankPad;
     // Rows past M are zero, whether or not the dy pass's tiles reach them
     // (the x pass's may be taller).
     float total = 0.0f;
-    if (m < M) total = ordered_sum(tiles, [&](int64_t t) { return gpart[(t * Mp + m) * kRankPad + j]; });
+    if (m < M && j < rank) total = ordered_sum(tiles, [&](int64_t t) { return gpart[(t * Mp + m) * kRankPad + j]; });
     const uint16_t bits = static_cast<uint16_t>(f32_to_bf16_bits(total));
     gt[j * Mp + m] = bits;
     if (g != nullptr) g[i] = bits;
@@ -403,7 +405,7 @@ __global__ __launch_bounds__(kThreads) void after_dy_kernel(const float* __restr
     if (block < grad_b_blocks) {
         finish<false, kRankPad>(colpart, grad_b, row_tiles, rank, N, scale, block * kThreads + threadIdx.x);
     } else {
-        sum_g<kRankPad>(gpart, gt, g, M, Mp, col_tiles, (block - grad_b_blocks) * kThreads + threadIdx.x);
+        sum_g<kRankPad>(gpart, gt, g, M, Mp, rank, col_tiles, (block - grad_b_blocks) * kThreads + threadIdx.x);
     }
 }
 

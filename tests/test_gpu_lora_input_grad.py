@@ -2,7 +2,7 @@
 plus the adapter's part added in place by the HIP kernels) against float64:
 every rank block count, ranks with and without whole 16-byte rows of a, row
 and column remainders, the generic path (fp32, odd widths, rank above 64),
-and the composed path a recorded backward takes."""
+infinite gradients, and the composed path a recorded backward takes."""
 
 from __future__ import annotations
 
@@ -49,6 +49,30 @@ def test_input_gradient_matches_float64(dtype, shape):
         err = (got.double() - want[name]).abs()
         bound = rel * want[name].abs() + floor * want[name].abs().max()
         assert bool((err <= bound).all()), f"{name}: max err {err.max().item():.3e}"
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("rank", [1, 5, 16, 17, 40, 64, 70])
+def test_infinite_gradients_stay_infinite(dtype, rank):
+    """dy = +-inf at a column where w, a and b are positive: every term of that
+    row of grad_x is the same infinity (ranks that the kernels pad included),
+    and the other rows are the ones without it."""
+    g.announce(f"LoRA input gradient with infinities {dtype} rank {rank}")
+    x, w, a, b, dy = _operands(70, 264, 72, rank, dtype, rank)
+    w[:, 5].abs_()
+    b[:, 5].abs_().clamp_(min=1e-3)
+    a.abs_().clamp_(min=1e-3)
+    plain = None
+    for mark in (False, True):
+        if mark:
+            dy[3, 5], dy[64, 5] = float("inf"), float("-inf")
+        leaves = [t.clone().requires_grad_() for t in (x, a, b)]
+        grad_x, _, _ = torch.autograd.grad(ops.lora_linear(leaves[0], w, leaves[1], leaves[2], 1.5), leaves, dy)
+        if mark:
+            assert bool((grad_x[3] == float("inf")).all()) and bool((grad_x[64] == float("-inf")).all())
+            rest = [i for i in range(70) if i not in (3, 64)]
+            assert torch.equal(grad_x[rest], plain[rest])
+        plain = grad_x
 
 
 def test_a_recorded_backward_can_be_differentiated_again():
