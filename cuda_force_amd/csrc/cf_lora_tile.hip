@@ -3,14 +3,15 @@
 //
 //   y[M, N] = x[M, K] @ w[K, N] + scale * bf16(x @ a)[M, r] @ b[r, N]
 //
-// The adapter is a continuation of the reduction: with u = bf16(x @ a) and
-// s * b split into bf16 high and low parts (one part when s * b is exact in
-// bf16), y = [x | u] @ [w ; s b], so the K-loop runs on over the rows of
-// s * b for one to eight more K-steps and the epilogue knows no adapter.
+// The adapter is the start of the reduction: with u = bf16(x @ a), the first
+// one to four K-steps run over the rows of b, the accumulators are multiplied
+// by the scale once, in fp32, and the K-steps of x @ w add on. So the adapter
+// is scale * (u @ b) in fp32, as written above, for any scale and any b
+// (infinities included), and the epilogue knows no adapter.
 //
 //   * lora_down_kernel forms x @ a first (16 rows per workgroup, its waves
-//     splitting K), rounds it to bf16 (as the reference materialises it) into
-//     u, and the rest of its grid writes the parts of s * b.
+//     splitting K) and rounds it to bf16 (as the reference materialises it)
+//     into u.
 //   * lora_tile_kernel: K-step 32, operands HBM -> LDS by buffer loads with the
 //     LDS destination into a ring of stages, one barrier per K-step; the
 //     fragments of step j + 1 are read while step j is multiplied, and the
@@ -26,9 +27,9 @@
 // that still fills the CUs wins, and the kernel and slice counts are chosen by
 // an estimate (below) from measured times per K-step. Before, these problems
 // ran 256x256 tiles on a fraction of the CUs or, for a rank above 16 or K not
-// a multiple of 64, fp32 FMA tiles: 333 x 4096 x 11008 r16 92 -> 59 us, 100 x
-// 4096 x 4096 r16 81 -> 24, 1237 x 4096 x 8192 r64 2801 -> 109, 3530 x 984 x
-// 11008 r16 1367 -> 104, 6000 x 11008 x 4096 r32 12650 -> 556.
+// a multiple of 64, fp32 FMA tiles: 333 x 4096 x 11008 r16 92 -> 58 us, 100 x
+// 4096 x 4096 r16 81 -> 23, 1237 x 4096 x 8192 r64 2801 -> 109, 3530 x 984 x
+// 11008 r16 1367 -> 107, 6000 x 11008 x 4096 r32 12650 -> 573.
 //
 // Everything past an edge reads as zero: rows past M and columns past N by the
 // buffer range, k past K by an offset bit (x) and by the range (w).
@@ -93,16 +94,18 @@ __device__ __forceinline__ void place_tile(int position, int tiles_m, int tiles_
 struct TileArgs {
     const uint16_t* x;    // [M, K]
     const uint16_t* w;    // [K, N]
-    const uint16_t* u;    // [M, ext]: bf16(x @ a) per part, zero-padded
-    const uint16_t* sb;   // [ext, N]: parts of scale * b, zero-padded
+    const uint16_t* u;    // [M, ext]: bf16(x @ a), zero-padded
+    const uint16_t* b;    // [rank, N]
     uint16_t* y;          // [M, N]
     float* part;          // split tiles: [tile - whole][slice][rows of the tile][columns]
     int64_t M;
     int64_t N;
     int64_t K;
-    int64_t ext;          // a multiple of kBK
-    int steps;            // K-steps of x @ w and of the adapter
-    int main_steps;       // of x @ w
+    int64_t rank;
+    int64_t ext;          // the rank as whole K-steps: a multiple of kBK
+    int steps;            // K-steps of the adapter, then of x @ w
+    int ext_steps;        // of the adapter
+    float scale;
     int tiles_m;
     int tiles_n;
     int whole;            // the first tiles take a workgroup each; those after
@@ -173,11 +176,11 @@ void lora_tile_kernel(TileArgs args) {
     const int x_chunk = (lane & 3) ^ k_swizzle(lane >> 2);
     const uint32_t x_lane = static_cast<uint32_t>(lane >> 2) * x_row + static_cast<uint32_t>(x_chunk * 16);
     const uint32_t u_lane = static_cast<uint32_t>(lane >> 2) * u_row + static_cast<uint32_t>(x_chunk * 16);
-    // w and s * b: an instruction fills 512 / kBN rows.
+    // w and b: an instruction fills 512 / kBN rows.
     constexpr int kRowChunks = kBN / 8;
     constexpr int kRowsPerPiece = 64 / kRowChunks;
     const i32x4_t wbuf = uniform(raw_buffer_words(args.w, static_cast<uint32_t>(args.K * N * 2)));
-    const i32x4_t bbuf = uniform(raw_buffer_words(args.sb, static_cast<uint32_t>(args.ext * N * 2)));
+    const i32x4_t bbuf = uniform(raw_buffer_words(args.b, static_cast<uint32_t>(args.rank * N * 2)));
     uint32_t w_lane[kWPieces];
 #pragma unroll
     for (int i = 0; i < kWPieces; ++i) {
@@ -201,8 +204,8 @@ void lora_tile_kernel(TileArgs args) {
         // Uniform already; said so that the selected descriptors stay scalar.
         step = __builtin_amdgcn_readfirstlane(step);
         slot = __builtin_amdgcn_readfirstlane(slot);
-        const bool ext = step >= args.main_steps;
-        const int k0 = (ext ? step - args.main_steps : step) * kBK;
+        const bool ext = step < args.ext_steps;
+        const int k0 = (ext ? step : step - args.ext_steps) * kBK;
         Source s;
         s.x = ext ? ubuf : xbuf;
         s.w = ext ? bbuf : wbuf;
@@ -284,6 +287,13 @@ void lora_tile_kernel(TileArgs args) {
     read_x(x0, lds);
 #pragma unroll
     for (int jb = 0; jb < kTN; ++jb) wf[jb] = read_w(lds, jb);
+    auto scale_adapter = [&]() {
+#pragma unroll
+        for (int jb = 0; jb < kTN; ++jb) {
+#pragma unroll
+            for (int i = 0; i < kTM; ++i) acc[jb][i] *= args.scale;
+        }
+    };
     int slot = 0;
     auto step = [&](int kt, bf16x8_t (&cur)[kTM], bf16x8_t (&nxt)[kTM]) {
         arrive();
@@ -304,6 +314,10 @@ void lora_tile_kernel(TileArgs args) {
             for (int q = 0; q < kEach; ++q) {
                 if (jb * kEach + q < kPieces) copy(s, jb * kEach + q);
             }
+            // In this order: left to itself the compiler gathers the 128x256
+            // tile's 32 MFMAs behind all the reads and copies (2000 x 4096 x
+            // 4096 r64 83.9 us, 80.3 like this).
+            if (kTN == 8 && jb < kTN - 1) __builtin_amdgcn_sched_barrier(0);
         }
     };
     auto final_step = [&](bf16x8_t (&cur)[kTM]) {
@@ -316,6 +330,17 @@ void lora_tile_kernel(TileArgs args) {
         }
     };
     int kt = 0;
+    // The adapter's K-steps of this slice (at most four), in a loop of their
+    // own: tested for in the loop below, the scale took config 0's 128
+    // accumulators out of the accumulation registers, and spilled.
+    const int lead = args.ext_steps > first ? args.ext_steps - first : 0;
+#pragma unroll 1
+    for (; kt < lead && kt + 1 < steps; ++kt) {
+        step(kt, x0, x1);
+#pragma unroll
+        for (int i = 0; i < kTM; ++i) x0[i] = x1[i];
+    }
+    if (lead > 0 && lead < steps) scale_adapter();
     for (; kt + 2 < steps; kt += 2) {
         step(kt, x0, x1);
         step(kt + 1, x1, x0);
@@ -326,6 +351,7 @@ void lora_tile_kernel(TileArgs args) {
     } else {
         final_step(x0);
     }
+    if (lead >= steps) scale_adapter();  // a slice within the adapter
 
     // acc[jb][i] lane: row m0 + 16 (kTM wm + i) + lane % 16, columns
     // n0 + 16 (kTN wn + jb) + 4 g .. +3; N is a multiple of 8, so those four
@@ -412,7 +438,7 @@ __global__ __launch_bounds__(kDefaultBlockSize) void lora_tile_sum_kernel(TileAr
 }
 
 // ---------------------------------------------------------------------------
-// x @ a and the parts of scale * b.
+// x @ a.
 // ---------------------------------------------------------------------------
 
 constexpr int kDownWaves = 8;
@@ -421,18 +447,12 @@ constexpr int kDownThreads = kDownWaves * 64;
 struct DownArgs {
     const uint16_t* x;  // [M, K]
     const uint16_t* a;  // [K, rank]
-    const uint16_t* b;  // [rank, N]
     uint16_t* u;        // [M, ext]
-    uint16_t* sb;       // [ext, N]
     float* xa_out;      // [M, rank] or null
     int64_t M;
-    int64_t N;
     int64_t K;
     int rank;
     int ext;
-    int parts;          // 1: s * b is exact in bf16; 2: high and low parts
-    float scale;
-    int row_blocks;     // workgroups of x @ a; the rest of the grid does s * b
     bool vector_a;      // rows of a are whole aligned 16-byte pieces
     bool pair_a;        // rows of a are whole aligned 4-byte pairs
 };
@@ -451,33 +471,6 @@ __global__ __launch_bounds__(kDownThreads) void lora_down_kernel(DownArgs args) 
     const int jl = lane & 15;
     const int rank = args.rank;
     const int ext = args.ext;
-
-    if (static_cast<int>(blockIdx.x) >= args.row_blocks) {
-        // Row j of part p of s * b goes to row p * rank + j, zeros behind.
-        const int64_t i =
-            (static_cast<int64_t>(blockIdx.x) - args.row_blocks) * kDownThreads + tid;
-        const int64_t chunks = args.N / 8;
-        const int64_t row = i / chunks;
-        if (row >= ext) return;
-        const int64_t col = (i - row * chunks) * 8;
-        uint32_t out[4] = {0, 0, 0, 0};
-        if (row < args.parts * rank) {
-            const bool low = row >= rank;
-            const uint4 v =
-                *reinterpret_cast<const uint4*>(args.b + (low ? row - rank : row) * args.N + col);
-            float f[8];
-            unpack16<bf16_t>(v, f);
-#pragma unroll
-            for (int e = 0; e < 8; ++e) {
-                const float s = args.scale * f[e];
-                uint32_t h = f32_to_bf16_bits(s);
-                if (low) h = f32_to_bf16_bits(s - bf16_bits_to_f32(static_cast<uint16_t>(h)));
-                out[e >> 1] |= h << (16 * (e & 1));
-            }
-        }
-        *reinterpret_cast<uint4*>(args.sb + row * args.N + col) = make_uint4(out[0], out[1], out[2], out[3]);
-        return;
-    }
 
     const int64_t m0 = static_cast<int64_t>(blockIdx.x) * 16;
     const int64_t rows_here = args.M - m0 < 16 ? args.M - m0 : 16;
@@ -583,17 +576,12 @@ __global__ __launch_bounds__(kDownThreads) void lora_down_kernel(DownArgs args) 
         for (int t = 0; t < 4; ++t) {
             if (j0 + t >= rank) continue;
             if (args.xa_out != nullptr) args.xa_out[(m0 + row) * rank + j0 + t] = v[t];
-            const uint32_t h = f32_to_bf16_bits(v[t]);
-            uint16_t* dst = args.u + (m0 + row) * ext + j0 + t;
-            dst[0] = static_cast<uint16_t>(h);
-            // An infinite x @ a meets only the high part of s * b: inf * lo
-            // would add NaN (lo = 0) or an infinity of the other sign.
-            if (args.parts == 2) dst[rank] = static_cast<uint16_t>((h & 0x7FFF) == 0x7F80 ? 0 : h);
+            args.u[(m0 + row) * ext + j0 + t] = static_cast<uint16_t>(f32_to_bf16_bits(v[t]));
         }
     }
-    const int pad = ext - args.parts * rank;
+    const int pad = ext - rank;
     for (int e = tid; e < static_cast<int>(rows_here) * pad; e += kDownThreads) {
-        args.u[(m0 + e / pad) * ext + args.parts * rank + e % pad] = 0;
+        args.u[(m0 + e / pad) * ext + rank + e % pad] = 0;
     }
 }
 
@@ -603,16 +591,7 @@ __global__ __launch_bounds__(kDownThreads) void lora_down_kernel(DownArgs args) 
 
 size_t align256(size_t bytes) { return (bytes + 255) / 256 * 256; }
 
-/// s * b is exact in bf16 for every bf16 b when s is 0 or +-2^k, k >= 0 (the
-/// exponent only moves up; an overflow gives the infinity the fp32 product
-/// has).
-bool exact_scale(float scale) {
-    int exponent = 0;
-    const float mantissa = std::frexp(std::fabs(scale), &exponent);
-    return scale == 0.0f || (mantissa == 0.5f && exponent >= 1);
-}
-
-int64_t ext_of(int64_t rank, int parts) { return ceil_div<int64_t>(parts * rank, kBK) * kBK; }
+int64_t ext_of(int64_t rank) { return ceil_div<int64_t>(rank, kBK) * kBK; }
 
 struct Config {
     int bm;
@@ -658,7 +637,7 @@ constexpr int kMinSliceSteps = 4;
 /// dozen candidates and 32-bit divisions: 0.3 us.)
 Plan best_plan(int64_t M, int64_t N, int64_t K, int64_t rank) {
     constexpr int kSlices[] = {1, 2, 3, 4, 5, 6, 8, 12, 16, 24, 32};
-    const int steps = static_cast<int>(ceil_div<int64_t>(K, kBK) + ext_of(rank, 2) / kBK);
+    const int steps = static_cast<int>(ceil_div<int64_t>(K, kBK) + ext_of(rank) / kBK);
     Plan best;
     best.us = INFINITY;
     for (int c = 0; c < 3; ++c) {
@@ -710,28 +689,26 @@ void launch_tile(const TileArgs& args, hipStream_t stream) {
            dim3(kWM * kWN * 64), 0, stream, args);
 }
 
-cf_status run_plan(const Plan& planned, const void* x, const void* w, const void* a, const void* b, void* y,
+cf_status run_plan(const Plan& plan, const void* x, const void* w, const void* a, const void* b, void* y,
                    float* xa_out, int64_t M, int64_t N, int64_t K, int64_t rank, float scale, void* workspace,
                    hipStream_t stream) {
-    const int parts = exact_scale(scale) ? 1 : 2;
-    const int64_t ext = rank > 0 ? ext_of(rank, parts) : 0;
+    const int64_t ext = ext_of(rank);
     uint8_t* p = static_cast<uint8_t*>(workspace);
     TileArgs args;
     args.x = static_cast<const uint16_t*>(x);
     args.w = static_cast<const uint16_t*>(w);
     args.u = reinterpret_cast<uint16_t*>(p);
-    p += align256(static_cast<size_t>(M * ext_of(rank, 2)) * 2);
-    args.sb = reinterpret_cast<uint16_t*>(p);
-    p += align256(static_cast<size_t>(ext_of(rank, 2) * N) * 2);
-    args.part = reinterpret_cast<float*>(p);
+    args.part = reinterpret_cast<float*>(p + align256(static_cast<size_t>(M * ext) * 2));
+    args.b = static_cast<const uint16_t*>(b);
     args.y = static_cast<uint16_t*>(y);
     args.M = M;
     args.N = N;
     args.K = K;
+    args.rank = rank;
     args.ext = ext;
-    args.main_steps = static_cast<int>(ceil_div<int64_t>(K, kBK));
-    args.steps = args.main_steps + static_cast<int>(ext / kBK);
-    const Plan plan = make_plan(planned.config, planned.whole, planned.slices, args.steps);
+    args.ext_steps = static_cast<int>(ext / kBK);
+    args.steps = static_cast<int>(ceil_div<int64_t>(K, kBK)) + args.ext_steps;
+    args.scale = scale;
     args.whole = plan.whole;
     args.slices = plan.slices;
     args.slice_steps = plan.slice_steps;
@@ -743,21 +720,15 @@ cf_status run_plan(const Plan& planned, const void* x, const void* w, const void
         DownArgs down;
         down.x = args.x;
         down.a = static_cast<const uint16_t*>(a);
-        down.b = static_cast<const uint16_t*>(b);
         down.u = const_cast<uint16_t*>(args.u);
-        down.sb = const_cast<uint16_t*>(args.sb);
         down.xa_out = xa_out;
         down.M = M;
-        down.N = N;
         down.K = K;
         down.rank = static_cast<int>(rank);
         down.ext = static_cast<int>(ext);
-        down.parts = parts;
-        down.scale = scale;
-        down.row_blocks = static_cast<int>(ceil_div<int64_t>(M, 16));
         down.vector_a = rank % 8 == 0 && host_aligned(a, 16);
         down.pair_a = rank % 2 == 0 && host_aligned(a, 4);
-        const dim3 grid(static_cast<unsigned>(down.row_blocks + ceil_div<int64_t>(ext * (N / 8), kDownThreads)));
+        const dim3 grid(static_cast<unsigned>(ceil_div<int64_t>(M, 16)));
         if (rank <= 16) {
             launch(lora_down_kernel<1>, grid, dim3(kDownThreads), 0, stream, down);
         } else if (rank <= 32) {
@@ -788,7 +759,7 @@ cf_status run_plan(const Plan& planned, const void* x, const void* w, const void
 
 bool lora_tile_shape(int64_t M, int64_t N, int64_t K, int64_t rank) {
     // Buffer offsets are 32-bit with an out-of-range marker at 2^31.
-    const int64_t ext = ext_of(rank, 2);
+    const int64_t ext = ext_of(rank);
     return M > 0 && N > 0 && K > 0 && N % 8 == 0 && K % 8 == 0 && rank >= 0 && rank <= kTileMaxRank &&
            (K + kBK) * N * 2 < (1LL << 31) && 256 * K * 2 < (1LL << 31) && ext * N * 2 < (1LL << 31) &&
            ceil_div<int64_t>(M, 64) * ceil_div<int64_t>(N, 128) < (1LL << 24);
@@ -808,8 +779,7 @@ size_t lora_tile_workspace_bytes(int64_t M, int64_t N, int64_t K, int64_t rank) 
     const Plan p = best_plan(M, N, K, rank);
     const Config& c = kConfigs[p.config];
     const int64_t tiles = ceil_div<int64_t>(M, c.bm) * ceil_div<int64_t>(N, c.bn);
-    return align256(static_cast<size_t>(M * ext_of(rank, 2)) * 2) +
-           align256(static_cast<size_t>(ext_of(rank, 2) * N) * 2) +
+    return align256(static_cast<size_t>(M * ext_of(rank)) * 2) +
            static_cast<size_t>((tiles - p.whole) * p.slices) * c.bm * c.bn * 4;
 }
 

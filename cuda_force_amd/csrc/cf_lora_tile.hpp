@@ -1,4 +1,4 @@
-// Internal interface of the tiled bf16 LoRA kernels with the adapter as extra
+// Internal interface of the tiled bf16 LoRA kernels with the adapter as leading
 // K-steps (cf_lora_tile.hip).
 #pragma once
 
@@ -21,7 +21,7 @@ bool lora_tile_shape(int64_t M, int64_t N, int64_t K, int64_t rank);
 /// these kernels and the 256x256-tile one of cf_lora_fused.hip.
 float lora_tile_estimate_us(int64_t M, int64_t N, int64_t K, int64_t rank);
 
-/// Bytes of workspace launch_lora_tile needs for any scale.
+/// Bytes of workspace launch_lora_tile needs.
 size_t lora_tile_workspace_bytes(int64_t M, int64_t N, int64_t K, int64_t rank);
 
 /// y = x @ w + scale * bf16(x @ a) @ b; writes the fp32 x @ a to xa_out when

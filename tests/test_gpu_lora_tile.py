@@ -2,8 +2,8 @@
 float64 oracle: each tile shape with part tiles in both directions, K not a
 multiple of the K-step, one K-step and fewer than the stages, ranks whose
 rows are 16-byte pieces, pairs and single elements, adapter parts that fill
-K-steps exactly and that do not (or lie in several slices), whole tiles, split
-tiles and both. The tolerance is that of the other bf16 LoRA tests (one bf16
+K-steps exactly and that do not, several slices, whole tiles, split tiles and
+both. The tolerance is that of the other bf16 LoRA tests (one bf16
 rounding 2^-9 relative, a floor for cancelling sums)."""
 
 from __future__ import annotations
@@ -57,8 +57,7 @@ def test_rank_zero_and_row_independence():
 @pytest.mark.parametrize("scale", [2.0, 1.7])
 def test_infinite_adapter_intermediate(scale):
     """x @ a overflows to infinity in one row: the row is +-inf by the sign of
-    b, as in fp32 arithmetic (the low part of a split scale * b must not add
-    NaN or an infinity of the other sign), and the other rows are zero."""
+    b, as in fp32 arithmetic, and the other rows are zero."""
     m, k, n, r = 100, 64, 136, 16
     x, w, a, b = (np.zeros_like(t) for t in make_operands(m, k, n, r, "bf16", seed=1))
     b = make_operands(m, k, n, r, "bf16", seed=2)[3]
@@ -69,3 +68,30 @@ def test_infinite_adapter_intermediate(scale):
     assert np.isposinf(xa[5, 0])
     np.testing.assert_array_equal(got[5], np.where(g.host_values(b, "bf16")[0] > 0, np.inf, -np.inf))
     assert (np.delete(got, 5, axis=0) == 0).all()
+
+
+@pytest.mark.parametrize("scale", [2.0, 0.25, 1.7])
+@pytest.mark.parametrize("shape", [(100, 64, 136, 24), (300, 4096, 264, 40), (2100, 520, 136, 7)], ids=str)
+def test_infinite_b_and_a_scaled_b_past_bf16(shape, scale):
+    """scale * (u @ b) in fp32: an infinite b gives +-inf by the sign of u, and a
+    b whose product with the scale is past the largest bf16 gives the finite
+    value it has with a small u."""
+    m, k, n, r = shape
+    g.announce(f"tiled LoRA with infinite and largest b {shape} scale {scale}")
+    x, w, a, b = make_operands(m, k, n, r, "bf16", seed=sum(shape))
+    w = np.zeros_like(w)
+    b[:, 3] = 0
+    b[r - 1, 3] = 0x7F80  # inf
+    b[:, 5] = 0
+    b[0, 5] = 0x7F7F      # 3.39e38, the largest bf16
+    x, a = x & 0x7FFF, a & 0x7FFF
+    x[::2] |= 0x8000      # rows of either sign
+    a = (0x3000 + (a & 0x7F)).astype(np.uint16)  # 2^-31 .. 2^-30: 2 u max(b) is finite
+    y, xa = run_forward(x, w, a, b, scale)
+    got = g.host_values(y, "bf16")
+    u = g.host_values(g.storage_bits(xa, "bf16"), "bf16").astype(np.float64)
+    assert (u != 0).all()
+    np.testing.assert_array_equal(got[:, 3], np.where(u[:, r - 1] > 0, np.inf, -np.inf))
+    np.testing.assert_allclose(got[:, 5], scale * u[:, 0] * g.host_values(b, "bf16")[0, 5], rtol=2.0**-8)
+    rest = [i for i in range(n) if i not in (3, 5)]
+    assert np.isfinite(got[:, rest]).all()
