@@ -186,3 +186,29 @@ def test_fused_bf16_lora_follows_the_reference_off_the_finite_range(shape):
     finite = np.isfinite(exact)
     err = np.abs(got[finite] - exact[finite])
     assert (err <= 1e-2 * np.abs(exact[finite]) + 1e-3 * arith[finite]).all()
+
+
+@pytest.mark.parametrize("scale", [2.0, 1.7, 0.25])
+@pytest.mark.parametrize("shape", [(256, 512, 256, 8), (300, 2048, 264, 16)], ids=str)
+def test_fused_bf16_lora_with_an_infinite_b(shape, scale):
+    """An infinite b gives +-inf down its column by the sign of x @ a, at a
+    scale whose product with b is split into two bf16 parts as at one whose
+    is not."""
+    m, k, n, r = shape
+    g.announce(f"bf16 fused LoRA with an infinite b {shape} scale {scale}")
+    gen = rng(sum(shape))
+    x = np.abs(gen.standard_normal((m, k))).astype(np.float32)
+    x[::2] *= -1
+    w = (0.02 * gen.standard_normal((k, n))).astype(np.float32)
+    a = np.abs(gen.standard_normal((k, r)) / 64).astype(np.float32)
+    b = (0.02 * gen.standard_normal((r, n))).astype(np.float32)
+    b[:, 3] = 0
+    b[r - 1, 3] = np.inf
+    xg, wg, ag, bg = (g.to_gpu(g.storage_bits(t, "bf16"), "bf16") for t in (x, w, a, b))
+    y = g.empty((m, n), torch.bfloat16)
+    g.call("cf_lora_linear", xg.data_ptr(), wg.data_ptr(), ag.data_ptr(), bg.data_ptr(), y.data_ptr(), None,
+           g.cf("bf16"), m, k, n, r, scale, g.stream())
+    torch.cuda.synchronize()
+    got = g.host_values(g.to_host(y), "bf16")
+    assert np.array_equal(got[:, 3], np.where(np.arange(m) % 2 == 0, -np.inf, np.inf))
+    assert np.isfinite(np.delete(got, 3, axis=1)).all()
