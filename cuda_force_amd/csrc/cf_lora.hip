@@ -303,10 +303,15 @@ __global__ __launch_bounds__(kDefaultBlockSize) void adapter_update_kernel(
 template <typename T>
 void launch_adapter_update(const float* g, const void* a, void* grad_x, int64_t rows, int64_t cols,
                            int64_t rank, float scale, hipStream_t stream) {
-    const dim3 grid(static_cast<unsigned>(ceil_div<int64_t>(cols, kDefaultBlockSize)),
-                    static_cast<unsigned>(ceil_div<int64_t>(rows, kUpdateRowsGeneric)));
-    launch(adapter_update_kernel<T>, grid, dim3(kDefaultBlockSize), 0, stream, g, static_cast<const T*>(a),
-           static_cast<T*>(grad_x), rows, cols, rank, scale);
+    // As many rows a launch as grid.y takes.
+    constexpr int64_t kRowsPerLaunch = kUpdateRowsGeneric * kMaxGridY;
+    for (int64_t row0 = 0; row0 < rows; row0 += kRowsPerLaunch) {
+        const int64_t count = rows - row0 < kRowsPerLaunch ? rows - row0 : kRowsPerLaunch;
+        const dim3 grid(static_cast<unsigned>(ceil_div<int64_t>(cols, kDefaultBlockSize)),
+                        static_cast<unsigned>(ceil_div<int64_t>(count, kUpdateRowsGeneric)));
+        launch(adapter_update_kernel<T>, grid, dim3(kDefaultBlockSize), 0, stream, g + row0 * rank,
+               static_cast<const T*>(a), static_cast<T*>(grad_x) + row0 * cols, count, cols, rank, scale);
+    }
 }
 
 template <typename T>

@@ -667,23 +667,28 @@ cf_status launch_lora_backward_fast(const void* x, const void* dy, const void* a
     : rank_pad == 32 ? finish_grad_a(finish_grad_a_kernel<32>)
                      : finish_grad_a(finish_grad_a_kernel<64>);
     if (grad_x != nullptr) {
-        UpdateArgs update;
-        update.g = ws.g;
-        update.a = static_cast<const uint16_t*>(a);
-        update.grad_x = static_cast<uint16_t*>(grad_x);
-        update.M = M;
-        update.K = K;
-        update.rank = static_cast<int>(rank);
-        update.scale = scale;
-        update.vector_a = rank % 8 == 0 && host_aligned(a, 16);
-        const dim3 grid(static_cast<unsigned>(ceil_div<int64_t>(K, kUpdateCols)),
-                        static_cast<unsigned>(ceil_div<int64_t>(M, update_rows(rank_pad / 16))));
-        if (rank_pad == 16) {
-            launch(lora_update_kernel<1>, grid, dim3(kThreads), 0, stream, update);
-        } else if (rank_pad == 32) {
-            launch(lora_update_kernel<2>, grid, dim3(kThreads), 0, stream, update);
-        } else {
-            launch(lora_update_kernel<4>, grid, dim3(kThreads), 0, stream, update);
+        // As many rows a launch as grid.y takes.
+        const int rows_each = update_rows(rank_pad / 16);
+        const int64_t rows_per_launch = rows_each * kMaxGridY;
+        for (int64_t row0 = 0; row0 < M; row0 += rows_per_launch) {
+            UpdateArgs update;
+            update.g = ws.g + row0 * rank_pad;
+            update.a = static_cast<const uint16_t*>(a);
+            update.grad_x = static_cast<uint16_t*>(grad_x) + row0 * K;
+            update.M = M - row0 < rows_per_launch ? M - row0 : rows_per_launch;
+            update.K = K;
+            update.rank = static_cast<int>(rank);
+            update.scale = scale;
+            update.vector_a = rank % 8 == 0 && host_aligned(a, 16);
+            const dim3 grid(static_cast<unsigned>(ceil_div<int64_t>(K, kUpdateCols)),
+                            static_cast<unsigned>(ceil_div<int64_t>(update.M, rows_each)));
+            if (rank_pad == 16) {
+                launch(lora_update_kernel<1>, grid, dim3(kThreads), 0, stream, update);
+            } else if (rank_pad == 32) {
+                launch(lora_update_kernel<2>, grid, dim3(kThreads), 0, stream, update);
+            } else {
+                launch(lora_update_kernel<4>, grid, dim3(kThreads), 0, stream, update);
+            }
         }
     }
     return check_launch("launching the bf16 LoRA backward", stream);

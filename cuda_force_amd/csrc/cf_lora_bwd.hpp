@@ -8,6 +8,9 @@
 
 namespace cf {
 
+/// Workgroups in y of one launch, at most (the device reports 65536).
+inline constexpr int64_t kMaxGridY = 65535;
+
 /// total += at(t) for t = t .. tiles - 1 in that order, loads issued in
 /// groups of 32, 16, 4, then 1 so a thread waits for memory a few times
 /// rather than once per eight partials.

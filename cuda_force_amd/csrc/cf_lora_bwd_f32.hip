@@ -241,7 +241,7 @@ void launch_pass(const PassArgs& args, hipStream_t stream) {
 bool lora_backward_f32_eligible(const void* x, const void* dy, const void* b, int64_t M, int64_t K,
                                 int64_t N, int64_t rank) {
     return M > 0 && K > 0 && N > 0 && rank > 0 && rank <= kMaxRank && K % 4 == 0 && N % 4 == 0 &&
-           ceil_div<int64_t>(M, 32) <= 65535 && host_aligned(x, 16) && host_aligned(dy, 16) &&
+           ceil_div<int64_t>(M, 32) <= kMaxGridY && host_aligned(x, 16) && host_aligned(dy, 16) &&
            host_aligned(b, 16);
 }
 

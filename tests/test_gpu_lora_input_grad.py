@@ -2,7 +2,8 @@
 plus the adapter's part added in place by the HIP kernels) against float64:
 every rank block count, ranks with and without whole 16-byte rows of a, row
 and column remainders, the generic path (fp32, odd widths, rank above 64),
-infinite gradients, and the composed path a recorded backward takes."""
+infinite gradients, more rows than one launch takes, and the composed path a
+recorded backward takes."""
 
 from __future__ import annotations
 
@@ -73,6 +74,23 @@ def test_infinite_gradients_stay_infinite(dtype, rank):
             rest = [i for i in range(70) if i not in (3, 64)]
             assert torch.equal(grad_x[rest], plain[rest])
         plain = grad_x
+
+
+@pytest.mark.parametrize("dtype,rows,n", [(torch.float32, 524_289, 8), (torch.float32, 524_289, 6),
+                                          (torch.bfloat16, 1_048_577, 8), (torch.bfloat16, 524_289, 6)])
+def test_more_rows_than_one_launch_of_the_update_takes(dtype, rows, n):
+    """16 or 8 rows a workgroup and 65535 workgroups in y: one row more than
+    that, on each kernel (widths that are not whole vectors take the plain
+    one)."""
+    g.announce(f"LoRA input gradient {dtype} {rows} rows, {n} columns")
+    x, w, a, b, dy = _operands(rows, 8, n, 2, dtype, rows)
+    leaves = [t.clone().requires_grad_() for t in (x, a, b)]
+    grads = torch.autograd.grad(ops.lora_linear(leaves[0], w, leaves[1], leaves[2], 1.5), leaves, dy)
+    for at in (slice(0, 64), slice(rows - 64, rows)):
+        want = dy[at].double() @ (w.double() + 1.5 * (a.double() @ b.double())).t()
+        rel, floor = (1e-2, 4e-3) if dtype == torch.bfloat16 else (1e-4, 2e-5)
+        err = (grads[0][at].double() - want).abs()
+        assert bool((err <= rel * want.abs() + floor * want.abs().max()).all())
 
 
 def test_a_recorded_backward_can_be_differentiated_again():
