@@ -95,6 +95,7 @@ SIGNATURES: dict[str, tuple[object, list[object]]] = {
     ),
     "cf_matmul": (_I32, [_P, _P, _P, _I32, _I64, _I64, _I64, _P]),
     "cf_lora_backward_workspace_bytes": (_SZ, [_I64, _I64, _I64, _I64]),
+    "cf_lora_backward_dtype_workspace_bytes": (_SZ, [_I32, _I64, _I64, _I64, _I64]),
     "cf_lora_backward": (
         _I32,
         [_P, _P, _P, _P, _P, _P, _I32, _I64, _I64, _I64, _I64, _F, _P, _SZ, _P],

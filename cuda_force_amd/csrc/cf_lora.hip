@@ -544,19 +544,28 @@ cf_status cf_matmul(const void* a, const void* b, void* c, cf_dtype dtype, int64
     return cf::launch_generic<cf::bf16_t>(a, b, nullptr, nullptr, c, nullptr, m, n, k, 0, 0.0f, s);
 }
 
-size_t cf_lora_backward_workspace_bytes(int64_t batch, int64_t in_features, int64_t out_features,
-                                        int64_t rank) {
+size_t cf_lora_backward_dtype_workspace_bytes(cf_dtype dtype, int64_t batch, int64_t in_features,
+                                              int64_t out_features, int64_t rank) {
     if (batch <= 0 || rank <= 0) return 0;
     const int64_t chunks = cf::ceil_div<int64_t>(batch, cf::kColRowsPerChunk);
     const int64_t widest = in_features > out_features ? in_features : out_features;
     const size_t g = static_cast<size_t>(batch * rank) * sizeof(float);
     const size_t part = static_cast<size_t>(chunks * rank * widest) * sizeof(float);
     const size_t generic = ((g + 255) / 256) * 256 + part;
-    // Enough for either path: which one runs depends on dtype and alignment.
-    const size_t fast = cf::lora_backward_fast_workspace_bytes(batch, in_features, out_features, rank);
-    const size_t f32 = cf::lora_backward_f32_workspace_bytes(batch, in_features, out_features, rank);
-    const size_t mfma = fast > f32 ? fast : f32;
+    // Enough for either path of the dtype: which one runs depends on alignment.
+    const size_t mfma =
+        dtype == CF_F32 ? cf::lora_backward_f32_workspace_bytes(batch, in_features, out_features, rank)
+                        : cf::lora_backward_fast_workspace_bytes(batch, in_features, out_features, rank);
     return generic > mfma ? generic : mfma;
+}
+
+size_t cf_lora_backward_workspace_bytes(int64_t batch, int64_t in_features, int64_t out_features,
+                                        int64_t rank) {
+    const size_t f32 =
+        cf_lora_backward_dtype_workspace_bytes(CF_F32, batch, in_features, out_features, rank);
+    const size_t bf16 =
+        cf_lora_backward_dtype_workspace_bytes(CF_BF16, batch, in_features, out_features, rank);
+    return f32 > bf16 ? f32 : bf16;
 }
 
 cf_status cf_lora_backward(const void* x, const void* dy, const void* b, const float* xa,
@@ -592,7 +601,8 @@ cf_status cf_lora_backward_input(const void* x, const void* dy, const void* a, c
     CF_REQUIRE(x != nullptr && dy != nullptr && b != nullptr && xa != nullptr,
                "cf_lora_backward: null input");
     CF_REQUIRE(grad_x == nullptr || a != nullptr, "cf_lora_backward_input: null adapter");
-    const size_t needed = cf_lora_backward_workspace_bytes(batch, in_features, out_features, rank);
+    const size_t needed =
+        cf_lora_backward_dtype_workspace_bytes(dtype, batch, in_features, out_features, rank);
     CF_REQUIRE(workspace != nullptr && workspace_bytes >= needed,
                "cf_lora_backward: workspace of %zu bytes given, %zu needed", workspace_bytes,
                needed);

@@ -588,8 +588,16 @@ void launch_pass(const ColumnArgs& args, int rank_pad, int chunks, hipStream_t s
 
 }  // namespace
 
+bool lora_backward_fast_shape(int64_t M, int64_t K, int64_t N, int64_t rank) {
+    // Buffer offsets are 32-bit with an out-of-range marker at 2^31.
+    const int64_t Mp = padded_rows(M);
+    return M > 0 && K > 0 && N > 0 && rank > 0 && rank <= kMaxRank && K % 8 == 0 && N % 8 == 0 &&
+           Mp * K * 2 < (1LL << 31) && Mp * N * 2 < (1LL << 31) && rank * N * 2 < (1LL << 31) &&
+           kMaxRank * Mp * 2 < (1LL << 31) && Mp * rank * 4 < (1LL << 31);
+}
+
 size_t lora_backward_fast_workspace_bytes(int64_t M, int64_t K, int64_t N, int64_t rank) {
-    if (M <= 0 || rank > kMaxRank) return 0;
+    if (!lora_backward_fast_shape(M, K, N, rank)) return 0;
     const int64_t Mp = padded_rows(M);
     const int rank_pad = rank_pad_of(rank);
     const size_t dy = colpart_bytes(M, N, rank_pad);
@@ -601,14 +609,8 @@ size_t lora_backward_fast_workspace_bytes(int64_t M, int64_t K, int64_t N, int64
 
 bool lora_backward_fast_eligible(const void* x, const void* dy, const void* b, const void* grad_x,
                                  int64_t M, int64_t K, int64_t N, int64_t rank) {
-    // Buffer offsets are 32-bit with an out-of-range marker at 2^31.
-    const int64_t Mp = padded_rows(M);
-    const bool fits = Mp * K * 2 < (1LL << 31) && Mp * N * 2 < (1LL << 31) &&
-                      rank * N * 2 < (1LL << 31) && kMaxRank * Mp * 2 < (1LL << 31) &&
-                      Mp * rank * 4 < (1LL << 31);
-    return M > 0 && K > 0 && N > 0 && rank > 0 && rank <= kMaxRank && K % 8 == 0 && N % 8 == 0 &&
-           fits && host_aligned(x, 16) && host_aligned(dy, 16) && host_aligned(b, 16) &&
-           host_aligned(grad_x, 16);
+    return lora_backward_fast_shape(M, K, N, rank) && host_aligned(x, 16) && host_aligned(dy, 16) &&
+           host_aligned(b, 16) && host_aligned(grad_x, 16);
 }
 
 cf_status launch_lora_backward_fast(const void* x, const void* dy, const void* a, const void* b,

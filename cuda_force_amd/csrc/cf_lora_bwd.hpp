@@ -40,7 +40,11 @@ __device__ __forceinline__ float ordered_sum(int64_t tiles, At at) {
 bool lora_backward_fast_eligible(const void* x, const void* dy, const void* b, const void* grad_x,
                                  int64_t M, int64_t K, int64_t N, int64_t rank);
 
-/// Workspace bytes of launch_lora_backward_fast (256-byte aligned pieces).
+/// The same on sizes alone.
+bool lora_backward_fast_shape(int64_t M, int64_t K, int64_t N, int64_t rank);
+
+/// Workspace bytes of launch_lora_backward_fast (256-byte aligned pieces); 0
+/// for sizes it does not take.
 size_t lora_backward_fast_workspace_bytes(int64_t M, int64_t K, int64_t N, int64_t rank);
 
 /// grad_a = scale * x^T bf16(dy b^T), grad_b = scale * bf16(xa)^T dy (bf16
@@ -56,7 +60,10 @@ cf_status launch_lora_backward_fast(const void* x, const void* dy, const void* a
 bool lora_backward_f32_eligible(const void* x, const void* dy, const void* b, int64_t M, int64_t K,
                                 int64_t N, int64_t rank);
 
-/// Workspace bytes of launch_lora_backward_f32.
+/// The same on sizes alone.
+bool lora_backward_f32_shape(int64_t M, int64_t K, int64_t N, int64_t rank);
+
+/// Workspace bytes of launch_lora_backward_f32; 0 for sizes it does not take.
 size_t lora_backward_f32_workspace_bytes(int64_t M, int64_t K, int64_t N, int64_t rank);
 
 /// grad_a = scale * x^T (dy b^T), grad_b = scale * xa^T dy in fp32; dy b^T is

@@ -238,15 +238,19 @@ void launch_pass(const PassArgs& args, hipStream_t stream) {
 
 }  // namespace
 
+bool lora_backward_f32_shape(int64_t M, int64_t K, int64_t N, int64_t rank) {
+    return M > 0 && K > 0 && N > 0 && rank > 0 && rank <= kMaxRank && K % 4 == 0 && N % 4 == 0 &&
+           ceil_div<int64_t>(M, 32) <= kMaxGridY;
+}
+
 bool lora_backward_f32_eligible(const void* x, const void* dy, const void* b, int64_t M, int64_t K,
                                 int64_t N, int64_t rank) {
-    return M > 0 && K > 0 && N > 0 && rank > 0 && rank <= kMaxRank && K % 4 == 0 && N % 4 == 0 &&
-           ceil_div<int64_t>(M, 32) <= kMaxGridY && host_aligned(x, 16) && host_aligned(dy, 16) &&
+    return lora_backward_f32_shape(M, K, N, rank) && host_aligned(x, 16) && host_aligned(dy, 16) &&
            host_aligned(b, 16);
 }
 
 size_t lora_backward_f32_workspace_bytes(int64_t M, int64_t K, int64_t N, int64_t rank) {
-    if (M <= 0 || rank > kMaxRank) return 0;
+    if (!lora_backward_f32_shape(M, K, N, rank)) return 0;
     const int64_t widest = K > N ? K : N;
     return align256(static_cast<size_t>(M * rank) * 4) +
            align256(static_cast<size_t>(ceil_div<int64_t>(N, kHalfCols) * M * rank) * 4) +

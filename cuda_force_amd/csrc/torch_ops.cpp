@@ -280,7 +280,8 @@ std::tuple<torch::Tensor, torch::Tensor, torch::Tensor> lora_backward_hip(
     }
     torch::Tensor grad_a = torch::empty({in_features, rank}, x.options());
     torch::Tensor grad_b = torch::empty({rank, out_features}, x.options());
-    const size_t bytes = cf_lora_backward_workspace_bytes(batch, in_features, out_features, rank);
+    const size_t bytes =
+        cf_lora_backward_dtype_workspace_bytes(to_cf(x, "x"), batch, in_features, out_features, rank);
     torch::Tensor workspace =
         torch::empty({static_cast<int64_t>(bytes > 0 ? bytes : 1)}, x.options().dtype(torch::kUInt8));
     check_status(cf_lora_backward_input(

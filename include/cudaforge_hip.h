@@ -319,6 +319,12 @@ cf_status cf_matmul(const void* a, const void* b, void* c, cf_dtype dtype, int64
 size_t cf_lora_backward_workspace_bytes(int64_t batch, int64_t in_features, int64_t out_features,
                                         int64_t rank);
 
+/* The bytes of one dtype (CF_F32 or CF_BF16), which is all cf_lora_backward
+ * and cf_lora_backward_input ask for; the function above returns the larger of
+ * the two. It has no counterpart in the reference. */
+size_t cf_lora_backward_dtype_workspace_bytes(cf_dtype dtype, int64_t batch, int64_t in_features,
+                                              int64_t out_features, int64_t rank);
+
 /* Adapter gradients of y = x @ w + scale * (x @ a) @ b, op layout:
  *   grad_a [in, rank]  = scale * x^T (dy @ b^T)
  *   grad_b [rank, out] = scale * (x @ a)^T dy

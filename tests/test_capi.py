@@ -75,6 +75,17 @@ def test_few_row_lora_stops_where_a_buffer_reaches_2_gib(lib, m, k, n, rank, few
         assert needed < partials
 
 
+@pytest.mark.parametrize("m,k,n,rank,most", [
+    (8192, 4096, 4096, 16, 13.2e6), (65536, 4096, 11008, 16, 274.8e6),
+    (4096, 4096, 4096, 16, 8.7e6), (2001, 1001, 1003, 300, 12.1e6),
+])
+def test_bf16_backward_does_not_reserve_for_the_fp32_kernels(lib, m, k, n, rank, most):
+    bf16 = lib.cf_lora_backward_dtype_workspace_bytes(_lib.CF_BF16, m, k, n, rank)
+    f32 = lib.cf_lora_backward_dtype_workspace_bytes(_lib.CF_F32, m, k, n, rank)
+    assert 0 < bf16 <= most
+    assert lib.cf_lora_backward_workspace_bytes(m, k, n, rank) == max(bf16, f32)
+
+
 def test_empty_inputs_return_ok_without_touching_the_device(lib):
     null = ctypes.c_void_p(0)
     assert lib.cf_quantize_int8(null, _lib.CF_F32, null, null, 0, null) == _lib.CF_OK
