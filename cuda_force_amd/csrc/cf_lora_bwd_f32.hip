@@ -12,17 +12,17 @@
 // a few MB of operands. One wave per row of G and 256-row chunks left 128
 // waves and 64 workgroups on the GPU (G 225 us, each column reduction 42 us),
 // so the work is cut small instead: 128 columns x 32 rows per workgroup (128
-// rows from 512 rows on, where that fills the GPU and partials cost more),
-// straight from memory into MFMA operands (a tile is 16 KiB and its second use
-// comes from cache), partial sums in the workspace, summed in a fixed order by
-// a launch each:
-//   1. the dy pass: G partials per 64 columns, grad_b partials per half tile of
+// or 256 rows of long problems, which still fill the GPU and leave fewer
+// partials), straight from memory into MFMA operands (a tile of 32
+// rows is 16 KiB and its second use comes from cache), partial sums in the
+// workspace, summed in a fixed order by a launch each:
+//   1. the dy pass: G partials per 64 columns, grad_b partials per tile of
 //      rows;
 //   2. their sums;
 //   3. the x pass with G: grad_a partials;
 //   4. their sum, stored transposed.
-// Measured, whole entry: 128 x 4096 x 4096 r16 178.6 -> 15.3 us, 1024 x 4096 x
-// 4096 r64 1544 -> 52, 8192 x 4096 x 4096 r16 1032 -> 117.
+// Measured, whole entry: 128 x 4096 x 4096 r16 178.6 -> 15.2 us, 1024 x 4096 x
+// 4096 r64 1544 -> 48, 8192 x 4096 x 4096 r16 1032 -> 91.
 // Operand layouts: an MFMA takes one k value per 16 lanes. For G a lane loads
 // four consecutive columns of its row of dy (and b) and each of four MFMAs
 // takes one of them; for the column reductions a lane loads four consecutive
@@ -43,7 +43,7 @@ struct PassArgs {
     const float* v;     // [M, C], the operand reduced over rows
     const float* p;     // [M, rank], the other factor
     const float* b;     // [rank, C] (dy pass)
-    float* colpart;     // [2 row tiles][rank][C]
+    float* colpart;     // [row tiles][rank][C]
     float* gpart;       // [ceil(C / 64)][M][rank] (dy pass)
     int64_t M;
     int64_t C;
@@ -114,7 +114,8 @@ __global__ __launch_bounds__(kThreads) void column_f32_kernel(PassArgs args) {
         }
     }
 
-    // The column reduction over half the tile's rows: A = p (row j, k = m),
+    // The column reduction, two waves taking half the tile's rows each: A = p
+    // (row j, k = m),
     // B = v (k = m, column n); MFMA e of the four takes column e of a lane's
     // four.
     const int half = wave >> 1;
@@ -152,11 +153,23 @@ __global__ __launch_bounds__(kThreads) void column_f32_kernel(PassArgs args) {
             }
         }
     }
-    // acc[rb][e] lane: [16 rb + 4 g + t][n + e].
-    if (n < C) {
-        float* dst = args.colpart + (2 * static_cast<int64_t>(blockIdx.y) + half) * rank * C + n;
+    // acc[rb][e] lane: [16 rb + 4 g + t][n + e]. The second half's sums reach
+    // the first half's waves through LDS.
+    __shared__ __attribute__((aligned(16))) f32x4_t sums[2][kRB][4][64];
+    if (half == 1) {
 #pragma unroll
         for (int rb = 0; rb < kRB; ++rb) {
+#pragma unroll
+            for (int e = 0; e < 4; ++e) sums[wave & 1][rb][e][lane] = acc[rb][e];
+        }
+    }
+    __syncthreads();
+    if (half == 0 && n < C) {
+        float* dst = args.colpart + static_cast<int64_t>(blockIdx.y) * rank * C + n;
+#pragma unroll
+        for (int rb = 0; rb < kRB; ++rb) {
+#pragma unroll
+            for (int e = 0; e < 4; ++e) acc[rb][e] += sums[wave][rb][e][lane];
 #pragma unroll
             for (int t = 0; t < 4; ++t) {
                 const int64_t j = 16 * rb + 4 * g + t;
@@ -209,16 +222,34 @@ __global__ __launch_bounds__(kThreads) void finish_grad_a_f32_kernel(const float
 
 size_t align256(size_t bytes) { return (bytes + 255) / 256 * 256; }
 
-int64_t rows_for(int64_t M) { return M >= 512 ? 128 : 32; }
+/// Rows of a tile, in both passes: 256 where the narrower one still has a
+/// workgroup per CU (4096 x 4096 x 4096 r16 58.7 -> 51.2 us, 8192 x 4096 x 4096
+/// r64 328 -> 280; 6000 x 512 x 512 r16, 96 workgroups, 28.0 -> 30.6).
+int64_t rows_for(int64_t M, int64_t K, int64_t N) {
+    const int64_t columns = ceil_div<int64_t>(K < N ? K : N, kTileCols);
+    if (M >= 4096 && ceil_div<int64_t>(M, 256) * columns >= 256) return 256;
+    return M >= 512 ? 128 : 32;
+}
 
-int64_t row_parts(int64_t M) { return 2 * ceil_div<int64_t>(M, rows_for(M)); }
+int64_t row_parts(int64_t M, int64_t K, int64_t N) { return ceil_div<int64_t>(M, rows_for(M, K, N)); }
 
+/// Rows whose G partials are held at a time, whole tiles of every size: all of
+/// them while those take 256 MiB (one partial per 64 columns is r / 64 of dy),
+/// more in turn.
+int64_t panel_rows(int64_t M, int64_t N, int64_t rank) {
+    constexpr int64_t kLimit = 256LL << 20;
+    const int64_t fit = kLimit / (ceil_div<int64_t>(N, kHalfCols) * rank * 4) / 256 * 256;
+    return M <= fit ? M : fit > 256 ? fit : 256;
+}
+
+/// `rows`: of a tile, as rows_for the whole problem.
 template <bool kRowDot, int kRB>
-void launch_pass(const PassArgs& args, hipStream_t stream) {
-    const int64_t rows = rows_for(args.M);
+void launch_pass(const PassArgs& args, int64_t rows, hipStream_t stream) {
     const dim3 grid(static_cast<unsigned>(ceil_div<int64_t>(args.C, kTileCols)),
                     static_cast<unsigned>(ceil_div<int64_t>(args.M, rows)));
-    if (rows == 128) {
+    if (rows == 256) {
+        launch(column_f32_kernel<kRowDot, kRB, 256>, grid, dim3(kThreads), 0, stream, args);
+    } else if (rows == 128) {
         launch(column_f32_kernel<kRowDot, kRB, 128>, grid, dim3(kThreads), 0, stream, args);
     } else {
         launch(column_f32_kernel<kRowDot, kRB, 32>, grid, dim3(kThreads), 0, stream, args);
@@ -226,13 +257,13 @@ void launch_pass(const PassArgs& args, hipStream_t stream) {
 }
 
 template <bool kRowDot>
-void launch_pass(const PassArgs& args, hipStream_t stream) {
+void launch_pass(const PassArgs& args, int64_t rows, hipStream_t stream) {
     if (args.rank <= 16) {
-        launch_pass<kRowDot, 1>(args, stream);
+        launch_pass<kRowDot, 1>(args, rows, stream);
     } else if (args.rank <= 32) {
-        launch_pass<kRowDot, 2>(args, stream);
+        launch_pass<kRowDot, 2>(args, rows, stream);
     } else {
-        launch_pass<kRowDot, 4>(args, stream);
+        launch_pass<kRowDot, 4>(args, rows, stream);
     }
 }
 
@@ -253,8 +284,8 @@ size_t lora_backward_f32_workspace_bytes(int64_t M, int64_t K, int64_t N, int64_
     if (!lora_backward_f32_shape(M, K, N, rank)) return 0;
     const int64_t widest = K > N ? K : N;
     return align256(static_cast<size_t>(M * rank) * 4) +
-           align256(static_cast<size_t>(ceil_div<int64_t>(N, kHalfCols) * M * rank) * 4) +
-           static_cast<size_t>(row_parts(M) * rank * widest) * 4;
+           align256(static_cast<size_t>(ceil_div<int64_t>(N, kHalfCols) * panel_rows(M, N, rank) * rank) * 4) +
+           static_cast<size_t>(row_parts(M, K, N) * rank * widest) * 4;
 }
 
 cf_status launch_lora_backward_f32(const float* x, const float* dy, const float* b, const float* xa,
@@ -264,18 +295,26 @@ cf_status launch_lora_backward_f32(const float* x, const float* dy, const float*
     float* g = reinterpret_cast<float*>(ws);
     ws += align256(static_cast<size_t>(M * rank) * 4);
     float* gpart = reinterpret_cast<float*>(ws);
-    ws += align256(static_cast<size_t>(ceil_div<int64_t>(N, kHalfCols) * M * rank) * 4);
+    const int64_t panel = panel_rows(M, N, rank);
+    ws += align256(static_cast<size_t>(ceil_div<int64_t>(N, kHalfCols) * panel * rank) * 4);
     float* colpart = reinterpret_cast<float*>(ws);
 
-    launch_pass<true>(PassArgs{dy, xa, b, colpart, gpart, M, N, static_cast<int>(rank)}, stream);
-    const int64_t grad_b_blocks = ceil_div<int64_t>(rank * N, kThreads);
-    const int64_t g_blocks = ceil_div<int64_t>(M * rank, kThreads);
-    launch(after_dy_f32_kernel, dim3(static_cast<unsigned>(grad_b_blocks + g_blocks)), dim3(kThreads), 0,
-           stream, colpart, grad_b, gpart, g, grad_b_blocks, row_parts(M),
-           ceil_div<int64_t>(N, kHalfCols), M, N, rank, scale);
-    launch_pass<false>(PassArgs{x, g, nullptr, colpart, nullptr, M, K, static_cast<int>(rank)}, stream);
+    const int64_t rows = rows_for(M, K, N);
+    for (int64_t m0 = 0; m0 < M; m0 += panel) {
+        const int64_t count = M - m0 < panel ? M - m0 : panel;
+        launch_pass<true>(PassArgs{dy + m0 * N, xa + m0 * rank, b, colpart + m0 / rows * rank * N, gpart, count, N,
+                                   static_cast<int>(rank)},
+                          rows, stream);
+        // G of these rows, and with the last of them grad_b.
+        const int64_t grad_b_blocks = m0 + count == M ? ceil_div<int64_t>(rank * N, kThreads) : 0;
+        const int64_t g_blocks = ceil_div<int64_t>(count * rank, kThreads);
+        launch(after_dy_f32_kernel, dim3(static_cast<unsigned>(grad_b_blocks + g_blocks)), dim3(kThreads), 0,
+               stream, colpart, grad_b, gpart, g + m0 * rank, grad_b_blocks, row_parts(M, K, N),
+               ceil_div<int64_t>(N, kHalfCols), count, N, rank, scale);
+    }
+    launch_pass<false>(PassArgs{x, g, nullptr, colpart, nullptr, M, K, static_cast<int>(rank)}, rows, stream);
     launch(finish_grad_a_f32_kernel, dim3(static_cast<unsigned>(ceil_div<int64_t>(rank * K, kThreads))),
-           dim3(kThreads), 0, stream, colpart, grad_a, row_parts(M), rank, K, scale);
+           dim3(kThreads), 0, stream, colpart, grad_a, row_parts(M, K, N), rank, K, scale);
     return check_launch("launching the fp32 LoRA backward", stream);
 }
 

@@ -86,6 +86,15 @@ def test_bf16_backward_does_not_reserve_for_the_fp32_kernels(lib, m, k, n, rank,
     assert lib.cf_lora_backward_workspace_bytes(m, k, n, rank) == max(bf16, f32)
 
 
+@pytest.mark.parametrize("m,k,n,rank,most", [
+    (8192, 4096, 4096, 16, 42.5e6), (65536, 4096, 11008, 16, 452.5e6), (65536, 4096, 11008, 64, 998e6),
+])
+def test_fp32_backward_partials_are_bounded(lib, m, k, n, rank, most):
+    """256 MiB of dy @ b^T partials, and one partial per 256 rows of the
+    adapter gradients."""
+    assert 0 < lib.cf_lora_backward_dtype_workspace_bytes(_lib.CF_F32, m, k, n, rank) <= most
+
+
 def test_empty_inputs_return_ok_without_touching_the_device(lib):
     null = ctypes.c_void_p(0)
     assert lib.cf_quantize_int8(null, _lib.CF_F32, null, null, 0, null) == _lib.CF_OK
