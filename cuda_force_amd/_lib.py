@@ -104,6 +104,7 @@ SIGNATURES: dict[str, tuple[object, list[object]]] = {
         _I32,
         [_P, _P, _P, _P, _P, _P, _P, _P, _I32, _I64, _I64, _I64, _I64, _F, _P, _SZ, _P],
     ),
+    "cf_lora_backward_updates_input": (_I32, [_I32, _I64, _I64, _I64, _I64]),
     "cf_silu": (_I32, [_P, _P, _I32, _I64, _P]),
     "cf_gelu": (_I32, [_P, _P, _I32, _I64, _P]),
     "cf_swiglu": (_I32, [_P, _P, _P, _I32, _I64, _P]),

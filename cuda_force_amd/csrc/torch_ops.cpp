@@ -231,8 +231,11 @@ torch::Tensor lora_linear_hip(const torch::Tensor& x, const torch::Tensor& w,
     return std::get<0>(lora_linear_fwd_hip(x, w, a, b, scale));
 }
 
+bool aligned16(const at::Tensor& t) { return reinterpret_cast<uintptr_t>(t.data_ptr()) % 16 == 0; }
+
 // Adapter gradients; with w and a also the input gradient: the plain GEMM
-// dy @ w^T through the vendor BLAS, the adapter's part added in place.
+// dy @ w^T through the vendor BLAS, the adapter's part added in place (by the
+// BLAS too where the library says that is the faster way).
 std::tuple<torch::Tensor, torch::Tensor, torch::Tensor> lora_backward_hip(
     const torch::Tensor& x, const torch::Tensor& dy, const torch::Tensor* w, const torch::Tensor* a,
     const torch::Tensor& b, const torch::Tensor& xa, double scale) {
@@ -269,6 +272,7 @@ std::tuple<torch::Tensor, torch::Tensor, torch::Tensor> lora_backward_hip(
     }
     const at::DeviceGuard guard(x.device());
     torch::Tensor grad_x;
+    bool own_update = false;
     if (w != nullptr) {
         // A backward inside an autocast block runs here with its keys on: mm
         // would then return another dtype than the kernel below is told.
@@ -277,6 +281,13 @@ std::tuple<torch::Tensor, torch::Tensor, torch::Tensor> lora_backward_hip(
         TORCH_CHECK(grad_x.scalar_type() == x.scalar_type() && grad_x.is_contiguous() &&
                         grad_x.sizes() == x.sizes(),
                     "dy @ w^T is not a contiguous ", x.scalar_type(), " tensor of x's shape");
+        own_update = aligned16(x) && aligned16(dy) && aligned16(b) &&
+                     cf_lora_backward_updates_input(to_cf(x, "x"), batch, in_features, out_features, rank) != 0;
+        if (!own_update) {
+            const torch::Tensor g = at::mm(dy, b.t());
+            // A GEMM with alpha = 0 reads nothing, and 0 * inf is NaN.
+            scale != 0.0 ? grad_x.addmm_(g, a->t(), 1, scale) : grad_x.add_(at::mm(g, a->t()), scale);
+        }
     }
     torch::Tensor grad_a = torch::empty({in_features, rank}, x.options());
     torch::Tensor grad_b = torch::empty({rank, out_features}, x.options());
@@ -287,7 +298,7 @@ std::tuple<torch::Tensor, torch::Tensor, torch::Tensor> lora_backward_hip(
     check_status(cf_lora_backward_input(
         x.data_ptr(), dy.data_ptr(), a != nullptr ? a->data_ptr() : nullptr, b.data_ptr(),
         xa.data_ptr<float>(), grad_a.data_ptr(), grad_b.data_ptr(),
-        w != nullptr ? grad_x.data_ptr() : nullptr, to_cf(x, "x"), batch, in_features, out_features, rank,
+        own_update ? grad_x.data_ptr() : nullptr, to_cf(x, "x"), batch, in_features, out_features, rank,
         static_cast<float>(scale), workspace.data_ptr(), bytes, stream_for(x)));
     return {grad_x, grad_a, grad_b};
 }
@@ -827,8 +838,6 @@ bool attention_rows(const at::Tensor& t, int64_t heads) {
     const int64_t d = t.size(2) / heads;
     return (d == 32 || d == 64 || d == 96 || d == 128) && t.size(1) % 8 == 0;
 }
-
-bool aligned16(const at::Tensor& t) { return reinterpret_cast<uintptr_t>(t.data_ptr()) % 16 == 0; }
 
 py::object try_attention_scores(py::handle q_, py::handle k_, py::handle heads_) {
     const at::Tensor* q = ordinary(q_);

@@ -353,6 +353,14 @@ cf_status cf_lora_backward_input(const void* x, const void* dy, const void* a, c
                                  int64_t out_features, int64_t rank, float scale, void* workspace,
                                  size_t workspace_bytes, void* stream);
 
+/* 1 where cf_lora_backward_input's own update of grad_x is the faster way for
+ * these sizes and 16-byte aligned operands, 0 where a caller with a GEMM library
+ * does better to give NULL and add scale * (dy @ b^T) @ a^T itself (large
+ * problems that the matrix-core update does not take). Either way the result is
+ * right. It has no counterpart in the reference. */
+int cf_lora_backward_updates_input(cf_dtype dtype, int64_t batch, int64_t in_features,
+                                   int64_t out_features, int64_t rank);
+
 /* ---- elementwise activations ------------------------------------------- */
 
 /* silu(x) = x * sigmoid(x), fp32 arithmetic for every dtype.

@@ -95,6 +95,19 @@ def test_fp32_backward_partials_are_bounded(lib, m, k, n, rank, most):
     assert 0 < lib.cf_lora_backward_dtype_workspace_bytes(_lib.CF_F32, m, k, n, rank) <= most
 
 
+def test_input_gradient_update_by_sizes(lib):
+    def own(dtype, m, k, n, rank):
+        return lib.cf_lora_backward_updates_input(dtype, m, k, n, rank)
+
+    assert own(_lib.CF_BF16, 4096, 4096, 4096, 64) == 1
+    assert own(_lib.CF_F32, 8192, 4096, 4096, 16) == 1
+    assert own(_lib.CF_F32, 2048, 4096, 4096, 1) == 1 and own(_lib.CF_F32, 2049, 4096, 4096, 17) == 0
+    for dtype in (_lib.CF_F32, _lib.CF_BF16):
+        assert own(dtype, 512, 128, 130, 128) == 1 and own(dtype, 513, 128, 130, 128) == 0
+        assert own(dtype, 2000, 1001, 1003, 16) == 0
+        assert own(dtype, 2**31, 2**31, 2**31, 100) == 0
+
+
 def test_empty_inputs_return_ok_without_touching_the_device(lib):
     null = ctypes.c_void_p(0)
     assert lib.cf_quantize_int8(null, _lib.CF_F32, null, null, 0, null) == _lib.CF_OK

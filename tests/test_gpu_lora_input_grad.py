@@ -1,7 +1,8 @@
 """The input gradient of the LoRA linear on the training path (the plain GEMM
 plus the adapter's part added in place by the HIP kernels) against float64:
 every rank block count, ranks with and without whole 16-byte rows of a, row
-and column remainders, the generic path (fp32, odd widths, rank above 64),
+and column remainders, the plain kernel (fp32, odd widths, rank above 64) and
+the sizes at which a GEMM takes its place,
 infinite gradients, more rows than one launch takes, and the composed path a
 recorded backward takes."""
 
@@ -30,7 +31,7 @@ def _operands(m, k, n, r, dtype, seed):
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
 @pytest.mark.parametrize("shape", [
     (1, 8, 16, 1), (17, 264, 72, 4), (64, 256, 256, 16), (130, 520, 264, 24), (333, 688, 1024, 64), (65, 48, 40, 7),
-    (100, 130, 70, 5), (40, 256, 136, 100),
+    (100, 130, 70, 5), (40, 256, 136, 100), (1100, 520, 264, 24), (300, 1001, 130, 70),
 ], ids=str)
 def test_input_gradient_matches_float64(dtype, shape):
     m, k, n, r = shape
