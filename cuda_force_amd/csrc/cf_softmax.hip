@@ -28,8 +28,8 @@
 // element at a time ([300, 50257] fp32 194 -> 38 us, [1024, 32001] bf16 to
 // fp32 142 -> 51).
 //
-// Fallback: longer rows use a workgroup per row with three passes over the row
-// (max, sum, normalise).
+// Fallback: longer rows, and ragged ones below 384 (fp32) or 512 columns, use a
+// workgroup per row with three passes over the row (max, sum, normalise).
 //
 // cf_softmax_scaled is the same kernel on scale * x with an optional causal
 // mask (column c of row r hidden when c > r mod period): the attention-score
@@ -414,6 +414,21 @@ __global__ __launch_bounds__(kThreads) void softmax_ragged_kernel(const Tin* x, 
     }
 }
 
+template <typename Tin, typename Tout, int kElems, bool kMasked, int kThreads>
+void launch_ragged(const void* x, void* y, int64_t rows, int64_t cols, const Masking& mask, hipStream_t stream) {
+    launch(softmax_ragged_kernel<Tin, Tout, kElems, kMasked, kThreads>,
+           dim3(static_cast<unsigned>(rows < (1 << 20) ? rows : (1 << 20))), dim3(kThreads), 0, stream,
+           static_cast<const Tin*>(x), static_cast<Tout*>(y), rows, cols, mask);
+}
+
+/// Ragged rows below this many columns take the three passes: a lane has an
+/// element or two, which stay in cache, and the other kernel would issue eight
+/// steps for them ([20000, 33] bf16 11.8 against 24.9 us, [20000, 255] 18.5
+/// against 26.0, [20000, 401] 24.5 against 26.3; fp32 [20000, 255] 18.0 against
+/// 22.5, [20000, 401] 24.8 against 23.0).
+template <typename Tin>
+constexpr int64_t kNarrowRagged = sizeof(Tin) == 4 ? 384 : 512;
+
 /// Any shape: one workgroup per row, three passes.
 template <typename Tin, typename Tout, bool kMasked>
 __global__ __launch_bounds__(kDefaultBlockSize) void softmax_block_kernel(const Tin* x, Tout* y,
@@ -530,19 +545,20 @@ cf_status dispatch(const void* x, void* y, int64_t rows, int64_t cols, const Mas
         } else {
             launch_row<Tin, Tout, 8, kMasked>(x, y, rows, cols, mask, stream);
         }
-    } else if (cols <= 64 * kRowThreads) {
-        const dim3 grid(static_cast<unsigned>(rows < (1 << 20) ? rows : (1 << 20)));
-        const auto* xin = static_cast<const Tin*>(x);
-        auto* out = static_cast<Tout*>(y);
+    } else if (cols >= kNarrowRagged<Tin> && cols <= 64 * kRowThreads) {
+        // As few threads as hold the row in 32 registers each, so that the
+        // waves' steps past its end stay few ([4096, 4097] bf16 in 32 x 1024
+        // threads 46.7 us, three passes 31.2).
         if (cols <= 16 * 256) {
-            launch(softmax_ragged_kernel<Tin, Tout, 16, kMasked, 256>, grid, dim3(256), 0, stream, xin, out, rows,
-                   cols, mask);
+            launch_ragged<Tin, Tout, 16, kMasked, 256>(x, y, rows, cols, mask, stream);
+        } else if (cols <= 32 * 256) {
+            launch_ragged<Tin, Tout, 32, kMasked, 256>(x, y, rows, cols, mask, stream);
+        } else if (cols <= 32 * 512) {
+            launch_ragged<Tin, Tout, 32, kMasked, 512>(x, y, rows, cols, mask, stream);
         } else if (cols <= 32 * kRowThreads) {
-            launch(softmax_ragged_kernel<Tin, Tout, 32, kMasked, kRowThreads>, grid, dim3(kRowThreads), 0, stream,
-                   xin, out, rows, cols, mask);
+            launch_ragged<Tin, Tout, 32, kMasked, kRowThreads>(x, y, rows, cols, mask, stream);
         } else {
-            launch(softmax_ragged_kernel<Tin, Tout, 64, kMasked, kRowThreads>, grid, dim3(kRowThreads), 0, stream,
-                   xin, out, rows, cols, mask);
+            launch_ragged<Tin, Tout, 64, kMasked, kRowThreads>(x, y, rows, cols, mask, stream);
         }
     } else {
         const int64_t max_blocks = static_cast<int64_t>(cu_count()) * 8;

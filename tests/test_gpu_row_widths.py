@@ -1,6 +1,6 @@
 """Row operators at the widths where their kernels change: ragged softmax rows
-(an element per lane: the edges of its three register sizes and one past the
-last), aligned rows of a workgroup each, with and without the causal mask and
+(three passes up to 383 or 511 columns, an element per lane above: the edges of
+its sizes and one past the last), aligned rows of a workgroup each, with and without the causal mask and
 in place, and RMSNorm rows of a workgroup each (few rows, and more than eight
 vectors per lane). Against float64 at the tolerances of test_gpu_rowops:
 1e-5 relative for fp32 results, 1e-2 for 16-bit ones."""
@@ -31,7 +31,7 @@ def _normal(rows, cols, dtype, seed, std=1.0):
 
 
 @pytest.mark.parametrize("src,dst", [("f32", "f32"), ("bf16", "f32"), ("bf16", "bf16"), ("f16", "f32"), ("f32", "f16")])
-@pytest.mark.parametrize("cols", [1, 63, 257, 4095, 4097, 32767, 32769, 50257, 65535, 65537, 8200, 16384, 32000])
+@pytest.mark.parametrize("cols", [1, 63, 257, 383, 385, 511, 513, 4095, 4097, 8191, 8193, 16383, 16385, 32767, 32769, 50257, 65535, 65537, 8200, 16384, 32000])
 def test_softmax_widths(src, dst, cols):
     g.announce(f"softmax width {cols} {src} -> {dst}")
     x = _normal(5, cols, DTYPES[src], cols, 2.0)
