@@ -50,10 +50,9 @@ constexpr int kWavesPerBlock = kDefaultBlockSize / kWaveSize;
 /// Store `n` (4 or 8) floats as Tout at `p` with 16- or 8-byte streaming stores.
 /// kMerge: eight fp32 values, 32 bytes of a lane, go out as plain stores. Each
 /// of the two instructions writes every other 16 bytes, so the lines are only
-/// whole once the L2 has merged the two; streaming stores sent the halves on
-/// ([1024, 32000] bf16 -> fp32 55.3 us, merged 36.9). With one vector per
-/// thread streaming is the faster one ([600, 8000] fp16 -> fp32 8.6 against
-/// 9.5).
+/// whole once the L2 has merged the two; streaming stores send the halves on
+/// ([1024, 32000] bf16 -> fp32 55.4 us, merged 35.6). While the result fits the
+/// L2s (32 MB) or a thread has one vector, streaming is the faster one (below).
 template <typename Tout, int kN, bool kMerge = false>
 __device__ __forceinline__ void store_vec(Tout* p, const float* v) {
     constexpr int kOutPer = Storage<Tout>::kPerVec;
@@ -241,7 +240,15 @@ __global__ __launch_bounds__(kDefaultBlockSize) void softmax_wave_kernel(const T
 /// cross-wave reductions through LDS.
 constexpr int kRowThreads = 1024;
 
-template <typename Tin, typename Tout, int kVecs, bool kFullCols, bool kMasked, int kThreads = kRowThreads>
+/// Elements of an fp32 result of 16-bit rows from which its stores merge in L2
+/// (28 MiB): [128, 49152] bf16 11.7 us streaming, 13.5 merged, [100, 65536] 12.5
+/// and 14.7, [257, 20000] 9.8 and 10.2; [400, 20000] 13.0 and 12.3, [257, 32000]
+/// 15.6 and 13.9, [400, 65536] 49.1 and 35.4. One vector a thread streams
+/// ([600, 8000] fp16 8.6, merged 9.5). Two kernels: a choice inside one cost
+/// either way 5-10%.
+constexpr int64_t kMergeElements = 7LL << 20;
+
+template <typename Tin, typename Tout, int kVecs, bool kFullCols, bool kMasked, int kThreads, bool kMerge>
 __global__ __launch_bounds__(kThreads) void softmax_row_kernel(const Tin* x, Tout* y, int64_t rows,
                                                                int64_t cols, Masking mask) {
     constexpr int kPer = Storage<Tin>::kPerVec;
@@ -308,7 +315,7 @@ __global__ __launch_bounds__(kThreads) void softmax_row_kernel(const Tin* x, Tou
             if (kFullCols || idx < vec_cols) {
 #pragma unroll
                 for (int i = 0; i < kPer; ++i) v[j][i] = v[j][i] * inv_sum;
-                store_probs<Tout, kPer, (kVecs >= 4)>(y + row * cols + idx * kPer, v[j], row_nan);
+                store_probs<Tout, kPer, kMerge>(y + row * cols + idx * kPer, v[j], row_nan);
             }
         }
     }
@@ -320,13 +327,17 @@ void launch_row(const void* x, void* y, int64_t rows, int64_t cols, const Maskin
     const unsigned grid = static_cast<unsigned>(rows < (1 << 20) ? rows : (1 << 20));
     const auto* xin = static_cast<const Tin*>(x);
     auto* out = static_cast<Tout*>(y);
-    if (full) {
-        launch(softmax_row_kernel<Tin, Tout, kVecs, true, kMasked, kThreads>, dim3(grid), dim3(kThreads), 0, stream,
-               xin, out, rows, cols, mask);
-    } else {
-        launch(softmax_row_kernel<Tin, Tout, kVecs, false, kMasked, kThreads>, dim3(grid), dim3(kThreads), 0, stream,
-               xin, out, rows, cols, mask);
+    auto run = [&](auto whole, auto merged) {
+        launch(softmax_row_kernel<Tin, Tout, kVecs, decltype(whole)::value, kMasked, kThreads, decltype(merged)::value>,
+               dim3(grid), dim3(kThreads), 0, stream, xin, out, rows, cols, mask);
+    };
+    if constexpr (sizeof(Tin) == 2 && sizeof(Tout) == 4 && kVecs >= 4) {
+        if (rows * cols > kMergeElements) {
+            full ? run(std::true_type{}, std::true_type{}) : run(std::false_type{}, std::true_type{});
+            return;
+        }
     }
+    full ? run(std::true_type{}, std::false_type{}) : run(std::false_type{}, std::false_type{});
 }
 
 /// Ragged rows (a width that is not whole 16-byte vectors, or unaligned

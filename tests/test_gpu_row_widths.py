@@ -1,7 +1,7 @@
 """Row operators at the widths where their kernels change: ragged softmax rows
 (three passes up to 383 or 511 columns, an element per lane above: the edges of
 its sizes and one past the last), aligned rows of a workgroup each, with and without the causal mask and
-in place, and RMSNorm rows of a workgroup each (few rows, and more than eight
+in place, fp32 results on both sides of the size from which their stores merge, and RMSNorm rows of a workgroup each (few rows, and more than eight
 vectors per lane). Against float64 at the tolerances of test_gpu_rowops:
 1e-5 relative for fp32 results, 1e-2 for 16-bit ones."""
 
@@ -41,6 +41,15 @@ def test_softmax_widths(src, dst, cols):
     keep = torch.arange(cols, device="cuda")[None] <= (torch.arange(5, device="cuda") % 3)[:, None]
     exact = torch.softmax((0.5 * x.double()).masked_fill(~keep, float("-inf")), -1)
     _close(y, exact, DTYPES[dst], f"masked {cols} {src}->{dst}")
+
+
+@pytest.mark.parametrize("rows,cols", [(229, 32000), (230, 32000), (224, 32768), (225, 32768), (112, 65536), (113, 65536)])
+def test_fp32_results_on_both_sides_of_28_mib(rows, cols):
+    """16-bit rows to fp32: streaming stores below, merged ones above, whole
+    register rows and part ones."""
+    g.announce(f"softmax [{rows}, {cols}] bf16 -> f32")
+    x = _normal(rows, cols, torch.bfloat16, rows, 2.0)
+    _close(ops.softmax_as(x, torch.float32), torch.softmax(x.double(), -1), torch.float32, f"{rows} x {cols}")
 
 
 def test_ragged_softmax_unaligned_and_in_place():
