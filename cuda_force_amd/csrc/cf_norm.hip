@@ -496,6 +496,20 @@ cf_status dispatch(const void* x, const void* residual, const void* w, void* y,
     if (kResidual) vec = vec && host_aligned(residual, 16) && host_aligned(residual_out, 16);
     const int64_t vectors_per_lane = ceil_div<int64_t>(cols / kPer, kWaveSize);
     const int64_t row_vectors = cols / kPer;
+    // Rows of 9 to 16 vectors per lane that a wave still holds better than a
+    // workgroup: the plain norm of 1536 and more rows that fill the wave ([2048,
+    // 8192] bf16 11.8 us against 13.8, [2000, 4096] fp32 11.3 against 13.1, even
+    // from 4096 rows on) or, in fp32 and bf16, fit the L2s ([2000, 5120] bf16 8.6
+    // against 9.8; [4096, 5120] 18.7 against 17.1), and with the residual fp32
+    // rows that fill the wave, up to 2048 ([700, 4096] 8.4 against 9.7, [1000,
+    // 4096] 11.5 against 12.4; [3000, 4096] 35.3 against 33.1, [2000, 8192] bf16
+    // 24.3 against 23.7).
+    const bool fills = row_vectors == 16 * kWaveSize;
+    const bool wave16 =
+        vectors_per_lane > 8 && vectors_per_lane <= 16 &&
+        (kResidual ? sizeof(T) == 4 && fills && rows > 512 && rows <= 2048
+                   : rows >= 1536 && (fills || (!std::is_same_v<T, f16_t> &&
+                                                rows * cols * static_cast<int64_t>(sizeof(T)) <= 32LL << 20)));
     // The tiled kernel wins once the matrix holds at least 16 x 1024
     // 16-byte vectors per CU, several rounds of workgroups (measured on [16384,
     // 2048 / 4096 / 8192] bf16: 1-3 points of HBM peak); below that
@@ -524,32 +538,37 @@ cf_status dispatch(const void* x, const void* residual, const void* w, void* y,
         } else {
             run(Tile1024{});
         }
-    } else if (vec && rows < (1LL << 31) && row_vectors <= 8192 &&
+    } else if (vec && rows < (1LL << 31) && row_vectors <= 8192 && !wave16 &&
                (vectors_per_lane > 8 || (rows <= cu_count() && vectors_per_lane > 4))) {
         // A workgroup per row where a wave would hold more than eight vectors
         // per lane (fused residual [8192, 5120] bf16 68.3 -> 56.5 us, [800,
         // 6712] fp16 19.6 -> 11.3, [8000, 2560] fp32 62.9 -> 54.1), and for
         // few rows of more than four ([4, 4096] bf16 4.06 -> 3.79). With up to
         // eight the wave kernel is the faster one ([4096, 4096] bf16 12.0
-        // against 13.8 us, [2048, 4096] fp32 11.0 against 13.3).
+        // against 13.8 us, [2048, 4096] fp32 11.0 against 13.3), and so it is
+        // where wave16 says.
         if (row_vectors <= 512) {
             launch_row<T, 1, 512, kResidual>(x, residual, w, y, residual_out, rows, cols, eps, stream);
         } else if (row_vectors <= 1024) {
             launch_row<T, 2, 512, kResidual>(x, residual, w, y, residual_out, rows, cols, eps, stream);
         } else if (row_vectors <= 2048) {
             launch_row<T, 2, 1024, kResidual>(x, residual, w, y, residual_out, rows, cols, eps, stream);
+        } else if (row_vectors <= 4096) {
+            launch_row<T, 4, 1024, kResidual>(x, residual, w, y, residual_out, rows, cols, eps, stream);
         } else {
             launch_row<T, 8, 1024, kResidual>(x, residual, w, y, residual_out, rows, cols, eps, stream);
         }
-    } else if (vec && vectors_per_lane <= 8) {
+    } else if (vec && vectors_per_lane <= 16) {
         if (vectors_per_lane <= 1) {
             launch_wave<T, 1, kResidual>(x, residual, w, y, residual_out, rows, cols, eps, stream);
         } else if (vectors_per_lane <= 2) {
             launch_wave<T, 2, kResidual>(x, residual, w, y, residual_out, rows, cols, eps, stream);
         } else if (vectors_per_lane <= 4) {
             launch_wave<T, 4, kResidual>(x, residual, w, y, residual_out, rows, cols, eps, stream);
-        } else {
+        } else if (vectors_per_lane <= 8) {
             launch_wave<T, 8, kResidual>(x, residual, w, y, residual_out, rows, cols, eps, stream);
+        } else {
+            launch_wave<T, 16, kResidual>(x, residual, w, y, residual_out, rows, cols, eps, stream);
         }
     } else {
         const int64_t max_blocks = static_cast<int64_t>(cu_count()) * 8;

@@ -1,8 +1,9 @@
 """Row operators at the widths where their kernels change: ragged softmax rows
 (three passes up to 383 or 511 columns, an element per lane above: the edges of
-its sizes and one past the last), aligned rows of a workgroup each, with and without the causal mask and
-in place, fp32 results on both sides of the size from which their stores merge, and RMSNorm rows of a workgroup each (few rows, and more than eight
-vectors per lane). Against float64 at the tolerances of test_gpu_rowops:
+its sizes and one past the last), aligned rows of a workgroup each, with and
+without the causal mask and in place, fp32 results on both sides of the size
+from which their stores merge, and RMSNorm rows of a workgroup each (few rows,
+and more than eight vectors per lane, on both sides of where a wave holds them). Against float64 at the tolerances of test_gpu_rowops:
 1e-5 relative for fp32 results, 1e-2 for 16-bit ones."""
 
 from __future__ import annotations
@@ -69,7 +70,8 @@ def test_ragged_softmax_unaligned_and_in_place():
 
 @pytest.mark.parametrize("dtype", ["f32", "bf16", "f16"])
 @pytest.mark.parametrize("shape", [(1, 2056), (4, 4096), (256, 4104), (257, 4104), (300, 5120), (40, 8192), (300, 2560),
-                                   (3, 16384), (700, 6712), (5, 32768)], ids=str)
+                                   (3, 16384), (700, 6712), (5, 32768), (3, 18440), (1536, 4096), (1535, 8192),
+                                   (1540, 8192), (513, 4096), (2049, 4096), (1600, 5120), (1700, 10240)], ids=str)
 def test_rmsnorm_row_workgroups(dtype, shape):
     rows, cols = shape
     g.announce(f"RMSNorm row workgroups {dtype} {shape}")
