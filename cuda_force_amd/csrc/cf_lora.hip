@@ -358,17 +358,35 @@ cf_status launch_generic(const void* x, const void* w, const void* a, const void
     return check_launch("launching the tiled LoRA GEMM", stream);
 }
 
-/// The kernels of cf_lora_forward for a bf16 problem, by its sizes.
-enum class Route { kLinear, kSkinny, kTile };
+/// The kernels of cf_lora_forward for a bf16 problem, by its sizes, and what
+/// they need.
+struct Route {
+    enum { kLinear, kSkinny, kTile } kernels = kLinear;
+    size_t workspace = 0;  // beyond cf_lora_linear_ws's
+    SkinnyPlan skinny;
+    TilePlan tile;
+};
 
 Route route_of(int64_t M, int64_t N, int64_t K, int64_t rank) {
-    if (lora_skinny_shape(M, N, K, rank)) return Route::kSkinny;
-    if (!lora_tile_shape(M, N, K, rank)) return Route::kLinear;
-    // The 256x256-tile kernel where it runs and is estimated no slower.
+    Route route;
+    // The 256x256-tile kernel where it runs and is estimated no slower (without
+    // an adapter it is some 3 us shorter: 16 x 128 x 4096 r0 7.3 us, r16 9.8).
     const bool fused = K % 64 == 0 && rank <= 16 && rank % 2 == 0;
-    return fused && lora_fused_estimate_us(M, N, K) <= 1.05f * lora_tile_estimate_us(M, N, K, rank)
-               ? Route::kLinear
-               : Route::kTile;
+    const float fused_us = fused ? lora_fused_estimate_us(M, N, K) : 0.0f;
+    if (lora_skinny_plan(M, N, K, rank, route.skinny)) {
+        const float shorter = rank == 0 ? 3.0f : 0.0f;
+        if (!fused || fused_us - shorter >= lora_skinny_estimate_us(route.skinny, M, N, K)) {
+            route.kernels = Route::kSkinny;
+            route.workspace = lora_skinny_workspace_bytes(route.skinny, M, N, rank);
+        }
+    } else if (lora_tile_shape(M, N, K, rank)) {
+        route.tile = lora_tile_plan(M, N, K, rank);
+        if (!fused || fused_us > 1.05f * route.tile.us) {
+            route.kernels = Route::kTile;
+            route.workspace = lora_tile_workspace_bytes(route.tile, M, N, rank);
+        }
+    }
+    return route;
 }
 
 }  // namespace
@@ -475,17 +493,7 @@ size_t cf_lora_forward_workspace_bytes(cf_dtype dtype, int64_t batch, int64_t in
                                        int64_t out_features, int64_t rank) {
     const size_t plain = cf_lora_linear_ws_bytes(dtype, batch, in_features, out_features, rank);
     if (dtype != CF_BF16) return plain;
-    size_t needed = 0;
-    switch (cf::route_of(batch, out_features, in_features, rank)) {
-        case cf::Route::kSkinny:
-            needed = cf::lora_skinny_workspace_bytes(batch, out_features, in_features, rank);
-            break;
-        case cf::Route::kTile:
-            needed = cf::lora_tile_workspace_bytes(batch, out_features, in_features, rank);
-            break;
-        case cf::Route::kLinear:
-            break;
-    }
+    const size_t needed = cf::route_of(batch, out_features, in_features, rank).workspace;
     return needed > plain ? needed : plain;
 }
 
@@ -500,23 +508,20 @@ cf_status cf_lora_forward(const void* x, const void* w, const void* a, const voi
                "cf_lora_forward: dtype %s has no kernel (float32 or bfloat16)", cf::dtype_name(dtype));
     CF_REQUIRE(x != nullptr && w != nullptr && y != nullptr, "cf_lora_forward: null pointer");
     CF_REQUIRE(rank == 0 || (a != nullptr && b != nullptr), "cf_lora_forward: null adapter");
-    const size_t needed =
-        cf_lora_forward_workspace_bytes(dtype, batch, in_features, out_features, rank);
+    const size_t plain = cf_lora_linear_ws_bytes(dtype, batch, in_features, out_features, rank);
+    cf::Route route;
+    if (dtype == CF_BF16) route = cf::route_of(batch, out_features, in_features, rank);
+    const size_t needed = route.workspace > plain ? route.workspace : plain;
     CF_REQUIRE(needed == 0 || (workspace != nullptr && workspace_bytes >= needed),
                "cf_lora_forward: workspace of %zu bytes given, %zu needed", workspace_bytes, needed);
     CF_REQUIRE(cf::host_aligned(workspace, 16), "cf_lora_forward: workspace must be 16-byte aligned");
-    if (dtype == CF_BF16) {
-        const cf::Route route = cf::route_of(batch, out_features, in_features, rank);
-        if (route == cf::Route::kSkinny &&
-            cf::lora_skinny_eligible(x, w, a, b, y, batch, out_features, in_features, rank)) {
-            return cf::launch_lora_skinny(x, w, a, b, y, xa_out, batch, out_features, in_features, rank,
-                                          scale, workspace, static_cast<hipStream_t>(stream));
-        }
-        if (route == cf::Route::kTile &&
-            cf::lora_tile_eligible(x, w, a, b, y, batch, out_features, in_features, rank)) {
-            return cf::launch_lora_tile(x, w, a, b, y, xa_out, batch, out_features, in_features, rank,
-                                        scale, workspace, static_cast<hipStream_t>(stream));
-        }
+    if (route.kernels == cf::Route::kSkinny && cf::lora_skinny_aligned(x, w, a, b, y, rank)) {
+        return cf::launch_lora_skinny(route.skinny, x, w, a, b, y, xa_out, batch, out_features, in_features,
+                                      rank, scale, workspace, static_cast<hipStream_t>(stream));
+    }
+    if (route.kernels == cf::Route::kTile && cf::lora_tile_aligned(x, w, a, b, y, rank)) {
+        return cf::launch_lora_tile(route.tile, x, w, a, b, y, xa_out, batch, out_features, in_features, rank,
+                                    scale, workspace, static_cast<hipStream_t>(stream));
     }
     return cf_lora_linear_ws(x, w, a, b, y, xa_out, dtype, batch, in_features, out_features, rank,
                              scale, workspace, workspace_bytes, stream);

@@ -342,20 +342,13 @@ __global__ __launch_bounds__(kFinishThreads) void lora_skinny_finish_kernel(Fini
     *reinterpret_cast<uint2*>(args.y + row * N + col) = packed;
 }
 
-struct Plan {
-    int strips;
-    int a_strips;
-    int slices;
-    int slice_blocks;
-};
-
 /// Workgroups of the streaming kernel that fit a CU, by their registers (140
 /// with one 16-row block of x, 192 to 214 with more; the element loads of a
 /// rank that is not a multiple of 8 spill 65 at three).
 int per_cu(int64_t M, int64_t rank) { return M <= 16 && rank % 8 == 0 ? 3 : 2; }
 
-Plan plan_for(int64_t M, int64_t N, int64_t K, int64_t rank) {
-    Plan plan;
+SkinnyPlan plan_for(int64_t M, int64_t N, int64_t K, int64_t rank) {
+    SkinnyPlan plan;
     plan.strips = static_cast<int>(ceil_div<int64_t>(N, kStrip));
     plan.a_strips = static_cast<int>(ceil_div<int64_t>(rank, kStrip));
     const int64_t blocks = ceil_div<int64_t>(K, kBlockK);
@@ -374,7 +367,7 @@ size_t align256(size_t bytes) { return (bytes + 255) / 256 * 256; }
 
 }  // namespace
 
-bool lora_skinny_shape(int64_t M, int64_t N, int64_t K, int64_t rank) {
+bool lora_skinny_plan(int64_t M, int64_t N, int64_t K, int64_t rank, SkinnyPlan& plan) {
     if (M < 1 || M > kSkinnyMaxRows || N <= 0 || K <= 0 || N % 8 != 0 || K % 8 != 0 || rank < 0 ||
         rank > kMaxRank) {
         return false;
@@ -383,26 +376,41 @@ bool lora_skinny_shape(int64_t M, int64_t N, int64_t K, int64_t rank) {
     // are 32-bit with the out-of-range marker at 2^31. (The partials of x @ a,
     // at most 768 slices of 64 x 256, are 50 MB.)
     constexpr int64_t kLimit = 1LL << 31;
-    return K < kLimit && N < kLimit && K * N * 2 < kLimit && M * K * 2 < kLimit && K * rank * 2 < kLimit &&
-           rank * N * 2 < kLimit && plan_for(M, N, K, rank).slices * M * N * 4 < kLimit;
+    if (K >= kLimit || N >= kLimit || K * N * 2 >= kLimit || M * K * 2 >= kLimit || K * rank * 2 >= kLimit ||
+        rank * N * 2 >= kLimit) {
+        return false;
+    }
+    plan = plan_for(M, N, K, rank);
+    return plan.slices * M * N * 4 < kLimit;
 }
 
-bool lora_skinny_eligible(const void* x, const void* w, const void* a, const void* b, const void* y,
-                          int64_t M, int64_t N, int64_t K, int64_t rank) {
-    return lora_skinny_shape(M, N, K, rank) && host_aligned(x, 16) && host_aligned(w, 16) &&
-           host_aligned(y, 8) && (rank == 0 || (host_aligned(a, 2) && host_aligned(b, 16)));
+bool lora_skinny_aligned(const void* x, const void* w, const void* a, const void* b, const void* y, int64_t rank) {
+    return host_aligned(x, 16) && host_aligned(w, 16) && host_aligned(y, 8) &&
+           (rank == 0 || (host_aligned(a, 2) && host_aligned(b, 16)));
 }
 
-size_t lora_skinny_workspace_bytes(int64_t M, int64_t N, int64_t K, int64_t rank) {
-    const Plan plan = plan_for(M, N, K, rank);
+// Two launches, w at the rate of a launch that ramps, and for each output its
+// bf16 and its fp32 partials written and read. Of short reductions little is left
+// to split, and the 256x256-tile kernel's one launch is the faster way: whole
+// call, that one and these, 1 x 64 x 4096 r16 8.3 and 9.3 us, 64 x 128 x 32000
+// 10.5 and 22.3, 48 x 1024 x 32000 26.8 and 29.9; 4 x 192 x 4096 11.0 and 9.5, 64 x
+// 512 x 4096 17.0 and 11.2, 32 x 2048 x 32000 45 and 36. (Fitted to 174 sizes, K 64
+// to 4096 and N 64 to 32000.)
+float lora_skinny_estimate_us(const SkinnyPlan& plan, int64_t M, int64_t N, int64_t K) {
+    const float outputs = static_cast<float>(M * N);
+    const float us = 0.4f + static_cast<float>(K * N * 2) / 5.5e6f +
+                     outputs * (5.5f + 3.5f * static_cast<float>(plan.slices)) / 1e6f;
+    return us > 5.0f ? us : 5.0f;
+}
+
+size_t lora_skinny_workspace_bytes(const SkinnyPlan& plan, int64_t M, int64_t N, int64_t rank) {
     return align256(static_cast<size_t>(plan.slices) * M * N * 4) +
            align256(static_cast<size_t>(plan.slices) * M * rank * 4);
 }
 
-cf_status launch_lora_skinny(const void* x, const void* w, const void* a, const void* b, void* y,
+cf_status launch_lora_skinny(const SkinnyPlan& plan, const void* x, const void* w, const void* a, const void* b, void* y,
                              float* xa_out, int64_t M, int64_t N, int64_t K, int64_t rank,
                              float scale, void* workspace, hipStream_t stream) {
-    const Plan plan = plan_for(M, N, K, rank);
     SkinnyArgs args;
     args.x = static_cast<const uint16_t*>(x);
     args.w = static_cast<const uint16_t*>(w);

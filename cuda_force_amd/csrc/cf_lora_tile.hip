@@ -600,16 +600,8 @@ struct Config {
 
 constexpr Config kConfigs[] = {{128, 256}, {128, 128}, {64, 128}};
 
-struct Plan {
-    int config;
-    int whole;        // tiles of one workgroup
-    int slices;       // of the tiles after them
-    int slice_steps;
-    float us;         // estimate
-};
-
-Plan make_plan(int config, int64_t whole, int64_t want, int64_t steps) {
-    Plan p;
+TilePlan make_plan(int config, int64_t whole, int64_t want, int64_t steps) {
+    TilePlan p;
     p.config = config;
     p.whole = static_cast<int>(whole);
     p.slice_steps = static_cast<int>(ceil_div<int64_t>(steps, want));
@@ -633,12 +625,12 @@ constexpr int kMinSliceSteps = 4;
 /// of one workgroup per CU and the tiles left over split (258 tiles of 333 x
 /// 4096 x 11008 take 65.4 us as 258 workgroups, where two CUs work twice as
 /// long, and 56.4 us as 256 plus 2 x 8 slices).
-/// (The workspace query and the launch both come here, so it is kept to a few
-/// dozen candidates and 32-bit divisions: 0.3 us.)
-Plan best_plan(int64_t M, int64_t N, int64_t K, int64_t rank) {
+/// (A call comes here twice, for the workspace and for the launch, so it is kept
+/// to a few dozen candidates and 32-bit divisions: 0.3 us.)
+TilePlan best_plan(int64_t M, int64_t N, int64_t K, int64_t rank) {
     constexpr int kSlices[] = {1, 2, 3, 4, 5, 6, 8, 12, 16, 24, 32};
     const int steps = static_cast<int>(ceil_div<int64_t>(K, kBK) + ext_of(rank) / kBK);
-    Plan best;
+    TilePlan best;
     best.us = INFINITY;
     for (int c = 0; c < 3; ++c) {
         const int bm = kConfigs[c].bm;
@@ -689,7 +681,7 @@ void launch_tile(const TileArgs& args, hipStream_t stream) {
            dim3(kWM * kWN * 64), 0, stream, args);
 }
 
-cf_status run_plan(const Plan& plan, const void* x, const void* w, const void* a, const void* b, void* y,
+cf_status run_plan(const TilePlan& plan, const void* x, const void* w, const void* a, const void* b, void* y,
                    float* xa_out, int64_t M, int64_t N, int64_t K, int64_t rank, float scale, void* workspace,
                    hipStream_t stream) {
     const int64_t ext = ext_of(rank);
@@ -765,28 +757,24 @@ bool lora_tile_shape(int64_t M, int64_t N, int64_t K, int64_t rank) {
            ceil_div<int64_t>(M, 64) * ceil_div<int64_t>(N, 128) < (1LL << 24);
 }
 
-bool lora_tile_eligible(const void* x, const void* w, const void* a, const void* b, const void* y,
-                        int64_t M, int64_t N, int64_t K, int64_t rank) {
-    return lora_tile_shape(M, N, K, rank) && host_aligned(x, 16) && host_aligned(w, 16) &&
-           host_aligned(y, 16) && (rank == 0 || (host_aligned(a, 2) && host_aligned(b, 16)));
+bool lora_tile_aligned(const void* x, const void* w, const void* a, const void* b, const void* y, int64_t rank) {
+    return host_aligned(x, 16) && host_aligned(w, 16) && host_aligned(y, 16) &&
+           (rank == 0 || (host_aligned(a, 2) && host_aligned(b, 16)));
 }
 
-float lora_tile_estimate_us(int64_t M, int64_t N, int64_t K, int64_t rank) {
-    return best_plan(M, N, K, rank).us;
-}
+TilePlan lora_tile_plan(int64_t M, int64_t N, int64_t K, int64_t rank) { return best_plan(M, N, K, rank); }
 
-size_t lora_tile_workspace_bytes(int64_t M, int64_t N, int64_t K, int64_t rank) {
-    const Plan p = best_plan(M, N, K, rank);
+size_t lora_tile_workspace_bytes(const TilePlan& p, int64_t M, int64_t N, int64_t rank) {
     const Config& c = kConfigs[p.config];
     const int64_t tiles = ceil_div<int64_t>(M, c.bm) * ceil_div<int64_t>(N, c.bn);
     return align256(static_cast<size_t>(M * ext_of(rank)) * 2) +
            static_cast<size_t>((tiles - p.whole) * p.slices) * c.bm * c.bn * 4;
 }
 
-cf_status launch_lora_tile(const void* x, const void* w, const void* a, const void* b, void* y,
-                           float* xa_out, int64_t M, int64_t N, int64_t K, int64_t rank,
-                           float scale, void* workspace, hipStream_t stream) {
-    return run_plan(best_plan(M, N, K, rank), x, w, a, b, y, xa_out, M, N, K, rank, scale, workspace, stream);
+cf_status launch_lora_tile(const TilePlan& plan, const void* x, const void* w, const void* a, const void* b,
+                           void* y, float* xa_out, int64_t M, int64_t N, int64_t K, int64_t rank, float scale,
+                           void* workspace, hipStream_t stream) {
+    return run_plan(plan, x, w, a, b, y, xa_out, M, N, K, rank, scale, workspace, stream);
 }
 
 }  // namespace cf

@@ -55,9 +55,9 @@ def test_workspace_queries(lib):
 
 
 @pytest.mark.parametrize("m,k,n,rank,few_rows", [
-    (64, 64, 8388600, 16, True),     # partials just below 2 GiB
-    (64, 64, 8388608, 16, False),    # at 2 GiB
-    (64, 64, 9000000, 16, False),
+    (64, 64, 8388600, 17, True),     # partials just below 2 GiB
+    (64, 64, 8388608, 17, False),    # at 2 GiB
+    (64, 64, 9000000, 17, False),
     (1, 8, 4194296, 256, True),      # b just below 2 GiB
     (1, 8, 4194304, 256, False),
     (1, 4194296, 8, 256, True),      # a just below 2 GiB
