@@ -24,8 +24,8 @@
 //      go to fp32 workspaces, one slice per 256-column tile (G) and per
 //      row tile (grad_b). Tall tiles mean few partials (512 rows against 256:
 //      37.8 against 39.5 us at 8192 x 4096 x 4096 r16, operands cache-cold),
-//      so they are lowered only until every CU has a workgroup; three or four
-//      chunks in flight were slower.
+//      so they are lowered only where CUs would idle (chunks_for); three or
+//      four chunks in flight were slower.
 //   2. One launch sums both in a fixed order: grad_b (times scale, cast) and
 //      G -> GT (bf16 [rank padded to 16, 32 or 64, Mp]).
 //   3. The same column-reduction pass over x with GT: grad_a partials.
@@ -531,13 +531,21 @@ size_t align256(size_t bytes) { return (bytes + 255) / 256 * 256; }
 
 int rank_pad_of(int64_t rank) { return rank <= 16 ? 16 : rank <= 32 ? 32 : 64; }
 
-/// Chunks of 64 rows per workgroup: 8, 4 or 2, the most that still give the
-/// pass over `cols` columns a workgroup per CU (partials grow as it shrinks);
-/// at most 4 for four rank blocks, whose eight unrolled chunks spill.
+/// Chunks of 64 rows per workgroup: 8, 4 or 2; shorter tiles fill more CUs and
+/// leave more partials. Up to rank 16, 512 rows, halved while that still makes
+/// one round of a workgroup per CU (2000 x 4096 x 4096 r16 23.7 us, with 128 rows
+/// 18.6; 9000 x 2048 x 2048 28.1, with 256 rows, 288 workgroups, 33.4) and at
+/// most 64 partials, which few threads would sum (20000 x 1024 x 1024 30.1 with
+/// 40, 37.4 with 79). Above, where two workgroups share a CU, the most that still
+/// give each CU one; at most 4 for four rank blocks, whose eight unrolled chunks
+/// spill.
 int chunks_for(int64_t M, int64_t cols, int rank_pad) {
+    constexpr int64_t kMaxParts = 64;
     const int64_t tiles = ceil_div<int64_t>(cols, kTileCols);
     for (int chunks = rank_pad == 64 ? 4 : 8; chunks > 2; chunks /= 2) {
-        if (ceil_div<int64_t>(M, chunks * kChunkRows) * tiles >= 256) return chunks;
+        const int64_t parts = ceil_div<int64_t>(M, chunks * kChunkRows);
+        const int64_t halved = ceil_div<int64_t>(M, chunks / 2 * kChunkRows);
+        if (rank_pad == 16 ? halved * tiles > 256 || halved > kMaxParts : parts * tiles >= 256) return chunks;
     }
     return 2;
 }
