@@ -723,9 +723,9 @@ bool lora_fused_eligible(const void* x, const void* w, const void* a, const void
 
 float lora_fused_estimate_us(int64_t M, int64_t N, int64_t K) {
     const int64_t tiles = ceil_div<int64_t>(M, kBM) * ceil_div<int64_t>(N, kBN);
-    const int64_t rounds = ceil_div<int64_t>(tiles, 256);
-    const float full = tiles >= 256 ? 1.0f : static_cast<float>(tiles) / 256.0f;
-    return 3.0f + static_cast<float>(rounds * (K / kBK)) * (0.61f + 0.21f * full);
+    const float rounds = static_cast<float>(tiles / 256);
+    const float rest = static_cast<float>(tiles % 256) / 256.0f;
+    return 3.0f + static_cast<float>(K / kBK) * (0.82f * rounds + (rest > 0.0f ? 0.61f + 0.21f * rest : 0.0f));
 }
 
 size_t lora_fused_workspace_bytes(int64_t M, int64_t rank) {

@@ -13,8 +13,9 @@ bool lora_fused_eligible(const void* x, const void* w, const void* a, const void
                          int64_t N, int64_t K, int64_t rank);
 
 /// Estimated time of the launch in microseconds on sizes the kernel takes:
-/// rounds of 256x256 tiles, one per CU (measured, K = 4096: 16 tiles 81 us,
-/// 86 tiles 90 us, 256 tiles 107 us, 512 tiles 215 us).
+/// rounds of 256x256 tiles, one per CU, the last one by how full it is
+/// (measured, K = 4096: 16 tiles 81 us, 86 tiles 90 us, 256 tiles 107 us, 512
+/// tiles 215 us; K = 8192: 384 tiles 349 us).
 float lora_fused_estimate_us(int64_t M, int64_t N, int64_t K);
 
 /// Bytes of workspace launch_lora_fused can use for an M-row problem of
