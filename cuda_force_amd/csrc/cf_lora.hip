@@ -6,10 +6,10 @@
 //   y = x @ w + scale * ((x @ a) @ b)
 //
 // Fast path (bf16, K % 64 == 0, N % 8 == 0, r <= 16, 16-byte aligned): the
-// fused MFMA kernel in cf_lora_fused.hip, one launch. With at most 64 rows
-// and a workspace, the kernels of cf_lora_skinny.hip (any rank up to 256);
-// with a workspace, smaller tiles and any rank up to 128 (K a multiple of 8)
-// in cf_lora_tile.hip.
+// fused MFMA kernel in cf_lora_fused.hip, one launch. With a workspace also,
+// by sizes: up to 64 rows the kernels of cf_lora_skinny.hip (any rank up to
+// 256) unless the reduction is short, above them smaller tiles and any rank up
+// to 128 in cf_lora_tile.hip (K a multiple of 8 in both).
 //
 // fp32 (r <= 16, K and N multiples of 4, 16-byte aligned): the MFMA kernel of
 // cf_lora_f32.hip, operands split into bf16 high and low parts on the way
@@ -25,11 +25,13 @@
 //   grad_b = scale * xa^T @ dy   [r, N]   column reduction over M
 //   grad_a = scale * x^T @ G     [K, r]   column reduction over M
 //   grad_x = dy @ w^T (the caller's GEMM) + scale * G @ a^T, in place
-// bf16 with rank <= 64 runs the MFMA kernels of cf_lora_bwd.hip, fp32 those
-// of cf_lora_bwd_f32.hip. The generic
-// path here (other shapes): G one wave per row of dy, the column
+// bf16 with rank <= 64 runs the MFMA kernels of cf_lora_bwd.hip, fp32 those of
+// cf_lora_bwd_f32.hip for the adapter gradients. The generic path here (other
+// shapes, and fp32's update of grad_x): G one wave per row of dy, the column
 // reductions in row chunks into an fp32 workspace and a second kernel summing
-// the chunks in a fixed order (deterministic).
+// the chunks in a fixed order (deterministic), the update a thread per column
+// and 8 rows. cf_lora_backward_updates_input says where that update is slower
+// than the caller's GEMMs.
 #include "cf_common.hpp"
 #include "cf_lora_bwd.hpp"
 #include "cf_lora_f32.hpp"

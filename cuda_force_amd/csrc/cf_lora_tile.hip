@@ -22,13 +22,14 @@
 // What bounds it: copying the operands into LDS, not the MFMAs. Timing-only
 // copies at 1000 x 4096 x 4096 (256 tiles of 128x128, no adapter): whole
 // kernel 53.4 us without the fragments read ahead and 43 us with them, copies
-// alone 40.8, MFMAs alone 22.4; deeper rings change nothing, and every shape
-// moves 14-19 TB/s from L2 to LDS (64-75 GB/s per CU). So the widest tile
-// that still fills the CUs wins, and the kernel and slice counts are chosen by
-// an estimate (below) from measured times per K-step. Before, these problems
+// alone 40.8, MFMAs alone 22.4; deeper rings change nothing, and shapes that
+// fill the CUs move 11-13 TB/s from L2 to LDS (42-51 GB/s per CU; by kernel
+// trace 1000 x 4096 x 4096 11.1, 1237 x 4096 x 8192 12.9, 6000 x 11008 x 4096
+// 12.2). So the widest tile that still fills the CUs wins, and the kernel and
+// slice counts are chosen by an estimate (below) from measured times per K-step. Before, these problems
 // ran 256x256 tiles on a fraction of the CUs or, for a rank above 16 or K not
 // a multiple of 64, fp32 FMA tiles: 333 x 4096 x 11008 r16 92 -> 58 us, 100 x
-// 4096 x 4096 r16 81 -> 23, 1237 x 4096 x 8192 r64 2801 -> 109, 3530 x 984 x
+// 4096 x 4096 r16 81 -> 23, 1237 x 4096 x 8192 r64 2801 -> 108, 3530 x 984 x
 // 11008 r16 1367 -> 107, 6000 x 11008 x 4096 r32 12650 -> 573.
 //
 // Everything past an edge reads as zero: rows past M and columns past N by the
@@ -622,9 +623,9 @@ constexpr int kCus = 256;
 constexpr int kMinSliceSteps = 4;
 
 /// The fastest of: every tile one workgroup; every tile split; whole rounds
-/// of one workgroup per CU and the tiles left over split (258 tiles of 333 x
-/// 4096 x 11008 take 65.4 us as 258 workgroups, where two CUs work twice as
-/// long, and 56.4 us as 256 plus 2 x 8 slices).
+/// of one workgroup per CU and the tiles left over split (333 x 4096 x
+/// 11008 r16, whole call: 60.8 us with 256 of the 258 tiles whole and the other
+/// two in 8 slices, 71.6 with nothing split, where two CUs work twice as long).
 /// (A call comes here twice, for the workspace and for the launch, so it is kept
 /// to a few dozen candidates and 32-bit divisions: 0.3 us.)
 TilePlan best_plan(int64_t M, int64_t N, int64_t K, int64_t rank) {

@@ -298,11 +298,15 @@ size_t cf_lora_forward_workspace_bytes(cf_dtype dtype, int64_t batch, int64_t in
  * partial sums live there. bf16 with at most 64 rows, in_features and
  * out_features multiples of 8 and a rank up to 256 streams w once, cut over
  * columns and the reduction range, and sums the slices in a fixed order
- * (deterministic; fp32 accumulation and the same bf16 rounding of x @ a).
- * bf16 with more rows and a rank up to 128, where 256 x 256 tiles would leave
- * the GPU idle or the fused kernel does not take the rank or in_features,
- * runs smaller tiles on the MFMA units. Every other problem runs as cf_lora_linear_ws. Calls that overlap (other
- * streams) need workspaces of their own. Replaces launch_lora_linear
+ * (deterministic; fp32 accumulation and the same bf16 rounding of x @ a),
+ * unless the fused kernel is estimated faster (short reductions). bf16 with
+ * more rows and a rank up to 128, where 256 x 256 tiles would leave the GPU
+ * idle or the fused kernel does not take the rank or in_features, runs smaller
+ * tiles on the MFMA units. Both hold the scale and the adapter's sum in fp32;
+ * the fused kernel multiplies by scale * b in two bf16 parts (one where that is
+ * exact), about 2^-17 of the adapter term. Every other problem runs as
+ * cf_lora_linear_ws. Calls that overlap (other streams) need workspaces of
+ * their own. Replaces launch_lora_linear
  * (cuda/include/cudaforge/lora_linear.cuh:49-51). */
 cf_status cf_lora_forward(const void* x, const void* w, const void* a, const void* b, void* y,
                           float* xa_out, cf_dtype dtype, int64_t batch, int64_t in_features,
